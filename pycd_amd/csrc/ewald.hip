@@ -21,128 +21,254 @@
 namespace pycd {
 
 // --------------------------------------------------------- structure factors
+// Y[i, m] = sqrt(w_m) cos, Y[i, K + m] = sqrt(w_m) sin for i < n, m < K; the
+// columns from 2 K to Kp and the rows from n to n_pad are zero.  A thread
+// keeps one k vector and walks kSfRows rows, so a wavefront's stores are 512
+// contiguous bytes and no index is divided.  Bound by sincos and by the
+// write of Y.
+constexpr int kSfRows = 16;
+
 __global__ void __launch_bounds__(256)
-structure_factor_f64(const double* __restrict__ pos, int n,
+structure_factor_f64(const double* __restrict__ pos, int n, int n_pad,
                      const double* __restrict__ kv, const double* __restrict__ sw,
                      int K, int Kp, double* __restrict__ Y) {
-  const int64_t total = int64_t(n) * K;
-  for (int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-       idx < total; idx += int64_t(gridDim.x) * blockDim.x) {
-    const int i = int(idx / K);
-    const int m = int(idx - int64_t(i) * K);
-    const double ph = kv[3 * m] * pos[3 * i] + kv[3 * m + 1] * pos[3 * i + 1] +
-                      kv[3 * m + 2] * pos[3 * i + 2];
-    double s, c;
-    sincos(ph, &s, &c);
-    Y[int64_t(i) * Kp + m] = sw[m] * c;
-    Y[int64_t(i) * Kp + K + m] = sw[m] * s;
+  const int m = blockIdx.x * 256 + threadIdx.x;
+  if (m >= Kp - K) return;
+  const bool real = m < K;
+  const double kx = real ? kv[3 * m] : 0.0, ky = real ? kv[3 * m + 1] : 0.0,
+               kz = real ? kv[3 * m + 2] : 0.0, w = real ? sw[m] : 0.0;
+  const int i0 = blockIdx.y * kSfRows, i1 = min(i0 + kSfRows, n_pad);
+  for (int i = i0; i < i1; ++i) {
+    double vc = 0.0, vs = 0.0;
+    if (real && i < n) {
+      const double ph = kx * pos[3 * i] + ky * pos[3 * i + 1] +
+                        kz * pos[3 * i + 2];
+      double s, c;
+      sincos(ph, &s, &c);
+      vc = w * c;
+      vs = w * s;
+    }
+    double* row = Y + int64_t(i) * Kp;
+    if (real) row[m] = vc;
+    row[K + m] = vs;
   }
 }
 
 // ------------------------------------------------- FP64 contraction + epilogue
-// One (16 kRt) x (16 kRt) tile of A per 256-thread workgroup; thread
-// (tx, ty) owns rows ty + 16 r and columns tx + 16 c (r, c < kRt).  K is
-// staged through LDS in slices of 16.  A thread reads 2 kRt LDS values per
-// k for kRt^2 FMAs: kRt = 4 (64 x 64 tiles) needs 4 bytes of LDS per FMA,
-// twice what the LDS can feed the FP64 units; kRt = 8 (128 x 128) halves
-// that at a quarter of the workgroups.  Every entry's sum over k runs in
-// the same order in both, so they give the same table bit for bit.
+// One (32 kB) x (32 kB) tile of A per 256-thread workgroup, each wavefront
+// one quarter of it in kB x kB blocks of v_mfma_f64_16x16x4: lane l gives
+// row (column) l mod 16 at k + l / 16 and holds rows l / 16 + 4 v of column
+// l mod 16.  The instruction adds its four products one after another in
+// ascending k, each rounded as an FMA (checked against that chain on random
+// operands), so an entry is the chain over k whatever the tile, and tiles
+// give the same table bit for bit.
+//
+// Bound by the FP64 matrix rate, 78.6 TF/s (77 measured with operands in
+// registers).  A wavefront reads 2 kB doubles of LDS per lane and k step for
+// kB^2 instructions of 64 cycles: 32 cycles of LDS per 1024 at kB = 4.  On
+// the vector units, where every FMA takes its operands from two LDS reads
+// shared by 8, the LDS was the limit (8 x 8 entries per thread, 2 bytes per
+// FMA).  At 12000 sites and 2 K = 9836: 34.0 -> 21.3 ms (66 TF/s over whole
+// tiles, two workgroups per CU); at 2592 sites and 2 K = 2142, fewer tiles
+// than CUs: 611 -> 275 us.
+//
+// K goes through LDS in slices of 16 in two stages, one barrier per slice
+// without a memory fence (only this wavefront's LDS operations are waited
+// for), global loads two slices ahead.  Y holds whole tiles of rows and Kp
+// whole pairs of slices (zero past n and 2 K), so loads are unconditional.  Rows
+// of 16 + 2 doubles put the 16 rows and two k of half a wavefront's read on
+// distinct banks.
 constexpr int kSlice = 16;
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
 
-template <int kRt>
+template <int kB>
 __global__ void __launch_bounds__(256)
-table_f64(const double* __restrict__ Y, int n, int Kp,
-          const double* __restrict__ pos, MicGeometry g, EwaldScalars es,
-          double* __restrict__ A, unsigned long long* __restrict__ pairs) {
-  constexpr int kTile = 16 * kRt;
-  __shared__ double As[kSlice][kTile + 2];
-  __shared__ double Bs[kSlice][kTile + 2];
-  const int t = threadIdx.x;
-  const int tx = t & 15, ty = t >> 4;
+__attribute__((amdgpu_waves_per_eu(2)))
+table_f64(const double* __restrict__ Y, int n, int Kp, EwaldScalars es,
+          double* __restrict__ A) {
+  constexpr int kTile = 32 * kB;
+  constexpr int kRow = kSlice + 2;
+  constexpr int kArr = kTile * kRow;
+  // stage s, operand a at S + (2 s + a) kArr
+  __shared__ __attribute__((aligned(16))) double S[4 * kArr];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   int bi, bj;
   tile_coords_upper(n, kTile, bi, bj);
   const int i0 = bi * kTile, j0 = bj * kTile;
   const bool mirror = bi != bj;
+  const int wr = (wave >> 1) * (kTile / 2), wc = (wave & 1) * (kTile / 2);
 
-  double acc[kRt][kRt];
+  v4d acc[kB][kB];
 #pragma unroll
-  for (int r = 0; r < kRt; ++r)
+  for (int x = 0; x < kB; ++x)
 #pragma unroll
-    for (int c = 0; c < kRt; ++c) acc[r][c] = 0.0;
+    for (int y = 0; y < kB; ++y) acc[x][y] = v4d{0.0, 0.0, 0.0, 0.0};
 
-  // loader: kTile rows x 16 k = 256 threads x (kTile / 16) doubles per
-  // array, as double2 pairs of consecutive k
-  constexpr int kPer = kTile / 16;          // doubles per thread and array
-  constexpr int kRowsPerPass = 256 * 4 / 16;  // rows per pass of 4 doubles
-  auto load_rows = [&](int k0, double (&av)[kPer], double (&bv)[kPer]) {
+  // loader: a thread takes 2 consecutive k of every 32nd row, 8 threads
+  // the 128 bytes of a row
+  const int lrow = t >> 3, lk = (t & 7) * 2;
+  typedef const __attribute__((address_space(1))) v2d* gp;
+  const double* ya = Y + int64_t(i0 + lrow) * Kp + lk;
+  const double* yb = Y + int64_t(j0 + lrow) * Kp + lk;
+  v2d ra[kB], rb[kB];
+  auto gload = [&](int k0) {
 #pragma unroll
-    for (int q = 0; q < kPer / 4; ++q) {
-      const int row = (t >> 2) + kRowsPerPass * q;
-      const int lk = (t & 3) * 4;
-      double2 a01 = make_double2(0.0, 0.0), a23 = a01, b01 = a01, b23 = a01;
-      if (i0 + row < n) {
-        const double* ya = Y + int64_t(i0 + row) * Kp + k0 + lk;
-        a01 = *reinterpret_cast<const double2*>(ya);
-        a23 = *reinterpret_cast<const double2*>(ya + 2);
-      }
-      if (j0 + row < n) {
-        const double* yb = Y + int64_t(j0 + row) * Kp + k0 + lk;
-        b01 = *reinterpret_cast<const double2*>(yb);
-        b23 = *reinterpret_cast<const double2*>(yb + 2);
-      }
-      av[4 * q] = a01.x;
-      av[4 * q + 1] = a01.y;
-      av[4 * q + 2] = a23.x;
-      av[4 * q + 3] = a23.y;
-      bv[4 * q] = b01.x;
-      bv[4 * q + 1] = b01.y;
-      bv[4 * q + 2] = b23.x;
-      bv[4 * q + 3] = b23.y;
+    for (int q = 0; q < kB; ++q) {
+      ra[q] = *(gp)(ya + int64_t(32 * q) * Kp + k0);
+      rb[q] = *(gp)(yb + int64_t(32 * q) * Kp + k0);
     }
   };
-
-  for (int k0 = 0; k0 < Kp; k0 += kSlice) {
-    double av[kPer], bv[kPer];
-    load_rows(k0, av, bv);
-    __syncthreads();
+  auto sstore = [&](int stage) {
+    double* a = S + 2 * stage * kArr + lrow * kRow + lk;
 #pragma unroll
-    for (int q = 0; q < kPer / 4; ++q) {
-      const int row = (t >> 2) + kRowsPerPass * q;
-      const int lk = (t & 3) * 4;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        As[lk + e][row] = av[4 * q + e];
-        Bs[lk + e][row] = bv[4 * q + e];
-      }
+    for (int q = 0; q < kB; ++q) {
+      *reinterpret_cast<v2d*>(a + 32 * q * kRow) = ra[q];
+      *reinterpret_cast<v2d*>(a + kArr + 32 * q * kRow) = rb[q];
     }
-    __syncthreads();
+  };
+  auto lds_barrier = [] {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  // fragments of k step u of the slice in `stage`: one double per block,
+  // two sets so that a step's reads are in flight behind the last step's
+  // instructions
+  double fa[2][kB], fb[2][kB];
+  auto fetch = [&](int set, int stage, int u) {
+    const double* a = S + 2 * stage * kArr + (wr + (lane & 15)) * kRow +
+                      (lane >> 4) + 4 * u;
+    const double* b = S + (2 * stage + 1) * kArr + (wc + (lane & 15)) * kRow +
+                      (lane >> 4) + 4 * u;
 #pragma unroll
-    for (int kk = 0; kk < kSlice; ++kk) {
-      double a[kRt], b[kRt];
-#pragma unroll
-      for (int r = 0; r < kRt; ++r) a[r] = As[kk][ty + 16 * r];
-#pragma unroll
-      for (int c = 0; c < kRt; ++c) b[c] = Bs[kk][tx + 16 * c];
-#pragma unroll
-      for (int r = 0; r < kRt; ++r)
-#pragma unroll
-        for (int c = 0; c < kRt; ++c) acc[r][c] = fma(a[r], b[c], acc[r][c]);
+    for (int x = 0; x < kB; ++x) {
+      fa[set][x] = a[16 * x * kRow];
+      fb[set][x] = b[16 * x * kRow];
     }
+  };
+  auto multiply = [&](int set) {
+#pragma unroll
+    for (int x = 0; x < kB; ++x)
+#pragma unroll
+      for (int y = 0; y < kB; ++y)
+        acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+            fa[set][x], fb[set][y], acc[x][y], 0, 0, 0);
+  };
+  // One k step: the fragments of the next step (and `more`, if any) issued
+  // between this step's instructions, one read per kB / 2 of them, so that
+  // neither the matrix core nor the LDS waits for a burst of the other.
+  auto k_step = [&](int set, int next_stage, int next_u, auto&& more) {
+    fetch(set ^ 1, next_stage, next_u);
+    more();
+    multiply(set);
+#pragma unroll
+    for (int q = 0; q < 2 * kB; ++q) {
+      __builtin_amdgcn_sched_group_barrier(0x008, kB / 2, 0);  // MFMA
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);       // LDS read
+      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);       // LDS write
+      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);       // global load
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Step for the slice at k0, in `stage`, its first fragments read: the next
+  // slice goes from registers to the other stage, the one after it is
+  // loaded; the barrier comes once this slice's last fragments are read, a k
+  // step before the slice is done, and the next slice's first fragments are
+  // read behind that k step.  (The last steps load and store the last slice
+  // again, into a stage that no step reads.)
+  auto step = [&](int stage, int k0) {
+    k_step(0, stage, 1, [] {});
+    k_step(1, stage, 2, [&] { sstore(stage ^ 1); });
+    k_step(0, stage, 3, [&] { gload(min(k0 + 2 * kSlice, Kp - kSlice)); });
+    lds_barrier();
+    k_step(1, stage ^ 1, 0, [] {});
+  };
+  gload(0);
+  sstore(0);
+  gload(min(kSlice, Kp - kSlice));
+  lds_barrier();
+  fetch(0, 0, 0);
+  for (int k0 = 0; k0 < Kp; k0 += 2 * kSlice) {
+    step(0, k0);
+    step(1, k0 + kSlice);
   }
 
+  // the reciprocal part alone, no mirror: finish_table does the rest
+#pragma unroll
+  for (int x = 0; x < kB; ++x)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = i0 + wr + 16 * x + (lane >> 4) + 4 * v;
+      double* row = A + int64_t(i) * n + j0 + wc + (lane & 15);
+#pragma unroll
+      for (int y = 0; y < kB; ++y)
+        if (i < n && j0 + wc + 16 * y + (lane & 15) < n)
+          row[16 * y] = recip_part(es, acc[x][y][v]);
+    }
+}
+
+// The rest of each entry after the contraction, and its mirror, one 64 x 64
+// block of the upper triangle per 256-thread workgroup: a wavefront takes
+// every 4th row, a lane a column, so that rows are read and written 512
+// bytes at a time and row positions come through scalar loads; the mirror
+// goes through LDS and is written the same way.  (In the contraction's
+// epilogue these were 64 minimum images and erfcs of straight-line code per
+// thread at two wavefronts per SIMD, and 8-byte mirror stores: 378 us in
+// one kernel at 2592 sites, 275 + 59 us apart.)  Off the diagonal tiles (j, i) is the same
+// number as (i, j): the same products in the same order, and squared
+// distances from negated differences (see store_pair).  A tile on the
+// diagonal has both as formed, so its blocks write no mirror.
+template <int kTile>
+__global__ void __launch_bounds__(256)
+finish_table(const double* __restrict__ pos, int n, MicGeometry g,
+             EwaldScalars es, double* __restrict__ A,
+             unsigned long long* __restrict__ pairs) {
+  constexpr int kSub = kTile / 64;  // blocks per tile side
+  __shared__ double T[64][65];
+  int bi, bj;
+  tile_coords_upper_at(n, kTile, int(blockIdx.x) / (kSub * kSub), bi, bj);
+  const int sub = int(blockIdx.x) % (kSub * kSub);
+  const int i0 = bi * kTile + sub / kSub * 64, j0 = bj * kTile + sub % kSub * 64;
+  const bool mirror = bi != bj;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j = j0 + lane;
+  const bool j_ok = j < n;
+  const double pjx = j_ok ? pos[3 * j] : 0.0;
+  const double pjy = j_ok ? pos[3 * j + 1] : 0.0;
+  const double pjz = j_ok ? pos[3 * j + 2] : 0.0;
+  const int i_end = min(64, n - i0);
   unsigned cnt = 0;
-#pragma unroll
-  for (int r = 0; r < kRt; ++r) {
-    const int i = i0 + ty + 16 * r;
-    if (i >= n) continue;
-#pragma unroll
-    for (int c = 0; c < kRt; ++c) {
-      const int j = j0 + tx + 16 * c;
-      if (j >= n) continue;
-      store_pair(A, n, i, j, mirror, pos, g, es, acc[r][c], cnt);
+  for (int k = wave; k < i_end; k += 4) {
+    const int i = i0 + k;
+    if (j_ok) {
+      const int64_t o = int64_t(i) * n + j;
+      const double recip = A[o];
+      double v = real_part_d(i, j, pjx - pos[3 * i], pjy - pos[3 * i + 1],
+                             pjz - pos[3 * i + 2], g, es, cnt) +
+                 recip;
+      if (i == j) v += es.self_term;
+      A[o] = v;
+      T[k][lane] = v;
     }
   }
-  count_pairs(cnt, pairs);
+  count_pairs(mirror ? 2 * cnt : cnt, pairs);
+  if (!mirror) return;
+  __syncthreads();
+  const int j_end = min(64, n - j0);
+  if (lane < i_end)
+    for (int k = wave; k < j_end; k += 4)
+      A[int64_t(j0 + k) * n + i0 + lane] = T[lane][k];
+}
+
+void launch_finish(hipStream_t s, int tile, const double* pos, int n,
+                   const MicGeometry& geo, const EwaldScalars& es, double* A,
+                   unsigned long long* pairs) {
+  const int nb = (n + tile - 1) / tile, tiles = nb * (nb + 1) / 2;
+  if (tile == 64)
+    finish_table<64><<<tiles, 256, 0, s>>>(pos, n, geo, es, A, pairs);
+  else
+    finish_table<128><<<4 * tiles, 256, 0, s>>>(pos, n, geo, es, A, pairs);
 }
 
 // ------------------------------------------------------------------ launch
@@ -150,44 +276,44 @@ int launch_table_mfma(pycd_ctx* ctx, int precision, const double* pos, int n,
                       const double* kv, const double* sw, int K,
                       const MicGeometry& geo, const EwaldScalars& es,
                       double* out, unsigned long long* pairs,
-                      hipEvent_t after_sf, hipEvent_t after_real,
+                      hipEvent_t after_sf, hipEvent_t (&real)[2],
                       bool& real_apart);
 
 int launch_table(pycd_ctx* ctx, int precision, const double* pos, int n,
                  const double* kv, const double* sw, int K,
                  const MicGeometry& geo, const EwaldScalars& es, double* out,
                  unsigned long long* pairs, hipEvent_t after_sf,
-                 hipEvent_t after_real, bool& real_apart) {
+                 hipEvent_t (&real)[2], bool& real_apart) {
   real_apart = false;
   if (precision != PYCD_PREC_F64)
     return launch_table_mfma(ctx, precision, pos, n, kv, sw, K, geo, es, out,
-                             pairs, after_sf, after_real, real_apart);
+                             pairs, after_sf, real, real_apart);
   hipStream_t s = ctx->stream;
-  const int Kp = ((2 * K + kSlice - 1) / kSlice) * kSlice + (K == 0 ? kSlice : 0);
-  DevBuf<double> Y;
-  PYCD_HIP(ctx, Y.alloc(size_t(n) * Kp));
-  PYCD_HIP(ctx, hipMemsetAsync(Y.ptr, 0, sizeof(double) * size_t(n) * Kp, s));
-  if (K > 0) {
-    const int64_t total = int64_t(n) * K;
-    const int blocks = int(std::min<int64_t>((total + 255) / 256, 65536));
-    structure_factor_f64<<<blocks, 256, 0, s>>>(pos, n, kv, sw, K, Kp, Y.ptr);
-    PYCD_HIP(ctx, hipGetLastError());
-  }
-  PYCD_HIP(ctx, hipEventRecord(after_sf, s));
-  // (the real-space term is in the epilogue: no time of its own)
-  PYCD_HIP(ctx, hipEventRecord(after_real, s));
   // tile variant: 1 = 64 x 64, 2 = 128 x 128; 0 picks 128 from 2048 sites
   int v = ctx->table_variant[PYCD_PREC_F64];
   if (v == 0) v = n >= 2048 ? 2 : 1;
-  if (v == 2) {
-    const int nb = (n + 127) / 128;
-    table_f64<8><<<nb * (nb + 1) / 2, 256, 0, s>>>(Y.ptr, n, Kp, pos, geo, es,
-                                                   out, pairs);
-  } else {
-    const int nb = (n + 63) / 64;
-    table_f64<4><<<nb * (nb + 1) / 2, 256, 0, s>>>(Y.ptr, n, Kp, pos, geo, es,
-                                                   out, pairs);
-  }
+  const int tile = v == 2 ? 128 : 64;
+  const int nb = (n + tile - 1) / tile;
+  // K in whole pairs of slices, rows in whole tiles
+  const int pair = 2 * kSlice;
+  const int Kp = std::max(pair, (2 * K + pair - 1) / pair * pair);
+  const int n_pad = nb * tile;
+  DevBuf<double> Y;
+  PYCD_HIP(ctx, Y.alloc(size_t(n_pad) * Kp));
+  structure_factor_f64<<<dim3((Kp - K + 255) / 256,
+                              (n_pad + kSfRows - 1) / kSfRows),
+                         256, 0, s>>>(pos, n, n_pad, kv, sw, K, Kp, Y.ptr);
+  PYCD_HIP(ctx, hipGetLastError());
+  PYCD_HIP(ctx, hipEventRecord(after_sf, s));
+  if (v == 2)
+    table_f64<4><<<nb * (nb + 1) / 2, 256, 0, s>>>(Y.ptr, n, Kp, es, out);
+  else
+    table_f64<2><<<nb * (nb + 1) / 2, 256, 0, s>>>(Y.ptr, n, Kp, es, out);
+  PYCD_HIP(ctx, hipGetLastError());
+  real_apart = true;
+  PYCD_HIP(ctx, hipEventRecord(real[0], s));
+  launch_finish(s, tile, pos, n, geo, es, out, pairs);
+  PYCD_HIP(ctx, hipEventRecord(real[1], s));
   PYCD_HIP(ctx, hipGetLastError());
   // Y is released when this returns; the stream must have consumed it.
   PYCD_HIP(ctx, hipStreamSynchronize(s));
@@ -309,15 +435,17 @@ extern "C" int pycd_pair_table(pycd_ctx* ctx, const double* pos, int64_t n,
     out = d_A.ptr;
   }
 
-  // structure factors, [separate real-space kernel], contraction
-  hipEvent_t ev[4];
+  // the whole table around the structure factors; the real-space kernel
+  hipEvent_t ev[3], real[2];
   for (auto& e : ev) PYCD_HIP(ctx, hipEventCreate(&e));
+  for (auto& e : real) PYCD_HIP(ctx, hipEventCreate(&e));
   PYCD_HIP(ctx, hipEventRecord(ev[0], s));
   bool real_apart = false;
   rc = launch_table(ctx, precision, d_pos.ptr, N, d_kv.ptr, d_sw.ptr, K, st.geo,
-                    es, out, d_pairs.ptr, ev[1], ev[3], real_apart);
+                    es, out, d_pairs.ptr, ev[1], real, real_apart);
   if (rc) {
     for (auto& e : ev) (void)hipEventDestroy(e);
+    for (auto& e : real) (void)hipEventDestroy(e);
     return rc;
   }
   PYCD_HIP(ctx, hipEventRecord(ev[2], s));
@@ -331,8 +459,9 @@ extern "C" int pycd_pair_table(pycd_ctx* ctx, const double* pos, int64_t n,
   float ms_sf = 0, ms_rest = 0, ms_real = 0;
   (void)hipEventElapsedTime(&ms_sf, ev[0], ev[1]);
   (void)hipEventElapsedTime(&ms_rest, ev[1], ev[2]);
-  (void)hipEventElapsedTime(&ms_real, ev[1], ev[3]);
+  if (real_apart) (void)hipEventElapsedTime(&ms_real, real[0], real[1]);
   for (auto& e : ev) (void)hipEventDestroy(e);
+  for (auto& e : real) (void)hipEventDestroy(e);
   if (report) {
     report->n_kvec = K;
     report->n_real_pairs = int64_t(pairs);
@@ -340,7 +469,7 @@ extern "C" int pycd_pair_table(pycd_ctx* ctx, const double* pos, int64_t n,
     report->precision = precision;
     report->volume = st.volume;
     report->ms_sf = ms_sf;
-    report->ms_real = real_apart ? ms_real : 0.0;
+    report->ms_real = ms_real;
     report->ms_recip = ms_rest;
     report->ms_total = double(ms_sf) + ms_rest;
   }

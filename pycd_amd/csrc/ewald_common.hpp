@@ -184,10 +184,15 @@ __device__ __forceinline__ double real_part(int i, int j,
 
 // Entry (i, j) from its real-space part and the reciprocal accumulator
 // `acc` (= sum over the half space of w cos, i.e. (Y Y^T)[i,j]).
+__device__ __forceinline__ double recip_part(const EwaldScalars& es,
+                                             double acc) {
+  return es.unit_eps ? 2.0 * acc : (2.0 * acc) / es.eps;
+}
+
 __device__ __forceinline__ double finish_entry(int i, int j,
                                                const EwaldScalars& es,
                                                double real, double acc) {
-  double out = real + (es.unit_eps ? 2.0 * acc : (2.0 * acc) / es.eps);
+  double out = real + recip_part(es, acc);
   if (i == j) out += es.self_term;
   return out;
 }
@@ -276,10 +281,17 @@ __device__ __forceinline__ void store_pair(double* __restrict__ A, int n, int i,
   }
 }
 
+// Adds the real-space and self terms to the entries that a contraction over
+// the upper triangle of `tile` x `tile` tiles (64 or 128) left in A, and
+// writes the mirrors of the tiles off the diagonal (finish_table, ewald.hip).
+void launch_finish(hipStream_t s, int tile, const double* pos, int n,
+                   const MicGeometry& geo, const EwaldScalars& es, double* A,
+                   unsigned long long* pairs);
+
 int launch_table(pycd_ctx* ctx, int precision, const double* pos, int n,
                  const double* kv, const double* sw, int K,
                  const MicGeometry& geo, const EwaldScalars& es, double* out,
                  unsigned long long* pairs, hipEvent_t after_sf,
-                 hipEvent_t after_real, bool& real_apart);
+                 hipEvent_t (&real)[2], bool& real_apart);
 
 }  // namespace pycd
