@@ -217,7 +217,7 @@ def run_plain(args, log):
     dev.free()
     nc = 16
     z = int(np.max(run.nbr_count))
-    per_hop = plain_bytes_per_hop(variant, nc, z)
+    per_hop = plain_bytes_per_hop(nc, z)
     gbs = per_hop * hops / (ms / 1e3) / 1e9
     _KEEP["plain"] = (run, table)
     return {"hops": hops, "ms": ms, "hops_per_s": hops / (ms / 1e3),
@@ -226,24 +226,17 @@ def run_plain(args, log):
             "roofline": {"bound": "hbm", "achieved": gbs,
                          "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": gbs / HBM_PEAK_GBS,
-                         "kernel": ("kmc_wave_kernel" if variant == "wave"
-                                    else "kmc_plain_kernel"),
+                         "kernel": "kmc_hop_kernel",
                          "algorithmic_bytes_per_hop": per_hop}}
 
 
-def plain_bytes_per_hop(variant, nc, z):
-    """Bytes the plain kernel's algorithm reads per hop.
-
-    wave (row cache in LDS): (1 + z)(2 n_c - 1) table entries (column m of
-    the other rows, the mover's 1 + z new rows), 10 doubles of rate inputs
-    for each of the mover's z new processes (phi_L and E at both ends, the
-    self term, lambda, V_ab, hop vector), 2 z^2 words of look-ahead slot
-    tables and 24 B of uniforms (u1, u2, log u2).
-    workgroup: n_c (1 + z) x n_c table entries (every row gathered again),
-    11 doubles per process and 16 B of uniforms."""
-    if variant == "wave":
-        return 8 * (1 + z) * (2 * nc - 1) + 80 * z + 8 * z * z + 24
-    return 8 * nc * (1 + z) * nc + 8 * 11 * nc * z + 16
+def plain_bytes_per_hop(nc, z):
+    """Bytes the plain kernel's algorithm reads per hop: two table entries
+    for each of the n_c (1 + z) rows (the mover's new and old site), n_c for
+    each of the mover's z new targets, 10 doubles of rate inputs for each of
+    its z new processes (the 64-byte slot record, E at both ends), 2 z^2
+    words of look-ahead slot tables and 24 B of uniforms (u1, u2, log u2)."""
+    return 8 * (2 * nc * (1 + z) + z * nc) + 80 * z + 8 * z * z + 24
 
 
 def run_serve(args, log):

@@ -204,14 +204,14 @@ int pycd_kmc_set_sites(pycd_kmc* s, const double* lattice_q,
  * otherwise.  No reference counterpart. */
 int pycd_kmc_table_rows(const pycd_kmc* s, int64_t* rows);
 
-/* Kernel of the hop loop.  PYCD_KMC_WAVE: one wavefront that keeps the
- * table entries of every carrier at every site the rates need in LDS
- * (n_c <= 64, n_c z <= 256, z <= 8 and the cache within a workgroup's
- * LDS); PYCD_KMC_WORKGROUP: a 256-thread workgroup that gathers them again
- * each hop (any size); PYCD_KMC_AUTO (the default): the wavefront kernel
- * where it applies.  Both give the same results bit for bit.  Asking for
+/* Instance of the hop loop.  PYCD_KMC_WAVE: few carriers (n_c <= 64,
+ * n_c z <= 256, z <= 8, the table entries of every carrier at every site
+ * the rates need within a workgroup's LDS and a table below 4 GiB);
+ * PYCD_KMC_WORKGROUP: any size; PYCD_KMC_AUTO (the default):
+ * PYCD_KMC_WAVE where it applies.  One kernel serves all of them, so they
+ * give the same results bit for bit and take the same time.  Asking for
  * PYCD_KMC_WAVE where it does not apply is an argument error.
- * pycd_kmc_variant reports the kernel the next pycd_kmc_advance runs.  No
+ * pycd_kmc_variant reports the instance of the next pycd_kmc_advance.  No
  * reference counterpart. */
 #define PYCD_KMC_AUTO 0
 #define PYCD_KMC_WORKGROUP 1

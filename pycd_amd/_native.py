@@ -413,14 +413,14 @@ class KmcSession:
         return n.value
 
     def set_variant(self, name):
-        """Kernel of the hop loop: 'auto' (default), 'workgroup' or 'wave'
-        (the one-wavefront kernel with its LDS row cache; refused where it
-        does not apply)."""
+        """Instance of the hop loop: 'auto' (default), 'workgroup' or 'wave'
+        (few carriers; refused where it does not apply).  One kernel serves
+        them all."""
         _check(self.ctx, lib().pycd_kmc_set_variant(self.h, KMC_VARIANT[name]),
                "pycd_kmc_set_variant")
 
     def variant(self):
-        """Kernel the next advance runs: 'wave' or 'workgroup'."""
+        """Instance of the next advance: 'wave' or 'workgroup'."""
         v = C.c_int32(0)
         _check(self.ctx, lib().pycd_kmc_variant(self.h, C.byref(v)),
                "pycd_kmc_variant")

@@ -8,18 +8,12 @@
 //
 // The N-long dot product is never formed.  With q = q_lattice + sum_c q_c
 // e_{occ_c},  q.A[x,:] = phi_L[x] + psi[x],  where phi_L = A q_lattice is
-// computed once per table and psi[x] = sum_c q_c A[x, occ_c] is gathered
-// each hop for the sites x that matter: every carrier's site and its z hop
-// targets.  That is n_c (1 + z) x n_c table reads per hop instead of
-// n_c z x N, with the same value of q.(A[n,:] - A[s,:]) up to rounding.
+// computed once per table and psi[x] = sum_c q_c A[x, occ_c] covers the
+// sites x that matter: every carrier's site and its z hop targets.  The
+// value of q.(A[n,:] - A[s,:]) is the same up to rounding.
 //
-// One persistent 256-thread workgroup runs the trajectory (the hop chain is
-// serial).  Phases per hop, separated by workgroup barriers:
-//   A  psi gathers                                    (all threads)
-//   B  dG0, Marcus/field rate per process             (all threads)
-//   C  k_tot, wavefront prefix scan of k/k_tot,
-//      selection, clock, state update                 (wavefront 0)
-//   D  path-step rows written for [start, end)        (all threads)
+// One persistent workgroup runs the trajectory (the hop chain is serial);
+// psi of every row is kept from hop to hop, see kmc_hop_kernel.
 #include "common.hpp"
 #include "packed_sites.hpp"
 #include "wave.hpp"
@@ -40,41 +34,16 @@ struct KmcScalars {
   int32_t no_select;  // hops where rounding left no cum > u1 (last taken)
 };
 
+// What the hop loop reads once and the state it begins with and leaves.
 struct KmcDev {
-  const double* A;
-  // periodic supercell (compact instance): the table rows of cell 0, the
-  // packed code of every site and of every slot's target
-  const double* Ac;
-  const uint32_t* pk;
-  const uint32_t* nbr_pk;
-  GeoPk gp;
-  const double* phiL;
-  const double* dphi;  // q_L . (A[n, :] - A[s, :]) per (site, slot)
-  const int32_t* nbr;
-  const double* vec;
-  const double* lam;
-  const double* vab;
-  const double* tself;
-  const double* E;
+  const uint32_t* pk;  // packed code of every site (cell-0 rows only)
   const double* cq;
-  int64_t N;
-  int32_t nc, z, max_z, field_on;
-  double field[3];
-  double nu, kT, dt;
-  double nkt;  // -1 / kT
-  int64_t P;
-  // state
   int32_t* occ;
   double* disp;
   double* base;
   double* drift;
-  double* rows;
-  double* epath;
-  double* dpath;
   KmcScalars* sc;
 };
-
-constexpr int kThreads = 256;
 
 // log(u2) of every uniform pair ahead of the hop loop (0 where u2 = 0, a
 // value the loop does not use), so that no hop waits for an FP64 log.
@@ -88,298 +57,8 @@ log_u2_kernel(const double* __restrict__ U, int64_t n,
   }
 }
 
-template <bool kCompact>
-__global__ void __launch_bounds__(kThreads)
-kmc_plain_kernel(KmcDev d, const double* __restrict__ U,
-                 const double* __restrict__ LU, int64_t n_pairs,
-                 int64_t max_hops, double* __restrict__ hop_time,
-                 int32_t* __restrict__ hop_proc, int32_t* __restrict__ status) {
-  extern __shared__ double smem[];
-  const int nc = d.nc, z = d.z, R = nc * (1 + z), nproc = nc * z;
-  double* psi = smem;                 // R
-  double* kk = psi + R;               // nproc
-  double* dg = kk + nproc;            // nproc
-  double* disp = dg + nproc;          // 3 nc
-  double* base = disp + 3 * nc;       // 3 nc
-  double* drift = base + 3 * nc;      // 3 nc
-  // per process p = c z + j (carrier c, slot j of its site): the values of
-  // its rate that depend only on the site, refreshed when c hops
-  double* pdphi = drift + 3 * nc;     // q_L . (A[n, :] - A[s, :])
-  double* ptq = pdphi + nproc;        // q_c tself[s, j]
-  double* pdE = ptq + nproc;          // E[n] - E[s]
-  double* plam = pdE + nproc;         // lambda
-  double* pi4l = plam + nproc;        // 1 / (4 lambda)
-  double* pvs = pi4l + nproc;         // V_ab + field . hop vector / 2
-  double* pvec = pvs + nproc;         // hop vector (3 nproc)
-  int32_t* pn = reinterpret_cast<int32_t*>(pvec + 3 * nproc);  // target n
-  int32_t* occ = pn + nproc;          // nc
-  // compact instance: packed codes of the carriers' sites and of each
-  // process's target
-  uint32_t* opk = reinterpret_cast<uint32_t*>(occ + nc);  // nc
-  uint32_t* pnpk = opk + nc;                              // nproc
-  __shared__ double sh_t, sh_energy, sh_dg;
-  __shared__ double sh_exp[64];  // 2^(j/64)
-  __shared__ int64_t sh_start, sh_hops, sh_row_lo, sh_row_hi, sh_dp_hi;
-  __shared__ int32_t sh_stop, sh_noselect, sh_mover;
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  // the site-dependent part of process p's rate, from the slot tables
-  auto load_process = [&](int p) {
-    const int c = p / z, j = p - c * z;
-    const int s = occ[c];
-    const int64_t sj = int64_t(s) * d.max_z + j;
-    const int n = d.nbr[sj];
-    pn[p] = n;
-    if constexpr (kCompact) pnpk[p] = d.pk[n];
-    pdphi[p] = d.dphi[sj];
-    ptq[p] = d.cq[c] * d.tself[sj];
-    pdE[p] = d.E[n] - d.E[s];
-    {
-      // the same arithmetic as the one-wavefront kernel's slot records
-#pragma clang fp contract(off)
-      const double lam = d.lam[sj];
-      double shift = 0.0;
-      if (d.field_on)
-        shift = 0.5 * (d.field[0] * d.vec[3 * sj] +
-                       d.field[1] * d.vec[3 * sj + 1] +
-                       d.field[2] * d.vec[3 * sj + 2]);
-      plam[p] = lam;
-      pi4l[p] = 1.0 / (4 * lam);
-      pvs[p] = d.vab[sj] + shift;
-    }
-    pvec[3 * p] = d.vec[3 * sj];
-    pvec[3 * p + 1] = d.vec[3 * sj + 1];
-    pvec[3 * p + 2] = d.vec[3 * sj + 2];
-  };
-  for (int c = tid; c < nc; c += kThreads) {
-    occ[c] = d.occ[c];
-    if constexpr (kCompact) opk[c] = d.pk[occ[c]];
-  }
-  for (int k = tid; k < 3 * nc; k += kThreads) {
-    disp[k] = d.disp[k];
-    base[k] = d.base[k];
-    drift[k] = d.drift[k];
-  }
-  if (tid < 64) sh_exp[tid] = __builtin_bit_cast(double, kExp2J64[tid]);
-  if (tid == 0) {
-    sh_t = d.sc->t;
-    sh_energy = d.sc->energy;
-    sh_start = d.sc->start;
-    sh_hops = d.sc->hops;
-    sh_noselect = d.sc->no_select;
-    sh_stop = d.sc->finished ? 1 : 0;
-    sh_mover = -1;
-  }
-  __syncthreads();
-  for (int p = tid; p < nproc; p += kThreads) load_process(p);
-  __syncthreads();
-  int64_t h = 0;  // hops made in this call
-  int stop = sh_stop;
-  int code = stop ? 0 : -1;
-
-  while (!stop) {
-    if (max_hops > 0 && sh_hops >= max_hops) {
-      code = 0;
-      break;
-    }
-    if (h >= n_pairs) {
-      code = 1;  // need uniforms
-      break;
-    }
-    // ---- A: psi[x] = sum_c q_c A[x, occ_c] for carrier sites and targets
-    for (int r = tid; r < R; r += kThreads) {
-      const int c = r / (1 + z);
-      const int slot = r - c * (1 + z);
-      const int s = occ[c];
-      // A[x, y]: the full table's row x, or (compact) the cell-0 row of x's
-      // sublattice at y moved by -cell(x); targets from the global slot
-      // tables, which the mover's reload below does not touch
-      const double* row;
-      RowKey key{};
-      if constexpr (kCompact) {
-        const uint32_t xp =
-            slot == 0 ? opk[c] : d.nbr_pk[int64_t(s) * d.max_z + slot - 1];
-        key = row_key(xp, d.gp);
-        row = d.Ac + int64_t(xp >> 24) * d.N;
-      } else {
-        const int x = slot == 0 ? s : d.nbr[int64_t(s) * d.max_z + slot - 1];
-        row = d.A + int64_t(x) * d.N;
-      }
-      auto col = [&](int c3) -> uint32_t {
-        if constexpr (kCompact) return rel_col(key, opk[c3], d.gp);
-        else return uint32_t(occ[c3]);
-      };
-      // the row's gathers in flight 16 (then 8) at a time, summed in
-      // carrier order
-      double acc = 0.0;
-      int c2 = 0;
-      for (; c2 + 16 <= nc; c2 += 16) {
-        double v[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) v[u] = row[col(c2 + u)];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) acc = fma(d.cq[c2 + u], v[u], acc);
-      }
-      for (; c2 + 8 <= nc; c2 += 8) {
-        double v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = row[col(c2 + u)];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) acc = fma(d.cq[c2 + u], v[u], acc);
-      }
-      for (; c2 < nc; ++c2) acc = fma(d.cq[c2], row[col(c2)], acc);
-      psi[r] = acc;
-    }
-    // the last hop's mover: its processes reloaded for its new site, by
-    // the last z threads while the gathers above are in flight
-    if (sh_mover >= 0 && tid >= kThreads - z)
-      load_process(sh_mover * z + (kThreads - 1 - tid));
-    __syncthreads();
-    // ---- B: rates
-    for (int p = tid; p < nproc; p += kThreads) {
-      // products and sums rounded one by one, as NumPy forms them
-#pragma clang fp contract(off)
-      const int c = p / z;
-      const int j = p - c * z;
-      const double qs = d.cq[c];
-      const double term01 =
-          pdphi[p] + (psi[c * (1 + z) + 1 + j] - psi[c * (1 + z)]);
-      const double term02 = ptq[p];
-      const double g0 = 2 * qs * (term01 + term02) + pdE[p];
-      kk[p] = marcus_rate(g0, plam[p], pi4l[p], pvs[p], d.nkt, d.nu, sh_exp);
-      dg[p] = g0;
-    }
-    __syncthreads();
-    // ---- C: selection, clock and state update on wavefront 0
-    if (tid < 64) {
-      const int per = (nproc + 63) / 64;
-      const int p0 = lane * per;
-      const int p1 = min(p0 + per, nproc);
-      // the first process whose cumulative rate exceeds u1 k_tot (the
-      // reference compares the cumulative sum of k / k_tot with u1: the
-      // same choice but where u1 lies within an ulp of a boundary)
-      double ksum = 0.0;
-      for (int p = p0; p < p1; ++p) ksum += kk[p];
-      const double incl = wave_incl_scan(ksum);
-      const double k_tot = read_lane(incl, 63);
-      const double u1 = U[2 * h];
-      const double u2 = U[2 * h + 1];
-      const double thr = u1 * k_tot;
-      double cum = dpp_f64<kDppWaveShr1, 0xf, true>(incl);
-      int found = -1;
-      for (int p = p0; p < p1; ++p) {
-        cum += kk[p];
-        if (cum > thr) {
-          found = p;
-          break;
-        }
-      }
-      const unsigned long long mask = __ballot(found >= 0);
-      int sel;
-      if (mask) {
-        const int src = __ffsll(static_cast<long long>(mask)) - 1;
-        sel = __shfl(found, src, 64);
-      } else {
-        sel = nproc - 1;
-      }
-      if (lane == 0) {
-#pragma clang fp contract(off)
-        if (!mask) ++sh_noselect;
-        const int c = sel / z;
-        const int s_new = pn[sel];
-        const double* v = pvec + 3 * sel;
-        double t = sh_t;
-        int64_t end;
-        if (u2 > 0.0) {
-          t -= LU[h] / k_tot;
-          const double q = t / d.dt;
-          end = q < 9.0e18 ? int64_t(q) : d.P;
-        } else {
-          t = INFINITY;
-          end = d.P;
-        }
-        sh_t = t;
-        const double g = dg[sel];
-        sh_dg = g;
-        // delg_0 path: [start, end) clipped to P (numpy slice semantics)
-        sh_dp_hi = min(end, d.P);
-        occ[c] = s_new;
-        if constexpr (kCompact) opk[c] = pnpk[sel];
-        sh_mover = c;
-        disp[3 * c] += v[0];
-        disp[3 * c + 1] += v[1];
-        disp[3 * c + 2] += v[2];
-        if (d.field_on) {
-          drift[3 * c] += v[0] * kk[sel];
-          drift[3 * c + 1] += v[1] * kk[sel];
-          drift[3 * c + 2] += v[2] * kk[sel];
-        }
-        sh_energy += g;
-        if (hop_time) hop_time[h] = t;
-        if (hop_proc) hop_proc[h] = sel;
-        sh_row_lo = sh_start;
-        sh_row_hi = sh_start;
-        if (end >= sh_start + 1) {
-          if (end >= d.P) end = d.P;
-          sh_row_hi = end;
-        }
-        sh_hops += 1;
-        // loop condition of the reference: continue while end < P
-        sh_stop = (sh_row_hi > sh_row_lo && sh_row_hi >= d.P) ? 1 : 0;
-      }
-    }
-    __syncthreads();
-    ++h;
-    // ---- D: path-step outputs on all threads, for a hop that ends one or
-    // more path steps (otherwise nothing is written and no barrier is due:
-    // the next hop's first two barriers order C's shared values)
-    if (sh_row_hi > sh_row_lo) {
-      const int64_t lo = sh_row_lo, hi = sh_row_hi;
-      const double g = sh_dg;
-      for (int64_t r = lo + tid; r < sh_dp_hi; r += kThreads) d.dpath[r] = g;
-      if (hi > lo) {
-        const int w = 3 * nc;
-        const double e = sh_energy;
-        for (int64_t idx = tid; idx < (hi - lo) * w; idx += kThreads) {
-          const int64_t r = lo + idx / w;
-          const int k = int(idx % w);
-          d.rows[r * w + k] = base[k] + disp[k];
-        }
-        for (int64_t r = lo + tid; r < hi; r += kThreads) d.epath[r] = e;
-      }
-      __syncthreads();
-      for (int k = tid; k < 3 * nc; k += kThreads) {
-        base[k] += disp[k];
-        disp[k] = 0.0;
-      }
-      if (tid == 0) sh_start = hi;
-      __syncthreads();
-    }
-    stop = sh_stop;
-    if (stop) code = 0;
-  }
-  // ---- write the state back
-  for (int c = tid; c < nc; c += kThreads) d.occ[c] = occ[c];
-  for (int k = tid; k < 3 * nc; k += kThreads) {
-    d.disp[k] = disp[k];
-    d.base[k] = base[k];
-    d.drift[k] = drift[k];
-  }
-  if (tid == 0) {
-    d.sc->t = sh_t;
-    d.sc->energy = sh_energy;
-    d.sc->start = sh_start;
-    d.sc->hops = sh_hops;
-    d.sc->no_select = sh_noselect;
-    if (stop) d.sc->finished = 1;
-    status[0] = code;
-    status[1] = int32_t(h);
-  }
-}
-
 // ---------------------------------------------------------------------------
-// Inputs of the one-wavefront kernel.  Per (site, slot) a 64-byte record:
+// Inputs of the hop loop.  Per (site, slot) a 64-byte record:
 // the self term A[s, s] - A[s, n], lambda, 1 / (4 lambda), V_ab plus the
 // field shift 0.5 F.d, the hop vector d and the lattice part
 // q_L . (A[n, :] - A[s, :]) of the hop's potential difference; per site
@@ -391,12 +70,11 @@ struct alignas(16) SlotRec {
   double dphi;
 };
 
-// What the one-wavefront kernel's hop loop reads, by value; state read only
-// before and after the loop comes from a KmcDev in device memory.
-struct WaveArgs {
+// What the hop loop reads, by value; state read only before and after it
+// comes from a KmcDev in device memory.
+struct HopArgs {
   const char* tab;       // the table (full, or the rows of cell 0)
   uint32_t row_bytes;    // N sizeof(double)
-  int32_t uq;            // every carrier has charge q0
   GeoPk gp;
   const SlotRec* rec;
   const double2* pe;
@@ -409,12 +87,12 @@ struct WaveArgs {
   double* hop_time;
   int32_t* hop_proc;
   int32_t nc, z, mz, field_on;
-  double q0, nu, nkt, dt;  // nkt = -1 / kT
+  double nu, nkt, dt;  // nkt = -1 / kT
   int64_t P, n_pairs, max_hops;
 };
 
-// Records of every (site, slot) from the slot tables (the workgroup
-// kernel's arithmetic: products and sums rounded one by one).
+// Records of every (site, slot) from the slot tables (products and sums
+// rounded one by one).
 __global__ void pack_slot_records(int64_t NM, const double* __restrict__ tself,
                                   const double* __restrict__ dphi,
                                   const double* __restrict__ lam,
@@ -450,390 +128,485 @@ __global__ void pack_site_pe(int64_t N, const double* __restrict__ phiL,
   if (k < N) pe[k] = make_double2(phiL[k], E[k]);
 }
 
-// One-wavefront instance with a row cache (used when it fits: n_c <= 64,
-// n_c z <= 256, z <= 8, the cache within the LDS of a workgroup and the
-// table below 4 GiB).
-//
-// Rows: process row p (p < n_c z) is the target site of process p, site row
-// c is carrier c's site.  The cache holds G[c][row] = A[x_row, occ_c] for
-// every carrier c and row, so psi[row] = sum_c q_c G[c][row] is summed from
-// LDS in carrier order: the FMA chain the workgroup kernel forms from its
-// gathers, so both give the same psi bit for bit.  When carrier m hops
-// s -> n only column m of the other rows changes (A[x_row, n], one gather
-// per row) and the mover's 1 + z rows are new (n_c gathers each): a hop
-// takes (1 + z)(2 n_c - 1) gathers instead of n_c (1 + z) n_c, all issued
-// together.  No gather address waits for another load: every process keeps
-// the z targets of its own target site (loaded when the process is made),
-// so the mover's new rows are in LDS when it is selected.
-//
-// Lane l owns processes l kNpl .. l kNpl + kNpl - 1 (the workgroup kernel's
-// split of the selection, so k_tot and the prefix are summed in the same
-// order) with their rate inputs in registers, site row l and carrier l's
-// displacement, path base and drift (l < n_c).  One wavefront: no workgroup
-// barriers; __syncthreads only waits for the wavefront's own LDS
-// operations.  Cheap per-lane work is done by every lane and kept by a
-// select rather than branched around; gathers of lanes that have no entry
-// to update read a valid address and are dropped.
 template <typename T>
 using gmem = const __attribute__((address_space(1))) T*;
 
-template <bool kCompact, int kNpl>
-__global__ void __launch_bounds__(64)
-kmc_wave_kernel(WaveArgs a, const KmcDev* __restrict__ dv,
-                int32_t* __restrict__ status) {
-  constexpr int kB = 5;  // (1 + z) n_c <= 320 mover-row gathers: 5 per lane
+// ---------------------------------------------------------------------------
+// Sums carried as an unevaluated pair h + l (about 106 bits), so that a sum
+// that is kept up by adding and taking away terms for the whole trajectory
+// stays the correctly rounded sum of its terms.
+struct Dd {
+  double h = 0.0, l = 0.0;
+};
+
+__device__ __forceinline__ void dd_add(Dd& a, double v) {
+#pragma clang fp contract(off)
+  const double s = a.h + v, b = s - a.h;
+  a.l += (a.h - (s - b)) + (v - b);
+  a.h = s;
+}
+
+// a += q v, the product's rounding error included.
+__device__ __forceinline__ void dd_add_prod(Dd& a, double q, double v) {
+#pragma clang fp contract(off)
+  const double p = q * v;
+  const double e = fma(q, v, -p);
+  dd_add(a, p);
+  a.l += e;
+}
+
+__device__ __forceinline__ void dd_add(Dd& a, const Dd& b) {
+#pragma clang fp contract(off)
+  dd_add(a, b.h);
+  a.l += b.l;
+}
+
+// h becomes the nearest double of the sum.
+__device__ __forceinline__ void dd_norm(Dd& a) {
+#pragma clang fp contract(off)
+  const double s = a.h + a.l;
+  a.l -= s - a.h;
+  a.h = s;
+}
+
+// A sum over each row of 16 lanes, in every lane of the row.
+template <int kRor>
+__device__ __forceinline__ void dd_rotate_add(Dd& a) {
+  Dd o;
+  o.h = dpp_f64<kDppRowRor + kRor, 0xf, true>(a.h);
+  o.l = dpp_f64<kDppRowRor + kRor, 0xf, true>(a.l);
+  dd_add(a, o);
+}
+
+__device__ __forceinline__ void dd_row_sum(Dd& a) {
+  dd_rotate_add<8>(a);
+  dd_rotate_add<4>(a);
+  dd_rotate_add<2>(a);
+  dd_rotate_add<1>(a);
+  dd_norm(a);
+}
+
+// f(std::integral_constant<int, n>) for the run-time n in [kMin, kMax],
+// small n first.
+template <int kMin, int kMax, typename F>
+__device__ __forceinline__ void with_count_up(int n, F&& f) {
+  if constexpr (kMin <= kMax) {
+    if (n == kMin)
+      f(std::integral_constant<int, kMin>{});
+    else
+      with_count_up<kMin + 1, kMax>(n, f);
+  }
+}
+
+// The hop loop.
+//
+// A block of wavefronts in three roles.  Process wavefronts: a lane owns a
+// process, its target row of psi and its rate inputs in registers.  Site
+// wavefronts: lane c owns carrier c's site row, displacement, path base and
+// drift; they keep the clock and write the path.  Helpers: the mover's new
+// rows.  psi[x] = sum_c q_c A[x, occ_c] of a row is a Dd that the hops keep
+// up: when carrier m hops s -> n every row gains q_m A[x, n] and loses
+// q_m A[x, s].  The mover's new site row continues the row of n; its z
+// slots are summed afresh by the helpers, four rows of 16 lanes at a time,
+// a lane over every 16th carrier.  A hop takes 2 n_c (1 + z) + z n_c
+// gathers in one round instead of the n_c (1 + z) n_c of summing every row,
+// and psi is the correctly rounded sum, where a chain over the carriers
+// carries a rounding per term.
+//
+// What bounds it is the chain of latencies of a hop: rates, their scan and
+// the selection, the LDS reads that the selected process names, one round
+// of gathers, the updates.  Two barriers per hop: after the rates, which
+// every wavefront sums and selects from by itself, and after the update;
+// both wait for LDS operations only.  What a hop changes in LDS that others
+// still read in its update (targets, sites) is written in the next hop's
+// rates phase.  With the look-ahead (every process's targets' targets in
+// LDS) no gather address waits for another load.
+//
+// Per hop, z = 4, before (n_c <= 64: one wavefront with every row's entries
+// in LDS; more: a workgroup that gathered them all again) and now: 1.40 and
+// 0.96 us with 1 carrier, 1.65 and 1.07 with 16 (6144 sites, 2600 cycles),
+// 21.6 and 1.5 with 96 (2592 sites).  At n_c = 16 a hop is about 660
+// cycles of rates, 660 of scan and selection, 700 to 1200 of LDS reads,
+// gathers and the clock, 200 of updates, the rest at the barriers; with 96
+// carriers the helper's z n_c gathers are the longest of the three.
+struct HopLds {
+  int nc, z, look;
+  __host__ __device__ int np() const { return nc * z; }
+  // rates of p at (p mod per) kStride + p / per, so that lane l's processes
+  // l per .. l per + per - 1 are read on distinct banks
+  static constexpr int kStride = 65;
+  __host__ __device__ int per() const { return (np() + 63) / 64; }
+  // psi of the site rows, charges, rates, dG0, hop vectors, the mover's
+  // rows; sites, targets and look-ahead with their codes; the end flag
+  __host__ __device__ size_t bytes() const {
+    return 8 * (2 * size_t(nc) + size_t(per()) * kStride + 4 * size_t(np()) +
+                2 * size_t(z) + 2) +
+           8 * (size_t(nc) + size_t(np()) + (look ? size_t(np()) * z : 0)) + 8;
+  }
+};
+
+// Wavefronts of each role: n_c z <= 640 processes, n_c <= 320 carriers.
+struct HopRoles {
+  int process, site, helper;
+  HopRoles() = default;
+  HopRoles(int nc, int z)
+      : process((nc * z + 63) / 64), site((nc + 63) / 64),
+        helper(z <= 4 ? 1 : z <= 8 ? 2 : 3) {}
+  int threads() const { return 64 * (process + site + helper); }
+};
+constexpr int kHopWaves = 16;  // at most
+
+template <bool kCompact, bool kLook>
+__global__ void __launch_bounds__(64 * kHopWaves)
+kmc_hop_kernel(HopArgs a, const KmcDev* __restrict__ dv, HopRoles roles,
+               int32_t* __restrict__ status) {
   extern __shared__ double smem[];
-  const int nc = a.nc, z = a.z, nproc = nc * z;
-  const int R = nproc + nc;
-  // carrier pairs of the cache, rounded up to whole groups of 4 (the
-  // padding's entries and charges are zero)
-  const int ncp = (((nc + 1) >> 1) + 3) & ~3;
-  const int lane = threadIdx.x;
   __shared__ double ext[64];  // 2^(j/64)
-  ext[lane] = __builtin_bit_cast(double, kExp2J64[lane]);
-  // cache: carriers 2p and 2p + 1 of a row side by side, so that one
-  // 16-byte read serves two terms of a row's sum
-  double2* G = reinterpret_cast<double2*>(smem);          // ncp x R
-  double* psis = reinterpret_cast<double*>(G + size_t(ncp) * R);  // nc
-  double* cqs = psis + nc;                                // 2 ncp
-  int32_t* occ = reinterpret_cast<int32_t*>(cqs + 2 * ncp);  // nc
-  uint32_t* opk = reinterpret_cast<uint32_t*>(occ + nc);  // nc
-  int32_t* tt = reinterpret_cast<int32_t*>(opk + nc);     // nproc z
-  uint32_t* ttpk = reinterpret_cast<uint32_t*>(tt + nproc * z);
-  auto gset = [&](int c, int row, double v) {
-    double* e = reinterpret_cast<double*>(G + size_t(c >> 1) * R + row);
-    e[c & 1] = v;
-  };
+  const int nc = a.nc, z = a.z, nproc = nc * z;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kT = blockDim.x;
+  const HopLds lay{nc, z, kLook ? 1 : 0};
+  const int per = lay.per();
+  double* psis = smem;                             // nc
+  double* cqs = psis + nc;                         // nc
+  double* kks = cqs + nc;                          // per kStride
+  double* dgs = kks + per * HopLds::kStride;       // nproc
+  double* pv3 = dgs + nproc;                       // 3 nproc
+  double* fresh = pv3 + 3 * nproc;                 // z pairs (h, l)
+  double* box = fresh + 2 * z;                     // psi[n] (h, l)
+  // sites with their packed codes (0 without cell-0 rows)
+  int2* occ = reinterpret_cast<int2*>(box + 2);    // carriers (nc)
+  int2* tgt = occ + nc;                            // targets (nproc)
+  int2* tt = tgt + nproc;                          // look-ahead (nproc z)
+  int* over = reinterpret_cast<int*>(tt + (kLook ? nproc * z : 0));
 
   // A[x, y]: the full table's row x, or (compact) the cell-0 row of x's
-  // sublattice at y moved by -cell(x); 32-bit byte offsets from the table's
-  // base (the host keeps the table below 4 GiB for this kernel)
-  auto entry = [&](int x, uint32_t xk, int y, uint32_t yk) -> double {
-    uint32_t off;
-    if constexpr (kCompact)
-      off = (xk >> 24) * a.row_bytes + rel_col(xk, yk, a.gp) * 8u;
-    else
-      off = uint32_t(x) * a.row_bytes + uint32_t(y) * 8u;
-    return *(gmem<double>)(a.tab + off);
+  // sublattice at y moved by -cell(x)
+  auto entry = [&](int2 x, int2 y) __attribute__((always_inline)) -> double {
+    if constexpr (kCompact) {
+      const uint32_t xk = uint32_t(x.y);
+      const uint32_t off =
+          (xk >> 24) * a.row_bytes + rel_col(xk, uint32_t(y.y), a.gp) * 8u;
+      return *(gmem<double>)(a.tab + off);
+    } else {
+      const uint64_t off = uint64_t(uint32_t(x.x)) * a.row_bytes +
+                           uint64_t(uint32_t(y.x)) * 8u;
+      return *(gmem<double>)(a.tab + off);
+    }
   };
-  // psi of this lane's rows (its processes' target rows and its site row):
-  // for each row the FMA chain over carriers 0 .. n_c - 1, the workgroup
-  // kernel's chain (the zero padding adds fma(q, 0, acc) = acc).  The cache
-  // entries of all the rows are read kC carrier pairs at a time before
-  // they are summed, so a group waits for the LDS once.  Rows of lanes
-  // without that process or carrier read row 0 and are not kept.
-  constexpr int kRows = kNpl + 1;
-  constexpr int kC = kRows <= 2 ? 4 : 2;  // divides the padded pair count
-  auto row_sums = [&](const int (&row)[kRows], double (&out)[kRows]) {
-    double acc[kRows];
-#pragma unroll
-    for (int r = 0; r < kRows; ++r) acc[r] = 0.0;
-    auto sum = [&](auto uniform_q) {
-      constexpr bool kUq = decltype(uniform_q)::value;
-      for (int p0 = 0; p0 < ncp; p0 += kC) {
-        double2 v[kC][kRows];
-#pragma unroll
-        for (int u = 0; u < kC; ++u)
-#pragma unroll
-          for (int r = 0; r < kRows; ++r)
-            v[u][r] = G[size_t(p0 + u) * R + row[r]];
-#pragma unroll
-        for (int u = 0; u < kC; ++u) {
-          const double q0 = kUq ? a.q0 : cqs[2 * (p0 + u)];
-          const double q1 = kUq ? a.q0 : cqs[2 * (p0 + u) + 1];
-#pragma unroll
-          for (int r = 0; r < kRows; ++r) {
-            acc[r] = fma(q0, v[u][r].x, acc[r]);
-            acc[r] = fma(q1, v[u][r].y, acc[r]);
-          }
-        }
-      }
-    };
-    if (a.uq) sum(std::true_type{});
-    else sum(std::false_type{});
-#pragma unroll
-    for (int r = 0; r < kRows; ++r) out[r] = acc[r];
+  // a barrier for what passes through LDS: loads in flight stay in flight
+  auto lds_barrier = [] {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  // the same site in every lane, in scalar registers
+  auto uniform = [](int2 v) {
+    return make_int2(__builtin_amdgcn_readfirstlane(v.x),
+                     __builtin_amdgcn_readfirstlane(v.y));
   };
 
-  // ---- processes of this lane: carrier, slot, target, rate inputs
-  int pc[kNpl], pj[kNpl], px[kNpl];
-  uint32_t pxk[kNpl];
-  bool pv[kNpl];
-  double pqs[kNpl], pdphi[kNpl], pts[kNpl], pEn[kNpl], pEs[kNpl], plam[kNpl],
-      pi4l[kNpl], pvs[kNpl], pvx[kNpl], pvy[kNpl], pvz[kNpl], pst[kNpl];
-  // the site-dependent part of process i's rate: slot j of site s, whose
-  // target is n.  Kept as loaded (the self term and both site energies,
-  // combined in the rate), so that nothing waits for these loads before
-  // the next hop's rates need them.
-  auto load_inputs = [&](int i, int s, int j, int n) {
-    const SlotRec& r = a.rec[int64_t(s) * a.mz + j];
-    const double2 ps = a.pe[s], pn = a.pe[n];
-    pdphi[i] = r.dphi;
-    pts[i] = r.tself;
-    pEn[i] = pn.y;
-    pEs[i] = ps.y;
-    plam[i] = r.lam;
-    pi4l[i] = r.i4l;
-    pvs[i] = r.vs;
-    pvx[i] = r.v[0];
-    pvy[i] = r.v[1];
-    pvz[i] = r.v[2];
-  };
-
-  for (int c = lane; c < nc; c += 64) {
+  if (tid < 64) ext[tid] = __builtin_bit_cast(double, kExp2J64[tid]);
+  if (tid == 0) *over = 0;
+  for (int c = tid; c < nc; c += kT) {
     const int s = dv->occ[c];
-    occ[c] = s;
-    opk[c] = kCompact ? dv->pk[s] : 0u;
+    occ[c] = make_int2(s, kCompact ? int(dv->pk[s]) : 0);
     cqs[c] = dv->cq[c];
   }
-  for (int c = nc + lane; c < 2 * ncp; c += 64) cqs[c] = 0.0;
-  // carrier `lane`'s displacement since the last path row, path base and
-  // drift (n_c <= 64)
+  // (the rates past the last process stay zero)
+  for (int k = tid; k < per * HopLds::kStride; k += kT) kks[k] = 0.0;
+  __syncthreads();
+  // every process's look-ahead: the z targets of its target
+  if constexpr (kLook)
+    for (int u = tid; u < nproc * z; u += kT) {
+      const int p = u / z, k = u - p * z;
+      const int c = p / z, j = p - c * z;
+      const int n = a.nbr2[int64_t(occ[c].x) * a.mz + j].x;
+      tt[u] = a.nbr2[int64_t(n) * a.mz + k];
+    }
+
+  // ---- hops made, the last selection
+  const KmcScalars sc0 = *dv->sc;
+  // hops that this call may make
+  int64_t due = a.n_pairs;
+  if (a.max_hops > 0)
+    due = min(due, max(a.max_hops - sc0.hops, int64_t(0)));
+  if (sc0.finished) due = 0;
+  int64_t h = 0;
+  int m = -1;  // the last hop's carrier (-1: none made yet)
+  int sel = 0, noselect = sc0.no_select;
+  double k_tot = 0.0, u1c = 0.0;
+  // sel / z = sel z_inv >> 16 for sel < 1024, z <= 64
+  const int z_inv = (65536 + z - 1) / z;
+  // lane l keeps the first uniform of hop (h & ~63) + l
+  auto take_u1 = [&]() __attribute__((always_inline)) {
+    if ((h & 63) == 0 && h + lane < a.n_pairs) u1c = a.U[2 * (h + lane)];
+  };
+  // k_tot and the selection: the first process whose cumulative rate
+  // exceeds u1 k_tot; lane l sums the processes l per .. l per + per - 1
+  // (the reference compares the cumulative sum of k / k_tot with u1: the
+  // same choice but where u1 lies within an ulp of a boundary)
+  auto select = [&]() __attribute__((always_inline)) {
+    sel = nproc - 1;  // rounding left no cum > u1: the last one
+    with_count_up<1, 10>(per, [&](auto n_per) __attribute__((always_inline)) {
+      constexpr int kP = decltype(n_per)::value;
+      double x[kP], ksum = 0.0;
+#pragma unroll
+      for (int i = 0; i < kP; ++i) {
+        x[i] = kks[i * HopLds::kStride + lane];
+        ksum = i == 0 ? x[0] : ksum + x[i];
+      }
+      const double incl = wave_incl_scan(ksum);
+      k_tot = read_lane(incl, 63);
+      const double thr = read_lane(u1c, int(h & 63)) * k_tot;
+      double cum = dpp_f64<kDppWaveShr1, 0xf, true>(incl);
+      // rates are not negative: a lane's running sums do not decrease, and
+      // the count of those <= thr is the index of its first crossing
+      int nb = 0;
+#pragma unroll
+      for (int i = 0; i < kP; ++i) {
+        cum += x[i];
+        nb += cum > thr ? 0 : 1;
+      }
+      const unsigned long long mask =
+          __ballot(nb < kP && lane * kP + nb < nproc);
+      if (mask) {
+        const int src = __ffsll(static_cast<long long>(mask)) - 1;
+        sel = src * kP + __builtin_amdgcn_readlane(nb, src);
+      } else {
+        ++noselect;
+      }
+    });
+    m = (sel * z_inv) >> 16;
+  };
+  // target k of the mover's new site
+  auto target = [&](int k) __attribute__((always_inline)) {
+    if constexpr (kLook) return tt[sel * z + k];
+    else return a.nbr2[int64_t(tgt[sel].x) * a.mz + k];
+  };
+  // the full sum of row x
+  auto row_sum = [&](int2 x) __attribute__((always_inline)) {
+    Dd r;
+    int c = 0;
+    for (; c + 8 <= nc; c += 8) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = entry(x, occ[c + u]);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) dd_add_prod(r, cqs[c + u], v[u]);
+    }
+    for (; c < nc; ++c) dd_add_prod(r, cqs[c], entry(x, occ[c]));
+    dd_norm(r);
+    return r;
+  };
+  // a row's update by the hop: its entries at the mover's new and old site
+  auto move = [](Dd& r, double q, double in, double out)
+                  __attribute__((always_inline)) {
+    dd_add_prod(r, q, in);
+    dd_add_prod(r, -q, out);
+    dd_norm(r);
+  };
+
+  if (wave < roles.process) {
+    // ================================================ process wavefronts
+    const bool pv = tid < nproc;
+    const int pp = pv ? tid : 0;
+    const int pk_at = (pp % per) * HopLds::kStride + pp / per;
+    const int pc = pp / z, pj = pp - pc * z;
+    const double pq = cqs[pc];
+    // the site-dependent part of the process's rate: slot j of site s,
+    // whose target is n.  Kept as loaded, so that nothing waits for these
+    // loads before the next hop's rates need them.
+    SlotRec r;
+    double En, Es;
+    auto load_inputs = [&](int s, int n) {
+      r = a.rec[int64_t(s) * a.mz + pj];
+      Es = a.pe[s].y;
+      En = a.pe[n].y;
+    };
+    auto post = [&](int2 x) {  // what a selected process is read by
+      tgt[pp] = x;
+      pv3[3 * pp] = r.v[0];
+      pv3[3 * pp + 1] = r.v[1];
+      pv3[3 * pp + 2] = r.v[2];
+    };
+    const int s0 = occ[pc].x;
+    int2 px = a.nbr2[int64_t(s0) * a.mz + pj];
+    load_inputs(s0, px.x);
+    Dd psi = row_sum(px);
+    if (pv) post(px);
+    __syncthreads();
+    for (; h < due;) {
+      take_u1();
+      // ---- the rate; the mover's rows are new
+      const bool mine = pc == m;
+      const double fh = fresh[2 * pj], fl = fresh[2 * pj + 1];
+      const double ps = psis[pc];
+      psi.h = mine ? fh : psi.h;
+      psi.l = mine ? fl : psi.l;
+      {
+        // products and sums rounded one by one, as NumPy forms them
+#pragma clang fp contract(off)
+        const double term01 = r.dphi + (psi.h - ps);
+        const double g0 = 2 * pq * (term01 + pq * r.tself) + (En - Es);
+        const double k = marcus_rate(g0, r.lam, r.i4l, r.vs, a.nkt, a.nu, ext);
+        if (pv) {
+          kks[pk_at] = k;
+          dgs[pp] = g0;
+        }
+      }
+      if (pv && mine) post(px);
+      const int last = *over;
+      lds_barrier();
+      if (last) break;
+      select();
+      // ---- one round of loads
+      int2 n = tgt[sel], s = occ[m];
+      const double qm = cqs[m];
+      const int2 tx = target(pj);
+      n = uniform(n);
+      s = uniform(s);
+      const double an = entry(px, n), as = entry(px, s);
+      // the mover's new process (its row comes with the next hop)
+      if (pc == m) {
+        px = tx;
+        load_inputs(n.x, px.x);
+      }
+      move(psi, qm, an, as);
+      if (pv && pp == sel) {
+        box[0] = psi.h;
+        box[1] = psi.l;
+        psis[m] = psi.h;
+      }
+      ++h;
+      lds_barrier();
+    }
+    return;
+  }
+
+  if (wave >= roles.process + roles.site) {
+    // ================================================ helpers
+    const int hw = wave - roles.process - roles.site;
+    const int fc = lane & 15;
+    // look-ahead load of this lane: target lk of the mover's new target lj
+    const int lu = 64 * hw + lane;
+    const bool la_on = kLook && lu < z * z;
+    const int lj = la_on ? lu / z : 0;
+    const int lk = la_on ? lu - lj * z : 0;
+    int2 la = make_int2(0, 0);
+    // a helper has the longest way from the selection to the barrier
+    __builtin_amdgcn_s_setprio(3);
+    // kF: carriers per lane whose sites and charges are kept here (the rest,
+    // past 128, read from LDS)
+    auto help = [&](auto n_f) __attribute__((always_inline)) {
+      constexpr int kF = decltype(n_f)::value;
+      int2 fo[kF];
+      double fq[kF];
+#pragma unroll
+      for (int u = 0; u < kF; ++u) {
+        const int c = fc + 16 * u;
+        fo[u] = occ[c < nc ? c : 0];
+        fq[u] = c < nc ? cqs[c] : 0.0;
+      }
+      __syncthreads();
+      while (h < due) {
+        take_u1();
+        if (la_on && m >= 0) tt[(m * z + lj) * z + lk] = la;
+        const int last = *over;
+        lds_barrier();
+        if (last) break;
+        select();
+        int2 n = tgt[sel];
+        const int2 lx = kLook ? target(lj) : n;
+        int k0 = 4 * hw;
+        int2 fx = target(k0 + (lane >> 4) < z ? k0 + (lane >> 4) : 0);
+        n = uniform(n);
+#pragma unroll
+        for (int u = 0; u < kF; ++u)
+          if (fc + 16 * u == m) fo[u] = n;
+        for (;;) {
+          const int k = k0 + (lane >> 4);
+          double e[kF];
+#pragma unroll
+          for (int u = 0; u < kF; ++u) e[u] = entry(fx, fo[u]);
+          if (la_on && k0 == 4 * hw) la = a.nbr2[int64_t(lx.x) * a.mz + lk];
+          Dd v;
+#pragma unroll
+          for (int u = 0; u < kF; ++u) dd_add_prod(v, fq[u], e[u]);
+          if constexpr (kF == 8)
+            for (int c = fc + 16 * kF; c < nc; c += 16)
+              dd_add_prod(v, cqs[c], entry(fx, c == m ? n : occ[c]));
+          dd_row_sum(v);
+          if (fc == 0 && k < z) {
+            fresh[2 * k] = v.h;
+            fresh[2 * k + 1] = v.l;
+          }
+          k0 += 4 * roles.helper;
+          if (k0 >= z) break;
+          fx = target(k0 + (lane >> 4) < z ? k0 + (lane >> 4) : 0);
+        }
+        ++h;
+        lds_barrier();
+      }
+    };
+    if (nc <= 16)
+      help(std::integral_constant<int, 1>{});
+    else if (nc <= 32)
+      help(std::integral_constant<int, 2>{});
+    else if (nc <= 64)
+      help(std::integral_constant<int, 4>{});
+    else
+      help(std::integral_constant<int, 8>{});
+    return;
+  }
+
+  // ================================================== site wavefronts
+  __builtin_amdgcn_s_setprio(1);
+  const int sw = wave - roles.process;
+  const int c = 64 * sw + lane;
+  const bool own = c < nc;  // (lanes past n_c keep carrier 0's row)
+  int2 sx = occ[own ? c : 0];
+  Dd psi = row_sum(sx);
   double dsp[3] = {0.0, 0.0, 0.0}, bse[3] = {0.0, 0.0, 0.0},
          drf[3] = {0.0, 0.0, 0.0};
-  if (lane < nc) {
+  if (own) {
+    psis[c] = psi.h;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      dsp[k] = dv->disp[3 * lane + k];
-      bse[k] = dv->base[3 * lane + k];
-      drf[k] = dv->drift[3 * lane + k];
+      dsp[k] = dv->disp[3 * c + k];
+      bse[k] = dv->base[3 * c + k];
+      drf[k] = dv->drift[3 * c + k];
     }
   }
-  __syncthreads();
-  int last_i = -1;
-#pragma unroll
-  for (int i = 0; i < kNpl; ++i) {
-    const int p = lane * kNpl + i;
-    pv[i] = p < nproc;
-    pc[i] = pv[i] ? p / z : 0;
-    pj[i] = pv[i] ? p - pc[i] * z : 0;
-    pqs[i] = cqs[pc[i]];
-    px[i] = 0;
-    pxk[i] = 0u;
-    pst[i] = 0.0;
-    if (pv[i]) {
-      last_i = i;
-      const int s = occ[pc[i]];
-      const int2 t = a.nbr2[int64_t(s) * a.mz + pj[i]];
-      px[i] = t.x;
-      pxk[i] = uint32_t(t.y);
-      load_inputs(i, s, pj[i], t.x);
-    } else {
-      pdphi[i] = pts[i] = pEn[i] = pEs[i] = pvs[i] = 0.0;
-      plam[i] = 1.0;
-      pi4l[i] = 0.25;
-      pvx[i] = pvy[i] = pvz[i] = 0.0;
-    }
-  }
-  // every process's look-ahead: the z targets of its target
-  for (int u = lane; u < nproc * z; u += 64) {
-    const int p = u / z, k = u - p * z;
-    const int c = p / z, j = p - c * z;
-    const int n = a.nbr2[int64_t(occ[c]) * a.mz + j].x;
-    const int2 t = a.nbr2[int64_t(n) * a.mz + k];
-    tt[u] = t.x;
-    ttpk[u] = uint32_t(t.y);
-  }
-  // the cache, every (carrier, row); the pairs past n_c stay zero
-  for (int u = lane; u < ncp * R; u += 64)
-    G[u] = make_double2(0.0, 0.0);
-  __syncthreads();
-  for (int u = lane; u < nc * R; u += 64) {
-    const int row = u / nc, c = u - row * nc;
-    int x;
-    uint32_t xk;
-    if (row < nproc) {
-      const int c2 = row / z, j2 = row - c2 * z;
-      const int2 t = a.nbr2[int64_t(occ[c2]) * a.mz + j2];
-      x = t.x;
-      xk = uint32_t(t.y);
-    } else {
-      x = occ[row - nproc];
-      xk = opk[row - nproc];
-    }
-    gset(c, row, entry(x, xk, occ[c], opk[c]));
-  }
-  // site row of this lane (lanes past n_c keep carrier 0's, never stored)
-  int sx = occ[lane < nc ? lane : 0];
-  uint32_t sxk = opk[lane < nc ? lane : 0];
-  __syncthreads();
-  // this lane's rows and where their sums go
-  auto lane_sums = [&]() {
-    int row[kRows];
-    double out[kRows];
-#pragma unroll
-    for (int i = 0; i < kNpl; ++i) row[i] = pv[i] ? lane * kNpl + i : 0;
-    row[kNpl] = lane < nc ? nproc + lane : 0;
-    row_sums(row, out);
-#pragma unroll
-    for (int i = 0; i < kNpl; ++i)
-      if (pv[i]) pst[i] = out[i];
-    if (lane < nc) psis[lane] = out[kNpl];
-  };
-  lane_sums();
-  // the mover-row gathers this lane takes: row brl (0: the mover's site,
-  // 1 + j: its target j) at carrier bc; nb of the kB rounds hold any
-  int brl[kB], bc[kB];
-#pragma unroll
-  for (int k = 0; k < kB; ++k) {
-    const int u = lane + 64 * k;
-    brl[k] = u < (1 + z) * nc ? u / nc : -1;
-    bc[k] = brl[k] >= 0 ? u - brl[k] * nc : 0;
-  }
-  const int nb = ((1 + z) * nc + 63) / 64;
-  // look-ahead load of this lane: target lk of the mover's new target lj
-  const bool la_on = lane < z * z;
-  const int lj = la_on ? lane / z : 0;
-  const int lk = la_on ? lane - lj * z : 0;
-  __syncthreads();
-
-  const KmcScalars sc0 = *dv->sc;
   double t = sc0.t, energy = sc0.energy;
-  int64_t start = sc0.start, hops = sc0.hops;
-  int noselect = sc0.no_select;
-  int stop = sc0.finished ? 1 : 0;
-  int code = stop ? 0 : -1;
-  int64_t h = 0;
-  double u1c = 0.0, u2c = 0.0, luc = 0.0;
-  // hop log of the current block of 64 hops: lane l holds hop (h & ~63) + l
+  int64_t start = sc0.start;
+  bool stop = sc0.finished != 0;
+  const double inv_dt = 1.0 / a.dt;
+  double u2c = 0.0, luc = 0.0;  // second uniforms, as u1c
+  // hop log of a block of 64 hops: lane l holds hop (h & ~63) + l
   double tlog = 0.0;
   int32_t plog = 0;
   auto flush_log = [&](int64_t block, int count) {
-    if (lane < count) {
+    if (sw == 0 && lane < count) {
       if (a.hop_time) a.hop_time[block + lane] = tlog;
       if (a.hop_proc) a.hop_proc[block + lane] = plog;
     }
   };
-  while (!stop) {
-    if (a.max_hops > 0 && hops >= a.max_hops) {
-      code = 0;
-      break;
-    }
-    if (h >= a.n_pairs) {
-      code = 1;  // need uniforms
-      break;
-    }
+  // clock, energy, log and path rows of hop h
+  auto tick = [&](double g_sel) {
     const int hl = int(h & 63);
-    if (hl == 0) {
-      // lane l keeps the uniforms of hop h + l
-      const int64_t q = h + lane;
-      if (q < a.n_pairs) {
-        u1c = a.U[2 * q];
-        u2c = a.U[2 * q + 1];
-        luc = a.LU[q];
-      }
-    }
-    // ---- rates of this lane's processes
-    double kk[kNpl], gg[kNpl];
-    double ksum = 0.0;
-#pragma unroll
-    for (int i = 0; i < kNpl; ++i) {
-      // products and sums rounded one by one, as NumPy forms them (and as
-      // the workgroup kernel does, whose rates pass through LDS)
-#pragma clang fp contract(off)
-      kk[i] = 0.0;
-      gg[i] = 0.0;
-      if (pv[i]) {
-        const double term01 = pdphi[i] + (pst[i] - psis[pc[i]]);
-        const double g0 =
-            2 * pqs[i] * (term01 + pqs[i] * pts[i]) + (pEn[i] - pEs[i]);
-        kk[i] = marcus_rate(g0, plam[i], pi4l[i], pvs[i], a.nkt, a.nu, ext);
-        gg[i] = g0;
-        ksum += kk[i];
-      }
-    }
-    // ---- k_tot and the selection: the first process whose cumulative
-    // rate exceeds u1 k_tot (the workgroup kernel's order of sums)
-    const double incl = wave_incl_scan(ksum);
-    const double k_tot = read_lane(incl, 63);
-    const double u1 = read_lane(u1c, hl);
-    const double u2 = read_lane(u2c, hl);
-    const double lu = read_lane(luc, hl);
-    const double thr = u1 * k_tot;
-    double cum = dpp_f64<kDppWaveShr1, 0xf, true>(incl);
-    int found = -1;
-#pragma unroll
-    for (int i = 0; i < kNpl; ++i) {
-      if (pv[i] && found < 0) {
-        cum += kk[i];
-        if (cum > thr) found = i;
-      }
-    }
-    const unsigned long long mask = __ballot(found >= 0);
-    int src;
-    if (mask) {
-      src = __ffsll(static_cast<long long>(mask)) - 1;
-    } else {
-      src = (nproc - 1) / kNpl;  // rounding left no cum > u1: the last one
-      ++noselect;
-    }
-    const int mi = found >= 0 ? found : last_i;
-    double k_my = kk[0], g_my = gg[0], vx_my = pvx[0], vy_my = pvy[0],
-           vz_my = pvz[0];
-    int c_my = pc[0], x_my = px[0];
-    uint32_t xk_my = pxk[0];
-#pragma unroll
-    for (int i = 1; i < kNpl; ++i) {
-      if (mi == i) {
-        k_my = kk[i];
-        g_my = gg[i];
-        vx_my = pvx[i];
-        vy_my = pvy[i];
-        vz_my = pvz[i];
-        c_my = pc[i];
-        x_my = px[i];
-        xk_my = pxk[i];
-      }
-    }
-    const int sel = __builtin_amdgcn_readlane(lane * kNpl + mi, src);
-    const int m = __builtin_amdgcn_readlane(c_my, src);
-    const int n = __builtin_amdgcn_readlane(x_my, src);
-    const uint32_t npk = uint32_t(__builtin_amdgcn_readlane(int(xk_my), src));
-    const double k_sel = read_lane(k_my, src);
-    const double g_sel = read_lane(g_my, src);
-    const double v_sel[3] = {read_lane(vx_my, src), read_lane(vy_my, src),
-                             read_lane(vz_my, src)};
-
-    // ---- one round of loads: column m of the other rows, the mover's new
-    // rows, the rate inputs of its new processes and their look-ahead
-    const int tsel = sel * z;  // the mover's new targets: tt[tsel + j]
-    double ga[kNpl];
-#pragma unroll
-    for (int i = 0; i < kNpl; ++i) ga[i] = entry(px[i], pxk[i], n, npk);
-    const double gs_site = entry(sx, sxk, n, npk);
-    // every round's LDS inputs read first, then every round's gather
-    // issued, unused rounds included (they read a valid entry that is not
-    // kept): no load then sits behind another round's LDS wait, and every
-    // load lands in its own register, so nothing waits for the gathers
-    // before the cache is written
-    int gx[kB], gy[kB];
-    uint32_t gxk[kB], gyk[kB];
-#pragma unroll
-    for (int k = 0; k < kB; ++k) {
-      const int rl = brl[k] > 0 ? brl[k] : 0;
-      const int ti = tsel + (rl > 0 ? rl - 1 : 0);
-      const int tx = tt[ti];
-      const uint32_t txk = ttpk[ti];
-      const int cc = bc[k];
-      const int oy = occ[cc];
-      const uint32_t oyk = opk[cc];
-      gx[k] = rl > 0 ? tx : n;
-      gxk[k] = rl > 0 ? txk : npk;
-      gy[k] = cc == m ? n : oy;
-      gyk[k] = cc == m ? npk : oyk;
-    }
-    double gb[kB];
-#pragma unroll
-    for (int k = 0; k < kB; ++k) gb[k] = entry(gx[k], gxk[k], gy[k], gyk[k]);
-    const int2 la = a.nbr2[int64_t(tt[tsel + lj]) * a.mz + lk];
-
-    // ---- clock, energy and path bookkeeping (uniform), while the loads
-    // are in flight
     int64_t end;
-    if (u2 > 0.0) {
-      t -= lu / k_tot;
-      const double qd = t / a.dt;
-      end = qd < 9.0e18 ? int64_t(qd) : a.P;
+    if (read_lane(u2c, hl) > 0.0) {
+      t -= read_lane(luc, hl) / k_tot;
+      // path step int(t / dt) of the correctly rounded quotient: below 1e6,
+      // t (1/dt) is within 4e-10 of it, so more than 1e-9 away from an
+      // integer its integer part is the quotient's; otherwise divide
+      const double qf = t * inv_dt, fl = floor(qf), fr = qf - fl;
+      if (fr > 1e-9 && fr < 1.0 - 1e-9 && qf < 1.0e6) {
+        end = int(fl);
+      } else {
+        const double qd = t / a.dt;
+        end = qd < 9.0e18 ? int64_t(qd) : a.P;
+      }
     } else {
       t = INFINITY;
       end = a.P;
@@ -841,106 +614,96 @@ kmc_wave_kernel(WaveArgs a, const KmcDev* __restrict__ dv,
     energy += g_sel;
     tlog = lane == hl ? t : tlog;
     plog = lane == hl ? sel : plog;
-    const int64_t row_lo = start;
-    int64_t row_hi = start;
-    if (end >= start + 1) row_hi = end >= a.P ? a.P : end;
+    if (hl == 63) flush_log(h - 63, 64);
+    if (end < start + 1) return;
     const int64_t dp_hi = min(end, a.P);
-    ++hops;
-    // loop condition of the reference: continue while end < P
-    stop = (row_hi > row_lo && row_hi >= a.P) ? 1 : 0;
-    {
-      // the mover's displacement and drift, in lane m
-#pragma clang fp contract(off)
-      const bool me = lane == m;
+    if (end >= a.P) end = a.P;
+    if (sw == 0) {
+      for (int64_t r = start + lane; r < dp_hi; r += 64) a.dpath[r] = g_sel;
+      for (int64_t r = start + lane; r < end; r += 64) a.epath[r] = energy;
+    }
+    if (own) {
+      const int w = 3 * nc;
+      for (int64_t r = start; r < end; ++r)
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          a.rows[r * w + 3 * c + k] = bse[k] + dsp[k];
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
-        dsp[k] = me ? dsp[k] + v_sel[k] : dsp[k];
-        if (a.field_on) drf[k] = me ? drf[k] + v_sel[k] * k_sel : drf[k];
+        bse[k] += dsp[k];
+        dsp[k] = 0.0;
       }
     }
-    if (lane == 0) {
-      occ[m] = n;
-      opk[m] = npk;
+    start = end;
+    // loop condition of the reference: continue while end < P
+    stop = end >= a.P;
+    if (stop && c == 0) *over = 1;
+  };
+  __syncthreads();
+  while (h < due) {
+    take_u1();
+    if ((h & 63) == 0 && h + lane < a.n_pairs) {
+      u2c = a.U[2 * (h + lane) + 1];
+      luc = a.LU[h + lane];
     }
-    if (lane == m) {
+    // ---- what the last hop left
+    if (c == m) {
+      psi.h = box[0];
+      psi.l = box[1];
+      occ[m] = sx;
+    }
+    lds_barrier();
+    if (stop) break;
+    select();
+    int2 n = tgt[sel], s = occ[m];
+    const double qm = cqs[m];
+    const double g_sel = dgs[sel];
+    const double k_sel = kks[(sel % per) * HopLds::kStride + sel / per];
+    double v[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) v[k] = pv3[3 * sel + k];
+    n = uniform(n);
+    s = uniform(s);
+    const double bn = entry(sx, n), bs = entry(sx, s);
+    if (c == m) {
+#pragma clang fp contract(off)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        dsp[k] = dsp[k] + v[k];
+        if (a.field_on) drf[k] = drf[k] + v[k] * k_sel;
+      }
+    }
+    tick(g_sel);  // while the gathers are in flight
+    move(psi, qm, bn, bs);
+    if (c == m)  // continued from the row of n, see box
       sx = n;
-      sxk = npk;
-    }
-    // the rate inputs of the mover's new processes (after the uniform work
-    // above, so that it overlaps the loads)
-#pragma unroll
-    for (int i = 0; i < kNpl; ++i) {
-      if (pv[i] && pc[i] == m) {
-        const int nn = tt[tsel + pj[i]];
-        px[i] = nn;
-        pxk[i] = ttpk[tsel + pj[i]];
-        load_inputs(i, n, pj[i], nn);
-      }
-    }
-    // ---- the cache: column m of the other rows first, then the mover's
-    // rows (which overwrite what the first writes put in them)
-#pragma unroll
-    for (int i = 0; i < kNpl; ++i)
-      if (pv[i]) gset(m, lane * kNpl + i, ga[i]);
-    if (lane < nc) gset(m, nproc + lane, gs_site);
-#pragma unroll
-    for (int k = 0; k < kB; ++k) {
-      if (k < nb && brl[k] >= 0) {
-        const int row = brl[k] == 0 ? nproc + m : m * z + brl[k] - 1;
-        gset(bc[k], row, gb[k]);
-      }
-    }
-    if (la_on) {
-      tt[(m * z + lj) * z + lk] = la.x;
-      ttpk[(m * z + lj) * z + lk] = uint32_t(la.y);
-    }
-    __syncthreads();
-    lane_sums();
-    __syncthreads();
-    // ---- path-step outputs, for a hop that ends one or more path steps
-    if (row_hi > row_lo) {
-      for (int64_t r = row_lo + lane; r < dp_hi; r += 64) a.dpath[r] = g_sel;
-      for (int64_t r = row_lo + lane; r < row_hi; r += 64) a.epath[r] = energy;
-      if (lane < nc) {
-        const int w = 3 * nc;
-        for (int64_t r = row_lo; r < row_hi; ++r)
-#pragma unroll
-          for (int k = 0; k < 3; ++k) a.rows[r * w + 3 * lane + k] =
-              bse[k] + dsp[k];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          bse[k] += dsp[k];
-          dsp[k] = 0.0;
-        }
-      }
-      start = row_hi;
-    }
-    if (hl == 63) flush_log(h - 63, 64);
+    else if (own)
+      psis[c] = psi.h;
     ++h;
-    if (stop) code = 0;
+    lds_barrier();
   }
   // ---- write the state back
   flush_log(h & ~int64_t(63), int(h & 63));
-  __syncthreads();
-  for (int c = lane; c < nc; c += 64) dv->occ[c] = occ[c];
-  if (lane < nc) {
+  if (own) {
+    dv->occ[c] = sx.x;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      dv->disp[3 * lane + k] = dsp[k];
-      dv->base[3 * lane + k] = bse[k];
-      dv->drift[3 * lane + k] = drf[k];
+      dv->disp[3 * c + k] = dsp[k];
+      dv->base[3 * c + k] = bse[k];
+      dv->drift[3 * c + k] = drf[k];
     }
   }
-  if (lane == 0) {
+  if (c == 0) {
     KmcScalars o = sc0;
     o.t = t;
     o.energy = energy;
     o.start = start;
-    o.hops = hops;
+    o.hops = sc0.hops + h;
     o.no_select = noselect;
     if (stop) o.finished = 1;
     *dv->sc = o;
-    status[0] = code;
+    // ended by its path or its hop count, or more uniforms are needed
+    status[0] = stop || (a.max_hops > 0 && o.hops >= a.max_hops) ? 0 : 1;
     status[1] = int32_t(h);
   }
 }
@@ -1095,22 +858,21 @@ struct pycd_kmc {
   Geo geo{};
   DevBuf<double> Ac;
   DevBuf<uint32_t> pk, nbr_pk;
-  // one-wavefront kernel: slot records, (phi_L, E) per site, targets with
-  // their codes, the device copy of the kernel's state pointers
+  // slot records, (phi_L, E) per site, targets with their codes, the device
+  // copy of the kernel's state pointers
   DevBuf<SlotRec> rec;
   DevBuf<double2> pe;
   DevBuf<int2> nbr2;
   DevBuf<KmcDev> dev;
   double qLAqL = 0.0;
-  size_t smem = 0;
-  // one-wavefront row-cache kernel: whether it fits, its LDS, processes
-  // per lane, and which kernel the hop loop runs (PYCD_KMC_*)
+  // the hop loop's roles, its look-ahead and its LDS
+  HopRoles hop_roles{};
+  int hop_look = 0;
+  size_t hop_smem = 0;
+  // PYCD_KMC_WAVE may be named, and what was named
   bool wave_ok = false;
   size_t wave_smem = 0;
-  int wave_npl = 0;
   int32_t variant = PYCD_KMC_AUTO;
-  bool uniform_q = false;  // every carrier has charge q0
-  double q0 = 0.0;
   bool begun = false;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms = 0.0;
@@ -1194,9 +956,10 @@ periodic_gap(const double* __restrict__ A, const double* __restrict__ Ac,
 // table equals its cell-0 translate to kTranslationTol of the table's
 // scale (a NaN anywhere fails);
 // otherwise the loop reads the full table.  Smaller tables stay in the
-// caches whole, and there the column arithmetic costs more than it saves
-// (768 sites: 3.51 us per hop on the full table, 3.65 on cell-0 rows;
-// 6144 sites, 302 MB: 3.94 and 3.60).
+// caches whole, and there the two are near each other (768 sites, 8 and 32
+// carriers: 1.12 and 1.28 us per hop on the full table, 1.07 and 1.29 on
+// cell-0 rows); above, the full table's misses show (2592 sites, 16
+// carriers: 1.26 and 1.07; 6144 sites: 1.39 and 1.08).
 constexpr int64_t kCellRowsFrom = int64_t(32) << 20;
 hipError_t compact_setup(pycd_kmc* s, const std::vector<int32_t>& nb) {
   const pycd_kmc_problem& pb = s->pb;
@@ -1256,9 +1019,9 @@ hipError_t compact_setup(pycd_kmc* s, const std::vector<int32_t>& nb) {
   return hipSuccess;
 }
 
-// Slot records, targets and (phi_L, E) pairs of every site for the
-// one-wavefront kernel, from the slot tables and the lattice terms.
-hipError_t pack_wave_inputs(pycd_kmc* s) {
+// Slot records, targets and (phi_L, E) pairs of every site, from the slot
+// tables and the lattice terms.
+hipError_t pack_hop_inputs(pycd_kmc* s) {
   hipStream_t st = s->ctx->stream;
   const int64_t N = s->pb.n_sites;
   const int64_t NM = N * s->pb.max_z;
@@ -1275,11 +1038,11 @@ hipError_t pack_wave_inputs(pycd_kmc* s) {
   return hipGetLastError();
 }
 
-// LDS of the one-wavefront kernel: the row cache (carrier pairs, rounded
-// up to groups of 4, x (n_c z + n_c) rows of 16 bytes), site-row psi
-// (n_c doubles) and charges (one per padded carrier), carrier sites and
-// their codes, and each process's look-ahead (2 n_c z z words).  0 when
-// the instance does not apply.
+// The sessions for which PYCD_KMC_WAVE can be named: those of few enough
+// carriers for one wavefront to keep every table entry that a hop reads in
+// LDS (entries of carrier pairs in groups of 4 for n_c z + n_c rows, psi and
+// charges, sites with codes, z z targets per carrier).  0 for the others.
+// Both names run the same kernel.
 size_t wave_lds_bytes(int nc, int z) {
   const int nproc = nc * z;
   if (nc > 64 || nproc > 256 || z > 8) return 0;
@@ -1340,7 +1103,6 @@ extern "C" int pycd_kmc_create(pycd_ctx* ctx, const pycd_kmc_problem* pb,
   if (!s) return PYCD_ERR_NOMEM;
   s->ctx = ctx;
   s->pb = *pb;
-  s->smem = smem;
   hipStream_t st = ctx->stream;
   auto bail = [&](int code) {
     delete s;
@@ -1384,18 +1146,6 @@ extern "C" int pycd_kmc_create(pycd_ctx* ctx, const pycd_kmc_problem* pb,
   S_HIP(upload(s->vab.ptr, pb->nbr_vab, NM, st));
   S_HIP(upload(s->E.ptr, pb->site_energy, N, st));
   S_HIP(upload(s->cq.ptr, pb->carrier_q, nc, st));
-  {
-    std::vector<double> cq(nc);
-    if (is_device_ptr(pb->carrier_q)) {
-      S_HIP(hipMemcpy(cq.data(), pb->carrier_q, 8 * size_t(nc),
-                      hipMemcpyDeviceToHost));
-    } else {
-      std::memcpy(cq.data(), pb->carrier_q, 8 * size_t(nc));
-    }
-    s->q0 = cq[0];
-    s->uniform_q = true;
-    for (double v : cq) s->uniform_q = s->uniform_q && v == cq[0];
-  }
   self_term_kernel<<<int((NM + 255) / 256), 256, 0, st>>>(s->A.ptr, s->nbr.ptr,
                                                          N, mz, s->tself.ptr);
   S_HIP(hipGetLastError());
@@ -1405,17 +1155,21 @@ extern "C" int pycd_kmc_create(pycd_ctx* ctx, const pycd_kmc_problem* pb,
   S_HIP(s->nbr2.alloc(NM));
   S_HIP(s->pe.alloc(size_t(N)));
   S_HIP(s->dev.alloc(1));
-  S_HIP(pack_wave_inputs(s));
+  S_HIP(pack_hop_inputs(s));
   {
     int lds_max = 0;
     S_HIP(hipDeviceGetAttribute(&lds_max,
                                 hipDeviceAttributeMaxSharedMemoryPerBlock,
                                 ctx->device));
     s->wave_smem = wave_lds_bytes(nc, z);
-    s->wave_npl = (nc * z + 63) / 64;
-    // the kernel addresses the table with 32-bit byte offsets
+    s->hop_roles = HopRoles(nc, z);
+    HopLds hl{nc, z, z * z <= 64 * s->hop_roles.helper ? 1 : 0};
+    if (hl.bytes() + 512 > size_t(lds_max)) hl.look = 0;
+    s->hop_look = hl.look;
+    s->hop_smem = hl.bytes();
+    // (512 bytes of 2^(j/64) beside the dynamic part; one wavefront's 32-bit
+    // table offsets)
     const double tab_bytes = 8.0 * double(s->compact ? s->geo.nu : N) * N;
-    // (the kernel's own 512 bytes of 2^(j/64) beside the dynamic part)
     s->wave_ok = s->wave_smem > 0 && s->wave_smem + 512 <= size_t(lds_max) &&
                  tab_bytes < 4294967296.0;
   }
@@ -1466,7 +1220,7 @@ extern "C" int pycd_kmc_set_sites(pycd_kmc* s, const double* lattice_q,
   PYCD_HIP(ctx, upload(s->qL.ptr, lattice_q, N, st));
   PYCD_HIP(ctx, upload(s->E.ptr, site_energy, N, st));
   PYCD_HIP(ctx, lattice_terms(s));
-  PYCD_HIP(ctx, pack_wave_inputs(s));
+  PYCD_HIP(ctx, pack_hop_inputs(s));
   return PYCD_OK;
 }
 
@@ -1540,42 +1294,35 @@ extern "C" int pycd_kmc_begin(pycd_kmc* s, const int64_t* occupancy,
 
 namespace {
 
-template <bool kCompact, int kNpl>
-hipError_t launch_wave_t(size_t smem, hipStream_t st, const WaveArgs& wa,
-                         const KmcDev* dv, int32_t* status) {
-  if (smem > 65536) {
+template <bool kCompact, bool kLook>
+hipError_t launch_hop_t(const pycd_kmc* s, hipStream_t st, const HopArgs& args,
+                        int32_t* status) {
+  if (s->hop_smem > 65536) {
     hipError_t e = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&kmc_wave_kernel<kCompact, kNpl>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, int(smem));
+        reinterpret_cast<const void*>(&kmc_hop_kernel<kCompact, kLook>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, int(s->hop_smem));
     if (e != hipSuccess) return e;
   }
-  kmc_wave_kernel<kCompact, kNpl><<<1, 64, smem, st>>>(wa, dv, status);
+  kmc_hop_kernel<kCompact, kLook>
+      <<<1, s->hop_roles.threads(), s->hop_smem, st>>>(args, s->dev.ptr,
+                                                       s->hop_roles, status);
   return hipGetLastError();
 }
 
-template <bool kCompact>
-hipError_t launch_wave_c(int npl, size_t smem, hipStream_t st,
-                         const WaveArgs& wa, const KmcDev* dv,
-                         int32_t* status) {
-  switch (npl) {
-    case 1:
-      return launch_wave_t<kCompact, 1>(smem, st, wa, dv, status);
-    case 2:
-      return launch_wave_t<kCompact, 2>(smem, st, wa, dv, status);
-    case 3:
-      return launch_wave_t<kCompact, 3>(smem, st, wa, dv, status);
-    case 4:
-      return launch_wave_t<kCompact, 4>(smem, st, wa, dv, status);
-    default:
-      return hipErrorInvalidValue;
-  }
-}
-
-hipError_t launch_wave(bool compact, int npl, size_t smem, hipStream_t st,
-                       const WaveArgs& wa, const KmcDev* dv,
-                       int32_t* status) {
-  return compact ? launch_wave_c<true>(npl, smem, st, wa, dv, status)
-                 : launch_wave_c<false>(npl, smem, st, wa, dv, status);
+hipError_t launch_hop(const pycd_kmc* s, hipStream_t st, const HopArgs& args,
+                      int32_t* status) {
+  // every process and carrier is owned by a lane; the kernel sums at most
+  // 10 processes per lane
+  const HopRoles& r = s->hop_roles;
+  if (r.threads() > 64 * kHopWaves || r.process > 10 ||
+      64 * r.process < s->pb.n_carriers * s->pb.z ||
+      64 * r.site < s->pb.n_carriers)
+    return hipErrorInvalidValue;
+  if (s->compact)
+    return s->hop_look ? launch_hop_t<true, true>(s, st, args, status)
+                       : launch_hop_t<true, false>(s, st, args, status);
+  return s->hop_look ? launch_hop_t<false, true>(s, st, args, status)
+                     : launch_hop_t<false, false>(s, st, args, status);
 }
 
 }  // namespace
@@ -1671,85 +1418,41 @@ int hop_loop(pycd_kmc* s, const double* dU, double* LU, int32_t* status_dev,
   pycd_ctx* ctx = s->ctx;
   hipStream_t st = ctx->stream;
   const pycd_kmc_problem& pb = s->pb;
-  KmcDev d;
-  d.A = s->A.ptr;
-  d.Ac = s->Ac.ptr;
-  d.pk = s->pk.ptr;
-  d.nbr_pk = s->nbr_pk.ptr;
-  d.gp = geo_pk(s->compact ? s->geo : Geo{1, 1, 1, 1});
-  d.phiL = s->phiL.ptr;
-  d.dphi = s->dphi.ptr;
-  d.nbr = s->nbr.ptr;
-  d.vec = s->vec.ptr;
-  d.lam = s->lam.ptr;
-  d.vab = s->vab.ptr;
-  d.tself = s->tself.ptr;
-  d.E = s->E.ptr;
-  d.cq = s->cq.ptr;
-  d.N = pb.n_sites;
-  d.nc = pb.n_carriers;
-  d.z = pb.z;
-  d.max_z = pb.max_z;
-  d.field_on = (pb.field[0] != 0.0 || pb.field[1] != 0.0 || pb.field[2] != 0.0);
-  for (int a = 0; a < 3; ++a) d.field[a] = pb.field[a];
-  d.nu = pb.nu;
-  d.kT = pb.kT;
-  d.nkt = -1.0 / pb.kT;
-  d.dt = pb.time_interval;
-  d.P = pb.n_path;
-  d.occ = s->occ.ptr;
-  d.disp = s->disp.ptr;
-  d.base = s->base.ptr;
-  d.drift = s->drift.ptr;
-  d.rows = s->rows.ptr;
-  d.epath = s->epath.ptr;
-  d.dpath = s->dpath.ptr;
-  d.sc = s->sc.ptr;
+  const KmcDev d{s->pk.ptr,    s->cq.ptr,    s->occ.ptr, s->disp.ptr,
+                 s->base.ptr, s->drift.ptr, s->sc.ptr};
+  HopArgs args;
+  args.tab = reinterpret_cast<const char*>(s->compact ? s->Ac.ptr : s->A.ptr);
+  args.row_bytes = uint32_t(pb.n_sites) * uint32_t(sizeof(double));
+  args.gp = geo_pk(s->compact ? s->geo : Geo{1, 1, 1, 1});
+  args.rec = s->rec.ptr;
+  args.pe = s->pe.ptr;
+  args.nbr2 = s->nbr2.ptr;
+  args.rows = s->rows.ptr;
+  args.epath = s->epath.ptr;
+  args.dpath = s->dpath.ptr;
+  args.U = dU;
+  args.LU = LU;
+  args.hop_time = dT;
+  args.hop_proc = dP;
+  args.nc = pb.n_carriers;
+  args.z = pb.z;
+  args.mz = pb.max_z;
+  args.field_on =
+      pb.field[0] != 0.0 || pb.field[1] != 0.0 || pb.field[2] != 0.0;
+  args.nu = pb.nu;
+  args.nkt = -1.0 / pb.kT;
+  args.dt = pb.time_interval;
+  args.P = pb.n_path;
+  args.n_pairs = n_pairs;
+  args.max_hops = max_hops;
   if (timed) PYCD_HIP(ctx, hipEventRecord(s->ev0, st));
   reset_status<<<1, 1, 0, st>>>(status_dev);
   if (n_pairs > 0)
     log_u2_kernel<<<int(std::min<int64_t>((n_pairs + 255) / 256, 4096)), 256,
                     0, st>>>(dU, n_pairs, LU);
-  const bool wave = s->variant == PYCD_KMC_WAVE ||
-                    (s->variant == PYCD_KMC_AUTO && s->wave_ok);
-  if (wave) {
-    WaveArgs wa;
-    wa.tab = reinterpret_cast<const char*>(s->compact ? s->Ac.ptr : s->A.ptr);
-    wa.row_bytes = uint32_t(pb.n_sites) * uint32_t(sizeof(double));
-    wa.gp = d.gp;
-    wa.rec = s->rec.ptr;
-    wa.pe = s->pe.ptr;
-    wa.nbr2 = s->nbr2.ptr;
-    wa.rows = d.rows;
-    wa.epath = d.epath;
-    wa.dpath = d.dpath;
-    wa.U = dU;
-    wa.LU = LU;
-    wa.hop_time = dT;
-    wa.hop_proc = dP;
-    wa.nc = pb.n_carriers;
-    wa.z = pb.z;
-    wa.mz = pb.max_z;
-    wa.field_on = d.field_on;
-    wa.uq = s->uniform_q ? 1 : 0;
-    wa.q0 = s->q0;
-    wa.nu = pb.nu;
-    wa.nkt = d.nkt;
-    wa.dt = pb.time_interval;
-    wa.P = pb.n_path;
-    wa.n_pairs = n_pairs;
-    wa.max_hops = max_hops;
-    PYCD_HIP(ctx, hipMemcpyAsync(s->dev.ptr, &d, sizeof(KmcDev),
-                                 hipMemcpyHostToDevice, st));
-    PYCD_HIP(ctx, launch_wave(s->compact, s->wave_npl, s->wave_smem, st, wa,
-                              s->dev.ptr, status_dev));
-  } else if (s->compact) {
-    kmc_plain_kernel<true><<<1, kThreads, s->smem, st>>>(
-        d, dU, LU, n_pairs, max_hops, dT, dP, status_dev);
-  } else {
-    kmc_plain_kernel<false><<<1, kThreads, s->smem, st>>>(
-        d, dU, LU, n_pairs, max_hops, dT, dP, status_dev);
-  }
+  PYCD_HIP(ctx, hipMemcpyAsync(s->dev.ptr, &d, sizeof(KmcDev),
+                               hipMemcpyHostToDevice, st));
+  PYCD_HIP(ctx, launch_hop(s, st, args, status_dev));
   PYCD_HIP(ctx, hipGetLastError());
   if (timed) PYCD_HIP(ctx, hipEventRecord(s->ev1, st));
   int32_t status[2] = {-1, 0};
