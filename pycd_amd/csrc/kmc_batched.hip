@@ -34,6 +34,21 @@
 // m's new slots are summed from scratch (n_c gathers each); every `refresh`
 // hops all of psi is recomputed from the table to bound the rounding.
 //
+// A lane holds its processes' targets, psi and table indexes and one
+// carrier's site row in registers, so that a hop goes through LDS only for
+// the psi of the processes' carrier sites and their rate inputs; the
+// selected process is read lane to lane.  The mover's new slots are summed
+// by rows of 16 lanes, a lane taking every 16th carrier, which leaves each
+// sum in the row that a lane permute hands to its process.  What bounds it:
+// alone on a SIMD, the latencies of a hop (LDS, scan, one round of gathers,
+// row sums); four to a SIMD, the issue of its ~380 vector instructions.
+// With sites, psi and process records in LDS instead (442 vector, 244
+// scalar, 44 LDS instructions, now 377, 108, 21) a hop took 2.26 us alone
+// and 3.09 among four at up to 16 carriers; now 1.18 and 2.01.  The loop is
+// instantiated per processes-per-lane count: with one instance for up to 4
+// the large trajectories' register spills made 4096 mixed trajectories 8%
+// slower.
+//
 // Random numbers: each trajectory carries its CPython MT19937 state (624
 // words + position) in LDS and draws 4 words per hop exactly like
 // random.random() (u1 selects, u2 advances the clock), so a batched
@@ -123,7 +138,8 @@ struct BatchArgs {
   const uint32_t* bin_start;
   const int16_t* key_bin;
   int32_t n_bins;
-  int32_t pad1;
+  // wavefronts on its SIMD from which one hands its trajectory over
+  int32_t hand_busy;
   // remaining hops of the wavefront in each SIMD wave slot (kSimdKeys x 16,
   // zeroed before the launch), for pacing, followed by the hand-over words
   // (see claim_mailbox); NULL: no pacing and no hand-over
@@ -249,23 +265,18 @@ __device__ inline double pair_entry(const Tab<TT>& t, const GeoPk& p,
   return double(t.at(t.row(a >> 24), rel_col(a, b, p)));
 }
 
-// psi[r] = sum_c q A[sites[r], occ[c]] for every slot r (lanes over slots).
+// sum_c q A[x, occ[c]].
 template <typename TT>
-__device__ inline void psi_from_table(const Tab<TT>& t, const GeoPk& gp,
-                                      double q, int R, int nc,
-                                      const uint32_t* sites,
-                                      const uint32_t* occ, double* psi,
-                                      int lane) {
-  for (int r = lane; r < R; r += 64) {
-    const uint32_t a = sites[r];
-    const RowKey key = row_key(a, gp);
-    const uint32_t row = t.row(key.sub);
-    double acc = 0.0;
+__device__ inline double psi_from_table(const Tab<TT>& t, const GeoPk& gp,
+                                        double q, int nc, uint32_t x,
+                                        const uint32_t* occ) {
+  const RowKey key = row_key(x, gp);
+  const uint32_t row = t.row(key.sub);
+  double acc = 0.0;
 #pragma unroll 4
-    for (int c2 = 0; c2 < nc; ++c2)
-      acc = fma(q, double(t.at(row, rel_col(key, occ[c2], gp))), acc);
-    psi[r] = acc;
-  }
+  for (int c2 = 0; c2 < nc; ++c2)
+    acc = fma(q, double(t.at(row, rel_col(key, occ[c2], gp))), acc);
+  return acc;
 }
 
 // Per (sublattice, slot) of the trajectory's family: the static part of a
@@ -273,7 +284,7 @@ __device__ inline void psi_from_table(const Tab<TT>& t, const GeoPk& gp,
 // the hop vector and target.  FP32 rates: 2 q (dphi + q tself) + dE, lambda,
 // 1 / (4 lambda), V_ab + field shift; FP64 rates: the six terms as the
 // reference adds them.
-struct PTabF32 {
+struct alignas(16) PTabF32 {
   double g0s;
   float lam, i4l, vs;
   uint32_t tgt;       // the hop record's packed target offset
@@ -287,23 +298,35 @@ struct PTabF64 {
 template <bool kF32Rate>
 using PTab = typename std::conditional<kF32Rate, PTabF32, PTabF64>::type;
 
-// Shared-memory layout of one wavefront (sizes from the batch's maxima:
-// pmax = nc_max z_max processes, rmax = nc_max (1 + z_max) slots):
+// The part of an entry that a rate takes.
+struct RateF32 {
+  double g0s;
+  float lam, i4l, vs;
+  __device__ RateF32() = default;
+  __device__ explicit RateF32(const PTabF32& p)
+      : g0s(p.g0s), lam(p.lam), i4l(p.i4l), vs(p.vs) {}
+};
+struct RateF64 {
+  double dphi, tq, dE, lam, vab, shift;
+  __device__ RateF64() = default;
+  __device__ explicit RateF64(const PTabF64& p)
+      : dphi(p.dphi), tq(p.tq), dE(p.dE), lam(p.lam), vab(p.vab),
+        shift(p.shift) {}
+};
+template <bool kF32Rate>
+using Rate = typename std::conditional<kF32Rate, RateF32, RateF64>::type;
+
+// Shared-memory layout of one wavefront:
 //   mt     624 words (2560 B)        MT19937 block
-//   psi    rmax doubles              potential of the carriers at each slot
+//   psis   64 doubles                potential at each carrier's site
+//   dsp    64 x 3 doubles            displacements since the last path row
+//   drf    64 x 3 doubles            drifts
+//   occ    64 words                  packed carrier sites (at the start and
+//                                    when psi is formed anew)
 //   ptab   sub_max PTab entries      per (sublattice, slot), see PTab
-//   sites  rmax words                packed slot sites (carrier, targets)
-//   occ    nc_max words              packed carrier sites
-//   cperm  nc_max words              slot permutation of each carrier's site
-//   pinfo  pmax words                per process: ptab index << 24 | slot
-//                                    permutation of its target site
-__host__ __device__ inline size_t batch_smem_bytes(int nc_max, int z_max,
-                                                  bool f32rate, int sub_max) {
-  const size_t rmax = size_t(nc_max) * (1 + z_max);
-  const size_t pmax = size_t(nc_max) * z_max;
+__host__ __device__ inline size_t batch_smem_bytes(bool f32rate, int sub_max) {
   const size_t pt = f32rate ? sizeof(PTabF32) : sizeof(PTabF64);
-  return 2560 + 8 * rmax + pt * size_t(sub_max) + 4 * rmax +
-         8 * size_t(nc_max) + 4 * pmax;
+  return 2560 + (7 * 8 + 4) * size_t(kMaxCarriers) + pt * size_t(sub_max);
 }
 
 template <bool kF32Rate>
@@ -360,7 +383,7 @@ __device__ inline uint32_t wave_slot() {
 // hops left highest, so that the SIMD's trajectories advance together and
 // end together; left alone, the SIMD favours its older wavefronts, whose
 // trajectories end first while the rest finish on a half-idle SIMD.
-__device__ inline void pace(uint32_t* prog, uint32_t slot, uint32_t left,
+__device__ inline int pace(uint32_t* prog, uint32_t slot, uint32_t left,
                             int lane) {
   if (lane == 0)
     __hip_atomic_store(prog + slot, left, __ATOMIC_RELAXED,
@@ -381,6 +404,7 @@ __device__ inline void pace(uint32_t* prog, uint32_t slot, uint32_t left,
     __builtin_amdgcn_s_setprio(1);
   else
     __builtin_amdgcn_s_setprio(0);
+  return __popcll(__ballot(v != 0u));
 }
 
 // Index into `order` of this wavefront's next trajectory, or n_traj once
@@ -408,13 +432,19 @@ __device__ inline uint32_t pop_ticket(const BatchArgs& a, int& bin) {
 }
 
 // Hand-over of running trajectories to idle wavefronts (batch launches with
-// SIMD bins: the words after the pacing slots).  SIMDs of the same chip run the same
-// work at speeds up to ~8% apart, so with every trajectory resident from
-// the start the launch would end with the slowest SIMDs.  Instead, a
-// wavefront that finds the queue empty opens a mailbox and waits; a
-// wavefront whose trajectory has hops to spare saves the trajectory's
+// SIMD bins: the words after the pacing slots).  Which trajectories fill
+// their path early is not known ahead, and SIMDs of the same chip run the
+// same work at speeds up to ~8% apart, so with every trajectory resident
+// from the start the launch would end with the fullest and slowest SIMDs.
+// Instead, a wavefront that finds the queue empty opens a mailbox and waits;
+// a wavefront whose trajectory has hops to spare saves the trajectory's
 // resumable state (exact, as at the end of a slice), puts its index in a
-// waiting mailbox and leaves.  Words of `hand`:
+// waiting mailbox and leaves.  A hop takes 1.2 us alone on a SIMD, 2.0 among
+// four (16 carriers), so with three or more wavefronts per SIMD a wavefront
+// waits beside up to one busy one and hands over only from three up; with
+// fewer the launch hands over from any busy SIMD to idle ones (4096 mixed
+// trajectories of 4000 hops, 1-64 carriers, whole run with its MSD: 22.3 ms
+// with idle SIMDs only and 2048 hops to spare, 20.8 so).  Words of `hand`:
 //   [0] trajectories not yet finished   [1] mailboxes taken by donors
 //   [2] mailboxes opened                [3] mailboxes (0: hand-over off)
 //   [kHandHdr + k] mailbox k: 0 empty, kMailClosed, or trajectory index + 1.
@@ -425,7 +455,7 @@ __device__ inline uint32_t pop_ticket(const BatchArgs& a, int& bin) {
 // grid + n_traj mailboxes are opened.
 constexpr int kHandHdr = 4;
 constexpr uint32_t kMailClosed = 0xffffffffu;
-constexpr uint32_t kHandMinHops = 2048;          // hops left to be worth it
+constexpr uint32_t kHandMinHops = 256;           // hops left to be worth it
 constexpr uint64_t kHandWaitTicks = 2000000000;  // 20 s at 100 MHz
 
 __device__ inline uint32_t* hand_words(uint32_t* progress) {
@@ -497,15 +527,33 @@ __global__ void __launch_bounds__(64) simd_probe(uint32_t* seen, int spin) {
   for (int i = 0; i < spin; ++i) __builtin_amdgcn_s_sleep(127);
 }
 
-// f(std::integral_constant<int, n>) for the run-time n in [1, kMax].
-template <int kMax, typename F>
-__device__ __forceinline__ void with_count(int n, F&& f) {
-  if constexpr (kMax >= 1) {
-    if (n == kMax)
-      f(std::integral_constant<int, kMax>{});
-    else
-      with_count<kMax - 1>(n, f);
+// f(std::integral_constant<int, kP>) for the smallest instance that holds
+// `per` processes per lane: 1 to 4 (kPer = 4), or 2, 4 or 8.
+template <int kPer, typename F>
+__device__ __forceinline__ void with_processes(int per, F&& f) {
+  if (kPer <= 4 && per == 1) {
+    if constexpr (kPer <= 4) f(std::integral_constant<int, 1>{});
+  } else if (per <= 2) {
+    f(std::integral_constant<int, 2>{});
+  } else if (kPer <= 4 && per == 3) {
+    if constexpr (kPer <= 4) f(std::integral_constant<int, 3>{});
+  } else if (per <= 4) {
+    f(std::integral_constant<int, 4>{});
+  } else if constexpr (kPer > 4) {
+    f(std::integral_constant<int, kPer>{});
   }
+}
+
+// *p += v in LDS.
+__device__ inline void lds_add(double* p, double v) {
+  (void)__hip_atomic_fetch_add(
+      (__attribute__((address_space(3))) double*)p, v, __ATOMIC_RELAXED,
+      __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// v of lane addr / 4 (mod 64).
+__device__ inline uint32_t lane_at(int addr, uint32_t v) {
+  return uint32_t(__builtin_amdgcn_ds_bpermute(addr, int(v)));
 }
 
 // Wavefronts per SIMD the register allocation targets: 4 (16 per CU, every
@@ -520,14 +568,13 @@ template <typename TT, bool kF32Rate, int kPer, int kZp>
 __device__ __forceinline__ void kmc_batched_body(const BatchArgs& a) {
   extern __shared__ unsigned char smem_raw[];
   const int lane = threadIdx.x;
-  const int rmax = a.nc_max * (1 + a.z_max);
   uint32_t* mt = reinterpret_cast<uint32_t*>(smem_raw);
-  double* psi = reinterpret_cast<double*>(smem_raw + 2560);
-  PTab<kF32Rate>* ptab = reinterpret_cast<PTab<kF32Rate>*>(psi + rmax);
-  uint32_t* sites = reinterpret_cast<uint32_t*>(ptab + a.sub_max);
-  uint32_t* occ = sites + rmax;
-  uint32_t* cperm = occ + a.nc_max;
-  uint32_t* pinfo = cperm + a.nc_max;
+  double* psis = reinterpret_cast<double*>(smem_raw + 2560);
+  double* dsp = psis + kMaxCarriers;
+  double* drf = dsp + 3 * kMaxCarriers;
+  uint32_t* occ = reinterpret_cast<uint32_t*>(drf + 3 * kMaxCarriers);
+  PTab<kF32Rate>* ptab =
+      reinterpret_cast<PTab<kF32Rate>*>(occ + kMaxCarriers);
 
   const uint32_t pslot = a.progress ? wave_slot() : 0u;
   int bin = 0;
@@ -552,14 +599,14 @@ __device__ __forceinline__ void kmc_batched_body(const BatchArgs& a) {
       tr = uni(a.order[ti]);
     } else {
       if (!a.progress) break;
-      // wait for a hand-over only on a SIMD that has run out of work, so
-      // that a trajectory moves from a busy SIMD to an idle one
+      // wait for a hand-over only on a SIMD that has nearly run out of work,
+      // so that a trajectory moves from a busy SIMD to an idle one
       uint32_t busy_here = 0;
       if (lane < 16)
         busy_here = __hip_atomic_load(a.progress + (pslot & ~15u) + lane,
                                       __ATOMIC_RELAXED,
                                       __HIP_MEMORY_SCOPE_AGENT);
-      if (__ballot(busy_here != 0u)) break;
+      if (__popcll(__ballot(busy_here != 0u)) > max(a.hand_busy - 2, 0)) break;
       int got = -1;
       if (lane == 0) got = wait_for_trajectory(hand_words(a.progress));
       got = uni(__shfl(got, 0, 64));
@@ -591,32 +638,16 @@ __device__ __forceinline__ void kmc_batched_body(const BatchArgs& a) {
     dtab.row_bytes = uint32_t(f.N) * uint32_t(sizeof(double));
     const bool use_d = f.D != nullptr;
     const int nc = uni(td.nc), z = uni(f.z), zp = z + 1;
-    const int R = nc * zp, nproc = nc * z;
+    const int nproc = nc * z;
     const int per = (nproc + 63) / 64;
-    // this lane's processes p = lane per + i, fixed for the trajectory:
-    // c | j << 6 | (slot of c's site) << 9 | (slot of the target) << 19,
-    // bit 31 set for a real process
-    uint32_t pdesc[kPer];
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int p = lane * per + i;
-      pdesc[i] = 0;
-      if (i < per && p < nproc) {
-        const int c = p / z, j = p - c * z;
-        pdesc[i] = uint32_t(c) | (uint32_t(j) << 6) |
-                   (uint32_t(c * zp) << 9) | (uint32_t(c * zp + 1 + j) << 19) |
-                   0x80000000u;
-      }
-    }
     const double q = td.q;
     double* rows = a.rows + td.row_off;
     const int w = 3 * nc;
     const bool field_on =
         td.field[0] != 0.0 || td.field[1] != 0.0 || td.field[2] != 0.0;
 
-    // resumable per-trajectory state in global memory (the displacement
-    // and drift there are written with the state and read on resumption;
-    // while the trajectory runs they are held in the carriers' lanes)
+    // resumable per-trajectory state in global memory (what changes from
+    // hop to hop is held in registers while the trajectory runs)
     uint32_t* mts = a.mts + int64_t(tr) * 625;
     uint32_t* socc = a.st_occ + int64_t(tr) * kMaxCarriers;
     double* svec = a.st_vec + int64_t(tr) * kVecStride;
@@ -629,13 +660,7 @@ __device__ __forceinline__ void kmc_batched_body(const BatchArgs& a) {
     // ---- load or start the state
     const uint32_t* m0 = resume ? mts : a.mt0 + int64_t(tr) * 625;
     for (int k = lane; k < 624; k += 64) mt[k] = m0[k];
-    int mti = int(m0[624]);
-    for (int c = lane; c < nc; c += 64) {
-      const uint32_t s =
-          resume ? socc[c] : site_pack(uint32_t(a.occ0[td.occ_off + c]), g);
-      occ[c] = s;
-      cperm[c] = as_global(f.perm)[site_index(s, g)];
-    }
+    int mti = uni(int(m0[624]));
     for (int k = lane; k < f.nu * z; k += 64) {
       fill_ptab<kF32Rate>(ptab[k], load_rec(f, k), q, td.field, field_on);
     }
@@ -644,30 +669,20 @@ __device__ __forceinline__ void kmc_batched_body(const BatchArgs& a) {
         sbase[k] = 0.0;
         rows[k] = 0.0;  // path row 0: the initial positions
       }
-    // displacement since the last path row and drift of carrier `lane`, in
-    // its lane while the trajectory runs (saved with the state)
-    double dsp[3] = {0.0, 0.0, 0.0}, drf[3] = {0.0, 0.0, 0.0};
-    if (resume && lane < nc)
+    // displacements since the last path row and drifts, zero past n_c
 #pragma unroll
-      for (int c3 = 0; c3 < 3; ++c3) {
-        dsp[c3] = sdisp[3 * lane + c3];
-        drf[c3] = sdrift[3 * lane + c3];
-      }
-    __syncthreads();
-    for (int r = lane; r < R; r += 64) {
-      const int c = r / zp, k = r - c * zp;
-      const uint32_t s = occ[c];
-      const uint32_t jj = (cperm[c] >> (3 * (k - 1))) & 7u;
-      sites[r] = k == 0 ? s : site_add(s, ptab[(s >> 24) * z + jj].tgt, g);
+    for (int c3 = 0; c3 < 3; ++c3) {
+      const int k = lane + 64 * c3;
+      dsp[k] = resume && k < w ? sdisp[k] : 0.0;
+      drf[k] = resume && k < w ? sdrift[k] : 0.0;
     }
-    // each process's table entry and the slot permutation of its target
-    for (int p = lane; p < nproc; p += 64) {
-      const int c = p / z, j = p - c * z;
-      const uint32_t s = occ[c];
-      const uint32_t k = (s >> 24) * z + ((cperm[c] >> (3 * j)) & 7u);
-      pinfo[p] = (k << 24) |
-                 as_global(f.perm)[site_index(site_add(s, ptab[k].tgt, g), g)];
-    }
+    // the site of carrier `lane`, in its lane while the trajectory runs (site
+    // 0 past n_c)
+    uint32_t sx = 0;
+    if (lane < nc)
+      sx = resume ? socc[lane]
+                  : site_pack(uint32_t(a.occ0[td.occ_off + lane]), g);
+    occ[lane] = sx;
     __syncthreads();
     double t_clk, energy;
     // path rows are int32 (the host keeps n_path below 2^31)
@@ -676,22 +691,20 @@ __device__ __forceinline__ void kmc_batched_body(const BatchArgs& a) {
     int64_t hops;
     int no_select;
     if (resume) {
-      for (int r = lane; r < R; r += 64) psi[r] = spsi[r];
       t_clk = o0.t;
       energy = o0.energy;
-      start = int32_t(o0.start);
-      hops = o0.hops;
-      no_select = o0.no_select;
+      start = uni(int32_t(o0.start));
+      hops = int64_t(uni(uint32_t(o0.hops))) |
+             (int64_t(uni(uint32_t(o0.hops >> 32))) << 32);
+      no_select = uni(o0.no_select);
     } else {
-      psi_from_table<TT>(tab, gp, q, R, nc, sites, occ, psi, lane);
       // initial energy: ewald_neut + q_L A q_L + sum_c q (2 phi_L + psi_self)
       double e_loc = 0.0;
-      for (int c = lane; c < nc; c += 64) {
-        const uint32_t s = occ[c];
+      if (lane < nc) {
         double inner = 0.0;
         for (int c2 = 0; c2 < nc; ++c2)
-          inner = fma(q, pair_entry<TT>(tab, gp, s, occ[c2]), inner);
-        e_loc += q * (2.0 * as_global(f.phiL)[s >> 24] + inner);
+          inner = fma(q, pair_entry<TT>(tab, gp, sx, occ[c2]), inner);
+        e_loc += q * (2.0 * as_global(f.phiL)[sx >> 24] + inner);
       }
       energy = td.ewald_neut + (f.qLAqL + wave_sum(e_loc));
       t_clk = 0.0;
@@ -699,7 +712,6 @@ __device__ __forceinline__ void kmc_batched_body(const BatchArgs& a) {
       hops = 0;
       no_select = 0;
     }
-    __syncthreads();
     int64_t slice_done = 0;
     bool finished = false;
     // next hop count that is a positive multiple of `refresh`
@@ -709,9 +721,11 @@ __device__ __forceinline__ void kmc_batched_body(const BatchArgs& a) {
           hops == 0 ? a.refresh : (hops + a.refresh - 1) / a.refresh * a.refresh;
     // FP32 rates: nu exp(-gs / kT) = 2^(gs (-log2(e) / kT) + log2(nu)),
     // one FMA ahead of v_exp_f32
-    const float exp_scale = float(-kLog2E / td.kT);
-    const float exp_bias = float(log2(a.nu));
-    const double inv_dt = 1.0 / td.dt;
+    const float exp_scale = __uint_as_float(
+        uni(__float_as_uint(float(-kLog2E / td.kT))));
+    const float exp_bias =
+        __uint_as_float(uni(__float_as_uint(float(log2(a.nu)))));
+    const double inv_dt = uni(1.0 / td.dt);
 
     // Uniforms of the coming hops, one hop per lane: at a refill (mti = m)
     // lane l takes u1 and log(u2) (-inf for u2 = 0) of the hop that draws
@@ -723,378 +737,412 @@ __device__ __forceinline__ void kmc_batched_body(const BatchArgs& a) {
     // instead of every lane taking one per hop.
     double c_u1 = 0.0, c_lu2 = 0.0;
     int c_next = 0, c_n = 0;
-    // outputs and resumable state: at the trajectory's end, or at a hop
-    // boundary when it is handed over
-    auto save = [&](bool done_now) {
-      // every carrier slot of the output, zero past the trajectory's own
-      static_assert(kMaxCarriers == 64, "one carrier per lane");
-#pragma unroll
-      for (int c3 = 0; c3 < 3; ++c3) {
-        a.drift[int64_t(tr) * 3 * kMaxCarriers + 3 * lane + c3] =
-            lane < nc ? drf[c3] : 0.0;
-        if (lane < nc) {
-          sdisp[3 * lane + c3] = dsp[c3];
-          sdrift[3 * lane + c3] = drf[c3];
-        }
-      }
-      for (int k = lane; k < 624; k += 64) mts[k] = mt[k];
-      for (int c = lane; c < nc; c += 64) socc[c] = occ[c];
-      for (int r = lane; r < R; r += 64) spsi[r] = psi[r];
-      if (lane == 0) {
-        mts[624] = uint32_t(mti);
-        TrajOut o;
-        o.t = t_clk;
-        o.energy = energy;
-        o.hops = hops;
-        o.start = start;
-        o.no_select = no_select;
-        o.done = done_now ? 1 : 0;
-        o.started = 1;
-        o.simd = int32_t(simd_key());
-        o.busy = (resume ? o0.busy : 0.0) + double(wall_clock64() - w_start);
-        a.out[tr] = o;
-      }
-      __syncthreads();
-    };
     int box = -1;  // mailbox of the wavefront taking the trajectory over
     // Hops this launch may still make: to max_hops (which finishes the
     // trajectory) and to the end of the slice (which pauses it).  The hop
     // loop counts them down in 32 bits and asks again when they run out, so
     // a budget above 2^31 - 1 is taken in parts.
-    auto budget = [&]() {
+    auto budget = [&]() __attribute__((always_inline)) {
       int64_t h = INT64_MAX;
       if (td.max_hops > 0) h = td.max_hops - hops;
       if (a.slice_hops > 0) h = min(h, a.slice_hops - slice_done);
       return h;
     };
     uint32_t left = 0;
-    for (;;) {
-      // Conditions on the lane and on the trajectory's sizes are formed
-      // again each hop from these copies, which the compiler cannot move
-      // out of the loop.  Hoisted, each such condition is a 64-bit lane mask
-      // held across the loop, and there are more of them than registers.
-      int lane_h = lane, per_h = per, z_h = z, nc_h = nc, R_h = R;
-      asm volatile("" : "+v"(lane_h));
-      asm volatile("" : "+s"(per_h), "+s"(z_h), "+s"(nc_h), "+s"(R_h));
-      uint32_t pd[kPer];
+    // The hops of this launch, kP processes per lane (per <= kP), and the
+    // state written back: outputs and resumable state, at the trajectory's
+    // end, at the slice's, or at a hop boundary when it is handed over.
+    with_processes<kPer>(per, [&](auto n_per) __attribute__((always_inline)) {
+      constexpr int kP = decltype(n_per)::value;
+      // Process p = lane per + i (the rest: carrier -1, rate 0): its
+      // carrier << 9 | its slot << 6, its target, the target's table index
+      // << 24 | slot permutation, and psi of the target
+      int pd[kP];
+      uint32_t px[kP], pinfo[kP];
+      double psi[kP];
 #pragma unroll
-      for (int i = 0; i < kPer; ++i) {
-        pd[i] = pdesc[i];
-        asm volatile("" : "+v"(pd[i]));
+      for (int i = 0; i < kP; ++i) {
+        const int p = lane * per + i;
+        const bool real = i < per && p < nproc;
+        const int c = real ? p / z : 0, j = real ? p - c * z : 0;
+        pd[i] = (real ? c << 9 : -512) | (j << 6);
+        const uint32_t s = occ[c];
+        const uint32_t k = (s >> 24) * z +
+                           ((as_global(f.perm)[site_index(s, g)] >> (3 * j)) & 7u);
+        px[i] = site_add(s, ptab[k].tgt, g);
+        pinfo[i] = (k << 24) | as_global(f.perm)[site_index(px[i], g)];
+        if (resume) psi[i] = spsi[c * zp + 1 + j];
       }
-      if (left == 0) {
-        asm volatile("");  // the 64-bit budget only when the count runs out
-        const int64_t b = budget();
-        if (b <= 0) {
-          finished = td.max_hops > 0 && hops >= td.max_hops;
-          break;
+      // psi at the site of carrier `lane`
+      double psi_s = resume && lane < nc ? spsi[lane * zp] : 0.0;
+      auto psi_anew = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kP; ++i)
+          psi[i] = psi_from_table<TT>(tab, gp, q, nc, px[i], occ);
+        psi_s = psi_from_table<TT>(tab, gp, q, nc, sx, occ);
+      };
+      if (!resume) psi_anew();
+      // lane fc + 16 r forms row r of the fresh sums with the carriers
+      // fc + 16 u
+      const int fc = lane & 15;
+      uint32_t fo[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) fo[u] = occ[fc + 16 * u];
+      for (;;) {
+        // Conditions on the lane and on the trajectory's sizes are formed
+        // again each hop from these copies, which the compiler cannot move
+        // out of the loop.  Hoisted, each such condition is a 64-bit lane
+        // mask held across the loop, and there are more of them than
+        // registers.
+        int lane_h = lane, z_h = z, nc_h = nc;
+        asm volatile("" : "+v"(lane_h));
+        asm volatile("" : "+s"(z_h), "+s"(nc_h));
+        const int fc_h = lane_h & 15;
+#pragma unroll
+        for (int i = 0; i < kP; ++i) asm volatile("" : "+v"(pd[i]));
+        if (left == 0) {
+          asm volatile("");  // the 64-bit budget only when the count runs out
+          const int64_t b = budget();
+          if (b <= 0) {
+            finished = td.max_hops > 0 && hops >= td.max_hops;
+            break;
+          }
+          left = uint32_t(min<int64_t>(b, INT32_MAX));
         }
-        left = uint32_t(min<int64_t>(b, INT32_MAX));
-      }
-      --left;
-      ++slice_done;
-      if (a.progress && (uint32_t(hops) & 63u) == 0) {
-        pace(a.progress, pslot, left + 1, lane_h);
-        if (!stolen && left >= kHandMinHops) {
-          if (lane_h == 0) box = claim_mailbox(hand_words(a.progress));
-          box = uni(__shfl(box, 0, 64));
-          if (box >= 0) break;  // hand over at this hop boundary
+        --left;
+        ++slice_done;
+        if (a.progress && (uint32_t(hops) & 63u) == 0) {
+          const int busy = pace(a.progress, pslot, left + 1, lane_h);
+          if (!stolen && busy >= a.hand_busy && left >= kHandMinHops) {
+            if (lane_h == 0) box = claim_mailbox(hand_words(a.progress));
+            box = uni(__shfl(box, 0, 64));
+            if (box >= 0) break;  // hand over at this hop boundary
+          }
         }
-      }
-      if (hops == next_refresh) {
-        next_refresh += a.refresh;
-        // bound the rounding carried by the incremental updates
-        psi_from_table<TT>(tab, gp, q, R_h, nc_h, sites, occ, psi, lane_h);
+        if (hops == next_refresh) {
+          next_refresh += a.refresh;
+          // bound the rounding carried by the incremental updates
+          occ[lane_h] = sx;
+          __syncthreads();
+          psi_anew();
+        }
+        psis[lane_h] = psi_s;
+        // ---- two uniforms, as random.random() draws them
+        if (c_next >= c_n && mti <= kMtN - 4) {
+          c_n = min(64, (kMtN - mti) / 4);
+          c_next = 0;
+          if (lane_h < c_n) {
+            const int w = mti + 4 * lane_h;
+            c_u1 = mt_uniform(mt_temper(mt[w]), mt_temper(mt[w + 1]));
+            const double u2 =
+                mt_uniform(mt_temper(mt[w + 2]), mt_temper(mt[w + 3]));
+            c_lu2 = u2 > 0.0 ? log(u2) : -INFINITY;
+          }
+        }
+        double u1, lu2;
+        if (c_next < c_n) {
+          u1 = read_lane(c_u1, c_next);
+          lu2 = read_lane(c_lu2, c_next);
+          ++c_next;
+          mti += 4;
+        } else {
+          uint32_t wd[4];
+          mt_next4(mt, mti, lane_h, wd);
+          u1 = uni(mt_uniform(wd[0], wd[1]));
+          const double u2 = mt_uniform(wd[2], wd[3]);
+          lu2 = uni(u2 > 0.0 ? log(u2) : -INFINITY);
+        }
         __syncthreads();
-      }
-      // ---- two uniforms, as random.random() draws them
-      if (c_next >= c_n && mti <= kMtN - 4) {
-        c_n = min(64, (kMtN - mti) / 4);
-        c_next = 0;
-        if (lane_h < c_n) {
-          const int w = mti + 4 * lane_h;
-          c_u1 = mt_uniform(mt_temper(mt[w]), mt_temper(mt[w + 1]));
-          const double u2 = mt_uniform(mt_temper(mt[w + 2]), mt_temper(mt[w + 3]));
-          c_lu2 = u2 > 0.0 ? log(u2) : -INFINITY;
-        }
-      }
-      double u1, lu2;
-      if (c_next < c_n) {
-        u1 = read_lane(c_u1, c_next);
-        lu2 = read_lane(c_lu2, c_next);
-        ++c_next;
-        mti += 4;
-      } else {
-        uint32_t wd[4];
-        mt_next4(mt, mti, lane_h, wd);
-        u1 = mt_uniform(wd[0], wd[1]);
-        const double u2 = mt_uniform(wd[2], wd[3]);
-        lu2 = u2 > 0.0 ? log(u2) : -INFINITY;
-      }
-      // ---- rates from shared memory only
-      double kv[kPer], gv[kPer];
-      double ksum = 0.0;
+        // ---- rates: psi of the carriers' sites and the rate inputs of all
+        // processes are read before the first is used
+        double kv[kP], gv[kP], ps[kP];
+        Rate<kF32Rate> e[kP];
+        double ksum = 0.0;
 #pragma unroll
-      for (int i = 0; i < kPer; ++i) {
-        kv[i] = 0.0;
-        gv[i] = 0.0;
-      }
-      // one straight-line body per processes-per-lane count, so that the
-      // processes' LDS reads are in flight together
-      with_count<kPer>(per_h, [&](auto n_per) {
-        constexpr int kP = decltype(n_per)::value;
+        for (int i = 0; i < kP; ++i) ps[i] = psis[max(pd[i], 0) >> 9];
+#pragma unroll
+        for (int i = 0; i < kP; ++i) e[i] = Rate<kF32Rate>(ptab[pinfo[i] >> 24]);
 #pragma unroll
         for (int i = 0; i < kP; ++i) {
-          const uint32_t d = pd[i];
-          const bool real = d >> 31;
-          const int p = real ? lane_h * kP + i : 0;
-          const PTab<kF32Rate>& e = ptab[pinfo[p] >> 24];
-          const double dpsi =
-              psi[(d >> 19) & 0x3ffu] - psi[(d >> 9) & 0x3ffu];
+          const bool real = pd[i] >= 0;
+          const double dpsi = psi[i] - ps[i];
           double g0;
           if constexpr (kF32Rate) {
-            g0 = e.g0s + 2 * q * dpsi;
+            g0 = e[i].g0s + 2 * q * dpsi;
             const float gf = float(g0);
-            const float gs = (e.lam + gf) * (e.lam + gf) * e.i4l - e.vs;
+            const float gs =
+                (e[i].lam + gf) * (e[i].lam + gf) * e[i].i4l - e[i].vs;
             const float kf =
                 __builtin_amdgcn_exp2f(fmaf(gs, exp_scale, exp_bias));
             kv[i] = double(real ? kf : 0.0f);
           } else {
-            g0 = 2 * q * ((e.dphi + dpsi) + e.tq) + e.dE;
-            const double lam = e.lam;
+            g0 = 2 * q * ((e[i].dphi + dpsi) + e[i].tq) + e[i].dE;
+            const double lam = e[i].lam;
             const double gs =
-                (((lam + g0) * (lam + g0) / (4 * lam)) - e.vab) - e.shift;
+                (((lam + g0) * (lam + g0) / (4 * lam)) - e[i].vab) - e[i].shift;
             const double k = a.nu * numpy_e_pow(-gs / td.kT);
             kv[i] = real ? k : 0.0;
           }
           gv[i] = g0;
           ksum = i == 0 ? kv[0] : ksum + kv[i];
         }
-      });
-      // ---- FP64 prefix and selection.  FP64 rates: the prefix of the
-      // quotients k / k_tot against u1, as the reference forms it; FP32
-      // rates: one scan of the rates themselves against u1 k_tot.
-      double k_tot, thr, cum;
-      double xq[kPer];
-      if (kF32Rate) {
-        const double incl = wave_incl_scan(ksum);
-        k_tot = read_lane(incl, 63);
-        cum = dpp_f64<kDppWaveShr1, 0xf, true>(incl);
-        thr = u1 * k_tot;
+        // ---- FP64 prefix and selection.  FP64 rates: the prefix of the
+        // quotients k / k_tot against u1, as the reference forms it; FP32
+        // rates: one scan of the rates themselves against u1 k_tot.
+        double k_tot, thr, cum;
+        double xq[kP];
+        if (kF32Rate) {
+          const double incl = wave_incl_scan(ksum);
+          k_tot = read_lane(incl, 63);
+          cum = dpp_f64<kDppWaveShr1, 0xf, true>(incl);
+          thr = u1 * k_tot;
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) xq[i] = kv[i];
-      } else {
-        k_tot = wave_sum(ksum);
-        double xs = 0.0;
+          for (int i = 0; i < kP; ++i) xq[i] = kv[i];
+        } else {
+          k_tot = wave_sum(ksum);
+          double xs = 0.0;
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-          xq[i] = kv[i] / k_tot;
-          xs += xq[i];
+          for (int i = 0; i < kP; ++i) {
+            xq[i] = kv[i] / k_tot;
+            xs += xq[i];
+          }
+          cum = wave_excl_scan(xs);
+          thr = u1;
         }
-        cum = wave_excl_scan(xs);
-        thr = u1;
-      }
-      // The selected process is the first (lane, i), lane-major, whose
-      // running sum cum + xq[0] + ... + xq[i] exceeds thr.  The terms are
-      // non-negative, so each lane's running sums do not decrease: the
-      // count of them that stay <= thr is the index of the lane's first
-      // crossing (a lane crosses iff the count is below per, and its first
-      // process is real: processes past nproc add zero at the lane's end).
-      int nb = 0;
+        // The selected process is the first (lane, i), lane-major, whose
+        // running sum cum + xq[0] + ... + xq[i] exceeds thr.  The terms are
+        // non-negative, so each lane's running sums do not decrease: the
+        // count of them that stay <= thr is the index of the lane's first
+        // crossing (a lane crosses iff the count is below per, and its first
+        // process is real: processes past nproc add zero at the lane's end).
+        int nb = 0;
 #pragma unroll
-      for (int i = 0; i < kPer; ++i) {
-        if (i < per_h) {
+        for (int i = 0; i < kP; ++i) {
           cum += xq[i];
           nb += cum > thr ? 0 : 1;
         }
-      }
-      const unsigned long long mask =
-          __ballot((pd[0] >> 31) != 0u && nb < per_h);
-      int src, isel;
-      if (mask) {
-        src = uni(__ffsll(static_cast<long long>(mask)) - 1);
-        isel = __builtin_amdgcn_readlane(nb, src);
-      } else {
-        // rounding left every running sum <= thr: take the last process
-        src = (nproc - 1) / per_h;
-        isel = nproc - 1 - src * per_h;
-        ++no_select;
-      }
-      const int sel = src * per_h + isel;
-      uint32_t dsel = 0;
-      double gsel = 0.0, ksel = 0.0;
-#pragma unroll
-      for (int i = 0; i < kPer; ++i)
-        if (i == isel) {
-          dsel = uint32_t(__builtin_amdgcn_readlane(int(pd[i]), src));
-          gsel = read_lane(gv[i], src);
-          ksel = read_lane(kv[i], src);
-        }
-      // ---- clock
-      int32_t end;
-      if (lu2 > -INFINITY) {  // u2 > 0
-        t_clk -= lu2 / k_tot;
-        // path step int(t / dt) of the correctly rounded quotient: below
-        // 1e6, t (1/dt) is within 4e-10 of it, so more than 1e-9 away from
-        // an integer its integer part is the quotient's; otherwise divide
-        const double qf = t_clk * inv_dt;
-        const double fr = qf - floor(qf);
-        if (fr > 1e-9 && fr < 1.0 - 1e-9 && qf < 1.0e6) {
-          end = int32_t(qf);
+        const unsigned long long mask =
+            __ballot(int(pd[0] >= 0) & int(nb < per));
+        int src, isel = 0;
+        if (mask) {
+          src = uni(__ffsll(static_cast<long long>(mask)) - 1);
+          if constexpr (kP > 1) isel = __builtin_amdgcn_readlane(nb, src);
         } else {
-          asm volatile("");  // the division only where it is needed
-          const double qq = t_clk / td.dt;
-          end = qq < double(P) ? int32_t(qq) : P;
+          // rounding left every running sum <= thr: take the last process
+          src = (nproc - 1) / per;
+          isel = nproc - 1 - src * per;
+          ++no_select;
         }
-      } else {
-        t_clk = INFINITY;
-        end = P;
-      }
-      energy += gsel;
-      // ---- one round of independent loads for the whole update
-      const int m = int(dsel & 63u);
-      const int j = int((dsel >> 6) & 7u);
-      const uint32_t s_old = uni(sites[m * zp]);
-      const uint32_t s_new = uni(sites[m * zp + 1 + j]);
-      const uint32_t sub_new = s_new >> 24;
-      const uint32_t info_sel = uni(pinfo[sel]);
-      const uint32_t perm_new = info_sel & 0xffffffu;
-      const uint32_t rec_old = info_sel >> 24;
-      // table entries of the new site's processes and the slot
-      // permutations of their targets (lanes < z), issued first
-      uint32_t info_new = 0, nsite = 0;
-      if (lane_h < z_h) {
-        const uint32_t k = sub_new * z_h + ((perm_new >> (3 * lane_h)) & 7u);
-        nsite = site_add(s_new, ptab[k].tgt, g);
-        info_new = (k << 24) | as_global(f.perm)[site_index(nsite, g)];
-      }
-      uint32_t nsel[kZp - 1];  // targets of the new site, in its slot order
+        int m = 0;
+        uint32_t s_new = 0, info_sel = 0;
+        double gsel = 0.0, ksel = 0.0;
 #pragma unroll
-      for (int k = 0; k < kZp - 1; ++k)
-        nsel[k] = k < z_h ? uint32_t(__builtin_amdgcn_readlane(int(nsite), k))
-                          : 0u;
-      const uint32_t rn = tab.row(sub_new), ro = tab.row(s_old >> 24);
-      const RowKey key_new = row_key(s_new, gp), key_old = row_key(s_old, gp);
-      const uint32_t rd = dtab.row(rec_old);
-      constexpr int kRPer = kMaxCarriers * kZp / 64;
-      // Every slot's change q (A[n, x] - A[s, x]) is loaded before any is
-      // used, so that the slots' gathers are in flight together: one entry
-      // of the family's hop differences (row rec_old, x's column in s_old's
-      // row) where it has them, else both table entries (an - double(ao),
-      // ao = 0 with differences)
-      double an[kRPer];
-      TT ao[kRPer];
-      // the slot sites of this lane's rows, read together (one LDS wait,
-      // not one per row)
-      uint32_t xs[kRPer];
+        for (int i = 0; i < kP; ++i)
+          if (kP == 1 || i == isel) {
+            m = __builtin_amdgcn_readlane(pd[i], src) >> 9;
+            s_new = uint32_t(__builtin_amdgcn_readlane(int(px[i]), src));
+            info_sel = uint32_t(__builtin_amdgcn_readlane(int(pinfo[i]), src));
+            gsel = read_lane(gv[i], src);
+            ksel = read_lane(kv[i], src);
+          }
+        // ---- one round of independent loads for the whole update
+        const uint32_t s_old = uint32_t(__builtin_amdgcn_readlane(int(sx), m));
+        const uint32_t sub_new = s_new >> 24;
+        const uint32_t perm_new = info_sel & 0xffffffu;
+        const uint32_t rec_old = info_sel >> 24;
+        // Slot k of the new site in the 16 lanes of row k mod 4: its target,
+        // the target's table index and slot permutation, and the entries of
+        // every carrier there (in FP32 or FP64, used after the update: the
+        // loads overlap)
+        constexpr int kT = kZp > 5 ? 2 : 1;  // rounds of 4 slots
+        uint32_t nsite[kT], ninfo[kT];
+        TT fent[kT][4];
 #pragma unroll
-      for (int i = 0; i < kRPer; ++i) {
-        const int r = lane_h + 64 * i;
-        xs[i] = sites[r < R_h ? r : 0];
-      }
+        for (int u = 0; u < 4; ++u) fo[u] = fc_h + 16 * u == m ? s_new : fo[u];
 #pragma unroll
-      for (int i = 0; i < kRPer; ++i) {
-        const int r = lane_h + 64 * i;
-        // set and read only for r < R (no zero fill of unused rows)
-        if (r < R_h) {
-          if (use_d) {
-            an[i] = dtab.at(rd, rel_col(key_old, xs[i], gp));
-            ao[i] = TT(0);
+        for (int t = 0; t < kT; ++t) {
+          const int k4 = (lane_h >> 4) + 4 * t, k = k4 < z_h ? k4 : 0;
+          const uint32_t rec = sub_new * z_h + ((perm_new >> (3 * k)) & 7u);
+          nsite[t] = site_add(s_new, ptab[rec].tgt, g);
+          ninfo[t] =
+              (rec << 24) | as_global(f.perm)[site_index(nsite[t], g)];
+          const uint32_t row = tab.row(nsite[t] >> 24);
+          const RowKey key = row_key(nsite[t], gp);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            fent[t][u] = TT(0);
+            if (16 * u < nc_h) fent[t][u] = tab.at(row, rel_col(key, fo[u], gp));
+          }
+        }
+        // Every row's change q (A[n, x] - A[s, x]) is loaded before any is
+        // used: one entry of the family's hop differences (row rec_old, x's
+        // column in s_old's row) where it has them, else both table entries
+        const uint32_t rn = tab.row(sub_new), ro = tab.row(s_old >> 24);
+        const RowKey key_new = row_key(s_new, gp), key_old = row_key(s_old, gp);
+        const uint32_t rd = dtab.row(rec_old);
+        double dx[kP], ds;
+        if (use_d) {
+#pragma unroll
+          for (int i = 0; i < kP; ++i)
+            dx[i] = dtab.at(rd, rel_col(key_old, px[i], gp));
+          ds = dtab.at(rd, rel_col(key_old, sx, gp));
+        } else {
+          TT an[kP], ao[kP];
+#pragma unroll
+          for (int i = 0; i < kP; ++i) {
+            an[i] = tab.at(rn, rel_col(key_new, px[i], gp));
+            ao[i] = tab.at(ro, rel_col(key_old, px[i], gp));
+          }
+          const TT sn = tab.at(rn, rel_col(key_new, sx, gp));
+          const TT so = tab.at(ro, rel_col(key_old, sx, gp));
+#pragma unroll
+          for (int i = 0; i < kP; ++i) dx[i] = double(an[i]) - double(ao[i]);
+          ds = double(sn) - double(so);
+        }
+        // ---- clock, while the loads are in flight
+        int32_t end;
+        if (lu2 > -INFINITY) {  // u2 > 0
+          t_clk -= lu2 / k_tot;
+          // path step int(t / dt) of the correctly rounded quotient: below
+          // 1e6, t (1/dt) is within 4e-10 of it, so more than 1e-9 away from
+          // an integer its integer part is the quotient's; otherwise divide
+          const double qf = t_clk * inv_dt;
+          const double fr = qf - floor(qf);
+          if (fr > 1e-9 && fr < 1.0 - 1e-9 && qf < 1.0e6) {
+            end = int32_t(qf);
           } else {
-            an[i] = double(tab.at(rn, rel_col(key_new, xs[i], gp)));
-            ao[i] = tab.at(ro, rel_col(key_old, xs[i], gp));
+            asm volatile("");  // the division only where it is needed
+            const double qq = t_clk / td.dt;
+            end = qq < double(P) ? int32_t(qq) : P;
           }
+        } else {
+          t_clk = INFINITY;
+          end = P;
         }
-      }
-      // fresh sums of the new slots (not the one that returns to s_old):
-      // one carrier per lane (n_c <= 64)
-      // (entries loaded here, used after the apply: the loads overlap)
-      constexpr int kFresh = (kZp - 1 + 3) / 4 * 4;
-      TT fent[kFresh];
-      {
-        const bool has = lane_h < nc_h;
-        const uint32_t o = has ? (lane_h == m ? s_new : occ[lane_h]) : 0u;
-#pragma unroll
-        for (int k = 0; k < kFresh; ++k) {
-          fent[k] = TT(0);
-          if (k < kZp - 1 && k < z_h && has && nsel[k] != s_old)
-            fent[k] = tab.at(tab.row(nsel[k] >> 24), rel_col(nsel[k], o, gp));
-        }
-      }
-      // hop vector of carrier m (the same address in every lane)
-      double hv[3];
-#pragma unroll
-      for (int c3 = 0; c3 < 3; ++c3) hv[c3] = ptab[rec_old].vec[c3];
-      // ---- apply (process m's old entries are dead once it is selected)
-      if (lane_h < z_h) pinfo[m * z_h + lane_h] = info_new;
-#pragma unroll
-      for (int i = 0; i < kRPer; ++i) {
-        const int r = lane_h + 64 * i;
-        if (r < R_h) psi[r] += q * (an[i] - double(ao[i]));
-      }
-      if (lane_h == m) {
+        energy += gsel;
+        // carrier m's displacement and drift, a lane per axis
+        if (lane_h < 3) {
 #pragma clang fp contract(off)
-#pragma unroll
-        for (int c3 = 0; c3 < 3; ++c3) {
-          dsp[c3] += hv[c3];
-          if (field_on) drf[c3] = drf[c3] + hv[c3] * ksel;
+          const double v = ptab[rec_old].vec[lane_h];
+          lds_add(dsp + 3 * m + lane_h, v);
+          if (field_on) lds_add(drf + 3 * m + lane_h, v * ksel);
         }
-      }
-      __syncthreads();
-      const double v_new = uni(psi[m * zp + 1 + j]);
-      const double v_old = uni(psi[m * zp]);
-      double part[kFresh], fresh_v[kFresh];
+        // ---- apply
 #pragma unroll
-      for (int k = 0; k < kFresh; ++k) part[k] = q * double(fent[k]);
+        for (int i = 0; i < kP; ++i) psi[i] = fma(q, dx[i], psi[i]);
+        psi_s = fma(q, ds, psi_s);
+        double v_new = 0.0;
 #pragma unroll
-      for (int k = 0; k < kFresh; k += 4) wave_sum4(part + k, fresh_v + k);
+        for (int i = 0; i < kP; ++i)
+          if (kP == 1 || i == isel) v_new = read_lane(psi[i], src);
+        const double v_old = read_lane(psi_s, m);
+        // the fresh rows' sums over the carriers: fc + 32 to fc, those of
+        // fc + 16 and fc + 48 to them, then over the 16 lanes
+        double fresh[kT];
 #pragma unroll
-      for (int k = 0; k < kZp - 1; ++k)
-        fresh_v[k] = (k < z_h && nsel[k] != s_old) ? fresh_v[k] : v_old;
-      __syncthreads();
-      if (lane_h == 0) {
-        occ[m] = s_new;
-        cperm[m] = perm_new;
-        sites[m * zp] = s_new;
-        psi[m * zp] = v_new;
+        for (int t = 0; t < kT; ++t) {
+          double part[4];
 #pragma unroll
-        for (int k = 0; k < kZp - 1; ++k)
-          if (k < z_h) {
-            sites[m * zp + 1 + k] = nsel[k];
-            psi[m * zp + 1 + k] = fresh_v[k];
+          for (int u = 0; u < 4; ++u)
+            part[u] = fc_h + 16 * u < nc_h ? q * double(fent[t][u]) : 0.0;
+          double x = part[0];
+          if (nc_h > 16) {
+            if (nc_h > 32) x += part[2];
+            x += nc_h > 48 ? part[1] + part[3] : part[1];
           }
-      }
-      // ---- path rows [start, end), written by the owner lane of each entry
-      ++hops;
-      bool full = false;
-      if (end >= start + 1) {
-        if (end >= P) end = P;
-        if (lane_h < nc_h)
+          x += dpp_f64<kDppRowRor + 8, 0xf, true>(x);
+          x += dpp_f64<kDppRowRor + 4, 0xf, true>(x);
+          x += dpp_f64<kDppRowRor + 2, 0xf, true>(x);
+          x += dpp_f64<kDppRowRor + 1, 0xf, true>(x);
+          // (the slot that returns to s_old has its row already)
+          fresh[t] = nsite[t] != s_old ? x : v_old;
+        }
+        // carrier m's new processes and site row
 #pragma unroll
-          for (int c3 = 0; c3 < 3; ++c3) {
-            const int k = 3 * lane_h + c3;
-            const double v = sbase[k] + dsp[c3];
-            dsp[c3] = 0.0;
-            for (int32_t r = start; r < end; ++r)
-              rows[int64_t(r) * w + k] = v;
+        for (int i = 0; i < kP; ++i) {
+          uint32_t nx = lane_at(pd[i], nsite[0]);
+          uint32_t ni = lane_at(pd[i], ninfo[0]);
+          uint32_t nl = lane_at(pd[i], lo32(fresh[0]));
+          uint32_t nh = lane_at(pd[i], hi32(fresh[0]));
+          if constexpr (kT > 1)
+            if (z_h > 4) {
+              const bool far = pd[i] & 256;  // slots 4 to 7
+              const uint32_t fx = lane_at(pd[i], nsite[1]);
+              const uint32_t fi = lane_at(pd[i], ninfo[1]);
+              const uint32_t fl = lane_at(pd[i], lo32(fresh[1]));
+              const uint32_t fh = lane_at(pd[i], hi32(fresh[1]));
+              nx = far ? fx : nx;
+              ni = far ? fi : ni;
+              nl = far ? fl : nl;
+              nh = far ? fh : nh;
+            }
+          const bool mine = (pd[i] >> 9) == m;
+          px[i] = mine ? nx : px[i];
+          pinfo[i] = mine ? ni : pinfo[i];
+          psi[i] = mine ? from32(nl, nh) : psi[i];
+        }
+        sx = lane_h == m ? s_new : sx;
+        psi_s = lane_h == m ? v_new : psi_s;
+        // ---- path rows [start, end), written by the owner lane of each entry
+        ++hops;
+        bool full = false;
+        if (end >= start + 1) {
+          if (end >= P) end = P;
+          for (int k = lane_h; k < 3 * nc_h; k += 64) {
+            const double v = sbase[k] + dsp[k];
+            dsp[k] = 0.0;
+            for (int32_t r = start; r < end; ++r) rows[int64_t(r) * w + k] = v;
             sbase[k] = v;
           }
-        start = end;
-        full = end >= P;
+          start = end;
+          full = end >= P;
+        }
+        __syncthreads();
+        if (full) {
+          finished = true;
+          break;
+        }
       }
-      __syncthreads();
-      if (full) {
-        finished = true;
-        break;
-      }
-    }
+      // (the psi rows of carrier c: its site's, then its targets')
+#pragma unroll
+      for (int i = 0; i < kP; ++i)
+        if (pd[i] >= 0) spsi[(pd[i] >> 9) * zp + 1 + ((pd[i] >> 6) & 7)] = psi[i];
+      if (lane < nc) spsi[lane * zp] = psi_s;
+    });
     if (a.progress) {  // nothing left: out of its SIMD mates' way
       if (lane == 0)
         __hip_atomic_store(a.progress + pslot, 0u, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
       __builtin_amdgcn_s_setprio(0);
     }
-    save(box < 0 && finished);
+    // every carrier slot of the output, zero past the trajectory's own
+    static_assert(kMaxCarriers == 64, "one carrier per lane");
+#pragma unroll
+    for (int c3 = 0; c3 < 3; ++c3) {
+      const int k = lane + 64 * c3;
+      a.drift[int64_t(tr) * 3 * kMaxCarriers + k] = drf[k];
+      if (k < w) {
+        sdisp[k] = dsp[k];
+        sdrift[k] = drf[k];
+      }
+    }
+    for (int k = lane; k < 624; k += 64) mts[k] = mt[k];
+    if (lane < nc) socc[lane] = sx;
+    if (lane == 0) {
+      mts[624] = uint32_t(mti);
+      TrajOut o;
+      o.t = t_clk;
+      o.energy = energy;
+      o.hops = hops;
+      o.start = start;
+      o.no_select = no_select;
+      o.done = box < 0 && finished ? 1 : 0;
+      o.started = 1;
+      o.simd = int32_t(simd_key());
+      o.busy = (resume ? o0.busy : 0.0) + double(wall_clock64() - w_start);
+      a.out[tr] = o;
+    }
+    __syncthreads();
     if (box >= 0) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
       int handed = 0;
@@ -1293,6 +1341,7 @@ struct pycd_batch {
   DevBuf<uint32_t> d_prog;
   int n_bins = 1;
   uint32_t hand_cap = 0;  // mailboxes (0 for the serving pool)
+  int32_t hand_busy = 1;  // see BatchArgs
   bool handover = true;
   DevBuf<double> d_rows, d_drift, d_msd;
   DevBuf<TrajOut> d_out;

@@ -1,6 +1,6 @@
 // Wavefront-wide reductions and scans of FP64 values on gfx950: DPP row
-// moves, row broadcasts and the permlane16/32 swaps, no LDS.  Every lane of
-// the wavefront must be active.
+// moves and row broadcasts, no LDS.  Every lane of the wavefront must be
+// active.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -60,42 +60,6 @@ __device__ inline uint32_t hi32(double x) {
 }
 __device__ inline double from32(uint32_t lo, uint32_t hi) {
   return __longlong_as_double(int64_t((uint64_t(hi) << 32) | lo));
-}
-
-// a + b after rows 2-3 of a are exchanged with rows 0-1 of b: rows 0-1
-// hold 32 partial sums of a, rows 2-3 32 partial sums of b.
-__device__ inline double fold32(double a, double b) {
-  const auto l = __builtin_amdgcn_permlane32_swap(lo32(a), lo32(b), false,
-                                                  false);
-  const auto h = __builtin_amdgcn_permlane32_swap(hi32(a), hi32(b), false,
-                                                  false);
-  return from32(l[0], h[0]) + from32(l[1], h[1]);
-}
-
-// a + b after the odd rows of a are exchanged with the even rows of b:
-// rows 0 and 2 hold partial sums of a, rows 1 and 3 of b.
-__device__ inline double fold16(double a, double b) {
-  const auto l = __builtin_amdgcn_permlane16_swap(lo32(a), lo32(b), false,
-                                                  false);
-  const auto h = __builtin_amdgcn_permlane16_swap(hi32(a), hi32(b), false,
-                                                  false);
-  return from32(l[0], h[0]) + from32(l[1], h[1]);
-}
-
-// Four sums over the wavefront at once, returned in scalar registers: two
-// folds leave 16 partial sums of v[r] in row r, a rotation butterfly sums
-// each row.  (Four wave_sum calls would take four full reductions.)
-__device__ inline void wave_sum4(const double* v, double* out) {
-  double x = fold16(fold32(v[0], v[2]), fold32(v[1], v[3]));
-  // a rotation reads a lane of its own row for every lane, so the bound
-  // control (which would zero a missing source) never applies; setting it
-  // spares the zeroed old value of each move
-  x += dpp_f64<kDppRowRor + 8, 0xf, true>(x);
-  x += dpp_f64<kDppRowRor + 4, 0xf, true>(x);
-  x += dpp_f64<kDppRowRor + 2, 0xf, true>(x);
-  x += dpp_f64<kDppRowRor + 1, 0xf, true>(x);
-#pragma unroll
-  for (int r = 0; r < 4; ++r) out[r] = read_lane(x, 16 * r);
 }
 
 __device__ inline double wave_excl_scan(double v) {
