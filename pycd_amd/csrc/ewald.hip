@@ -85,8 +85,8 @@ typedef double v2d __attribute__((ext_vector_type(2)));
 template <int kB>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(2)))
-table_f64(const double* __restrict__ Y, int n, int Kp, EwaldScalars es,
-          double* __restrict__ A) {
+table_f64(const double* __restrict__ Y, int n, int Kp, int chunk,
+          EwaldScalars es, double* __restrict__ A) {
   constexpr int kTile = 32 * kB;
   constexpr int kRow = kSlice + 2;
   constexpr int kArr = kTile * kRow;
@@ -110,8 +110,10 @@ table_f64(const double* __restrict__ Y, int n, int Kp, EwaldScalars es,
   // the 128 bytes of a row
   const int lrow = t >> 3, lk = (t & 7) * 2;
   typedef const __attribute__((address_space(1))) v2d* gp;
-  const double* ya = Y + int64_t(i0 + lrow) * Kp + lk;
-  const double* yb = Y + int64_t(j0 + lrow) * Kp + lk;
+  // this workgroup's columns of Y: part blockIdx.y, `chunk` wide
+  const int kb = int(blockIdx.y) * chunk, kn = min(chunk, Kp - kb);
+  const double* ya = Y + int64_t(i0 + lrow) * Kp + kb + lk;
+  const double* yb = Y + int64_t(j0 + lrow) * Kp + kb + lk;
   v2d ra[kB], rb[kB];
   auto gload = [&](int k0) {
 #pragma unroll
@@ -179,21 +181,24 @@ table_f64(const double* __restrict__ Y, int n, int Kp, EwaldScalars es,
   auto step = [&](int stage, int k0) {
     k_step(0, stage, 1, [] {});
     k_step(1, stage, 2, [&] { sstore(stage ^ 1); });
-    k_step(0, stage, 3, [&] { gload(min(k0 + 2 * kSlice, Kp - kSlice)); });
+    k_step(0, stage, 3, [&] { gload(min(k0 + 2 * kSlice, kn - kSlice)); });
     lds_barrier();
     k_step(1, stage ^ 1, 0, [] {});
   };
   gload(0);
   sstore(0);
-  gload(min(kSlice, Kp - kSlice));
+  gload(min(kSlice, kn - kSlice));
   lds_barrier();
   fetch(0, 0, 0);
-  for (int k0 = 0; k0 < Kp; k0 += 2 * kSlice) {
+  for (int k0 = 0; k0 < kn; k0 += 2 * kSlice) {
     step(0, k0);
     step(1, k0 + kSlice);
   }
 
-  // the reciprocal part alone, no mirror: finish_table does the rest
+  // the reciprocal part alone (of several parts: the sum itself, each part
+  // its own table), no mirror: finish_table does the rest
+  const bool whole = gridDim.y == 1;
+  A += int64_t(blockIdx.y) * n * n;
 #pragma unroll
   for (int x = 0; x < kB; ++x)
 #pragma unroll
@@ -203,8 +208,45 @@ table_f64(const double* __restrict__ Y, int n, int Kp, EwaldScalars es,
 #pragma unroll
       for (int y = 0; y < kB; ++y)
         if (i < n && j0 + wc + 16 * y + (lane & 15) < n)
-          row[16 * y] = recip_part(es, acc[x][y][v]);
+          row[16 * y] =
+              whole ? recip_part(es, acc[x][y][v]) : acc[x][y][v];
     }
+}
+
+// Parts of the columns of Y.  A small table has few tiles, and a tile is a
+// serial chain of K steps: 120 sites, 3 tiles of 64 x 64 and 2 K = 6914,
+// took 197 us on 3 of 256 CUs.  The columns are split so that tiles times parts
+// come to about two workgroups per CU, each part of at least 8 slices; the
+// parts are added in order (reduce_parts): 10 + 5 us.  Against sums in
+// 80 bits the parts' error is a quarter of the chain's (7e-16 and 3e-15 of
+// the table there).  From 23 tiles a side (a workgroup per CU) there is one
+// part.  The count is by n and K alone, not by the tile, so that tile
+// variants keep giving the same table.
+int k_parts(int n, int Kp) {
+  const int nb = (n + 63) / 64, tiles = nb * (nb + 1) / 2;
+  return std::max(1, std::min(512 / tiles, Kp / (8 * kSlice)));
+}
+
+// Sum of the parts of every entry in the upper triangle of tiles (the
+// others hold nothing and are written by finish_table).
+__global__ void __launch_bounds__(256)
+reduce_parts(const double* __restrict__ P, int n, int parts, int tile,
+             EwaldScalars es, double* __restrict__ A) {
+  const int j = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int i = blockIdx.y * 4 + (threadIdx.x >> 6);
+  if (i >= n || j >= n || i / tile > j / tile) return;
+  const int64_t o = int64_t(i) * n + j, step = int64_t(n) * n;
+  double acc = P[o];
+  int k = 1;
+  for (; k + 8 <= parts; k += 8) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = P[o + (k + u) * step];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc += v[u];
+  }
+  for (; k < parts; ++k) acc += P[o + k * step];
+  A[o] = recip_part(es, acc);
 }
 
 // The rest of each entry after the contraction, and its mirror, one 64 x 64
@@ -216,19 +258,25 @@ table_f64(const double* __restrict__ Y, int n, int Kp, EwaldScalars es,
 // thread at two wavefronts per SIMD, and 8-byte mirror stores: 378 us in
 // one kernel at 2592 sites, 275 + 59 us apart.)  Off the diagonal tiles (j, i) is the same
 // number as (i, j): the same products in the same order, and squared
-// distances from negated differences (see store_pair).  A tile on the
+// distances from negated differences: fractional coordinates, the
+// round-half-even wrap and the candidate images (the kept offsets come in
+// +/- pairs) of (j, i) are the negatives of those of (i, j).  A tile on the
 // diagonal has both as formed, so its blocks write no mirror.
-template <int kTile>
+//
+// kRows: rows of a block.  16 instead of 64 where those blocks are fewer
+// than two per CU (120 sites: 18 -> 7 us).
+template <int kTile, int kRows>
 __global__ void __launch_bounds__(256)
 finish_table(const double* __restrict__ pos, int n, MicGeometry g,
              EwaldScalars es, double* __restrict__ A,
              unsigned long long* __restrict__ pairs) {
-  constexpr int kSub = kTile / 64;  // blocks per tile side
-  __shared__ double T[64][65];
+  constexpr int kCol = kTile / 64, kSub = kCol * (kTile / kRows);
+  __shared__ double T[kRows][65];
   int bi, bj;
-  tile_coords_upper_at(n, kTile, int(blockIdx.x) / (kSub * kSub), bi, bj);
-  const int sub = int(blockIdx.x) % (kSub * kSub);
-  const int i0 = bi * kTile + sub / kSub * 64, j0 = bj * kTile + sub % kSub * 64;
+  tile_coords_upper_at(n, kTile, int(blockIdx.x) / kSub, bi, bj);
+  const int sub = int(blockIdx.x) % kSub;
+  const int i0 = bi * kTile + sub / kCol * kRows;
+  const int j0 = bj * kTile + sub % kCol * 64;
   const bool mirror = bi != bj;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -237,7 +285,7 @@ finish_table(const double* __restrict__ pos, int n, MicGeometry g,
   const double pjx = j_ok ? pos[3 * j] : 0.0;
   const double pjy = j_ok ? pos[3 * j + 1] : 0.0;
   const double pjz = j_ok ? pos[3 * j + 2] : 0.0;
-  const int i_end = min(64, n - i0);
+  const int i_end = min(kRows, n - i0);
   unsigned cnt = 0;
   for (int k = wave; k < i_end; k += 4) {
     const int i = i0 + k;
@@ -255,20 +303,24 @@ finish_table(const double* __restrict__ pos, int n, MicGeometry g,
   count_pairs(mirror ? 2 * cnt : cnt, pairs);
   if (!mirror) return;
   __syncthreads();
-  const int j_end = min(64, n - j0);
-  if (lane < i_end)
-    for (int k = wave; k < j_end; k += 4)
-      A[int64_t(j0 + k) * n + i0 + lane] = T[lane][k];
+  // rows of the mirror, kRows entries each
+  constexpr int kPer = 64 / kRows;
+  const int j_end = min(64, n - j0), r = lane % kRows;
+  if (r < i_end)
+    for (int k = kPer * wave + lane / kRows; k < j_end; k += 4 * kPer)
+      A[int64_t(j0 + k) * n + i0 + r] = T[r][k];
 }
 
 void launch_finish(hipStream_t s, int tile, const double* pos, int n,
                    const MicGeometry& geo, const EwaldScalars& es, double* A,
                    unsigned long long* pairs) {
   const int nb = (n + tile - 1) / tile, tiles = nb * (nb + 1) / 2;
-  if (tile == 64)
-    finish_table<64><<<tiles, 256, 0, s>>>(pos, n, geo, es, A, pairs);
+  if (tile != 64)
+    finish_table<128, 64><<<4 * tiles, 256, 0, s>>>(pos, n, geo, es, A, pairs);
+  else if (tiles >= 512)
+    finish_table<64, 64><<<tiles, 256, 0, s>>>(pos, n, geo, es, A, pairs);
   else
-    finish_table<128><<<4 * tiles, 256, 0, s>>>(pos, n, geo, es, A, pairs);
+    finish_table<64, 16><<<4 * tiles, 256, 0, s>>>(pos, n, geo, es, A, pairs);
 }
 
 // ------------------------------------------------------------------ launch
@@ -276,18 +328,16 @@ int launch_table_mfma(pycd_ctx* ctx, int precision, const double* pos, int n,
                       const double* kv, const double* sw, int K,
                       const MicGeometry& geo, const EwaldScalars& es,
                       double* out, unsigned long long* pairs,
-                      hipEvent_t after_sf, hipEvent_t (&real)[2],
-                      bool& real_apart);
+                      hipEvent_t after_sf, hipEvent_t (&real)[2]);
 
 int launch_table(pycd_ctx* ctx, int precision, const double* pos, int n,
                  const double* kv, const double* sw, int K,
                  const MicGeometry& geo, const EwaldScalars& es, double* out,
                  unsigned long long* pairs, hipEvent_t after_sf,
-                 hipEvent_t (&real)[2], bool& real_apart) {
-  real_apart = false;
+                 hipEvent_t (&real)[2]) {
   if (precision != PYCD_PREC_F64)
     return launch_table_mfma(ctx, precision, pos, n, kv, sw, K, geo, es, out,
-                             pairs, after_sf, real, real_apart);
+                             pairs, after_sf, real);
   hipStream_t s = ctx->stream;
   // tile variant: 1 = 64 x 64, 2 = 128 x 128; 0 picks 128 from 2048 sites
   int v = ctx->table_variant[PYCD_PREC_F64];
@@ -305,12 +355,24 @@ int launch_table(pycd_ctx* ctx, int precision, const double* pos, int n,
                          256, 0, s>>>(pos, n, n_pad, kv, sw, K, Kp, Y.ptr);
   PYCD_HIP(ctx, hipGetLastError());
   PYCD_HIP(ctx, hipEventRecord(after_sf, s));
+  // (parts of whole pairs of slices, none empty)
+  const int want = k_parts(n, Kp);
+  const int chunk = (Kp / pair + want - 1) / want * pair;
+  const int parts = (Kp + chunk - 1) / chunk;
+  DevBuf<double> P;
+  if (parts > 1) PYCD_HIP(ctx, P.alloc(size_t(parts) * n * n));
+  double* sums = parts > 1 ? P.ptr : out;
+  const dim3 grid(nb * (nb + 1) / 2, parts);
   if (v == 2)
-    table_f64<4><<<nb * (nb + 1) / 2, 256, 0, s>>>(Y.ptr, n, Kp, es, out);
+    table_f64<4><<<grid, 256, 0, s>>>(Y.ptr, n, Kp, chunk, es, sums);
   else
-    table_f64<2><<<nb * (nb + 1) / 2, 256, 0, s>>>(Y.ptr, n, Kp, es, out);
+    table_f64<2><<<grid, 256, 0, s>>>(Y.ptr, n, Kp, chunk, es, sums);
   PYCD_HIP(ctx, hipGetLastError());
-  real_apart = true;
+  if (parts > 1) {
+    reduce_parts<<<dim3((n + 63) / 64, (n + 3) / 4), 256, 0, s>>>(
+        P.ptr, n, parts, tile, es, out);
+    PYCD_HIP(ctx, hipGetLastError());
+  }
   PYCD_HIP(ctx, hipEventRecord(real[0], s));
   launch_finish(s, tile, pos, n, geo, es, out, pairs);
   PYCD_HIP(ctx, hipEventRecord(real[1], s));
@@ -412,6 +474,12 @@ extern "C" int pycd_pair_table(pycd_ctx* ctx, const double* pos, int64_t n,
   es.eps = eps_r;
   es.self_term = -1.0 * std::sqrt(alpha / M_PI) / eps_r;
   es.unit_eps = eps_r == 1.0;
+  // (the margins are far above the rounding of f)
+  for (int k = 0; k < 3; ++k) {
+    const double* c = st.geo.inv + k;
+    es.far[k] = r_cut * std::sqrt(c[0] * c[0] + c[3] * c[3] + c[6] * c[6]) *
+                    (1.0 + 1e-9) + 1e-9;
+  }
 
   DevBuf<double> d_pos, d_kv, d_sw, d_A;
   DevBuf<unsigned long long> d_pairs;
@@ -440,9 +508,8 @@ extern "C" int pycd_pair_table(pycd_ctx* ctx, const double* pos, int64_t n,
   for (auto& e : ev) PYCD_HIP(ctx, hipEventCreate(&e));
   for (auto& e : real) PYCD_HIP(ctx, hipEventCreate(&e));
   PYCD_HIP(ctx, hipEventRecord(ev[0], s));
-  bool real_apart = false;
   rc = launch_table(ctx, precision, d_pos.ptr, N, d_kv.ptr, d_sw.ptr, K, st.geo,
-                    es, out, d_pairs.ptr, ev[1], real, real_apart);
+                    es, out, d_pairs.ptr, ev[1], real);
   if (rc) {
     for (auto& e : ev) (void)hipEventDestroy(e);
     for (auto& e : real) (void)hipEventDestroy(e);
@@ -459,7 +526,7 @@ extern "C" int pycd_pair_table(pycd_ctx* ctx, const double* pos, int64_t n,
   float ms_sf = 0, ms_rest = 0, ms_real = 0;
   (void)hipEventElapsedTime(&ms_sf, ev[0], ev[1]);
   (void)hipEventElapsedTime(&ms_rest, ev[1], ev[2]);
-  if (real_apart) (void)hipEventElapsedTime(&ms_real, real[0], real[1]);
+  (void)hipEventElapsedTime(&ms_real, real[0], real[1]);
   for (auto& e : ev) (void)hipEventDestroy(e);
   for (auto& e : real) (void)hipEventDestroy(e);
   if (report) {

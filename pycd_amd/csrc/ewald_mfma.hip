@@ -6,15 +6,15 @@
 //   BF16X3  Y = hi + lo with hi = bf16(Y), lo = bf16(Y - hi) (both from the
 //           FP64 structure factor), Y Y^T ~ hi hi^T + hi lo^T + lo hi^T on
 //           v_mfma_f32_16x16x32_bf16, FP32 accumulation.
-// The real-space term (minimum image, erfc), the self term and the final
-// FP64 store are the FP64 epilogue shared with the FP64 kernel, so only the
-// reciprocal sum carries the reduced precision.
+// The real-space term (minimum image, erfc) and the self term are added in
+// FP64 by finish_table, as for the FP64 kernel, so only the reciprocal sum
+// carries the reduced precision.
 //
 // Tiling: 256 threads = 4 wavefronts per 128 x 128 output tile; each
 // wavefront owns 64 x 64 = 4 x 4 MFMA blocks of 16 x 16.  K is staged
-// through LDS in slices of 32 (row-major, padded rows); the global loads of
-// the next slice are in flight while the current one is multiplied.  The
-// BF16X3 mode also has two-stage kernels (one barrier per slice, loads two
+// through LDS in slices (row-major, padded rows); the global loads of the
+// next slice are in flight while the current one is multiplied.  The F32
+// mode has two stages; the BF16X3 mode also has two-stage kernels (one barrier per slice, loads two
 // or three slices ahead) on 128 x 128 tiles and on 256 x 256 tiles of 8
 // wavefronts; the latter is the default from 4096 sites on.
 #include "ewald_common.hpp"
@@ -27,7 +27,6 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 constexpr int kMTile = 128;
-constexpr int kMSlice = 32;
 
 // 16-byte load through a global (address-space-1) pointer.  A generic
 // pointer would compile to a flat load, which also counts against the LDS
@@ -43,124 +42,181 @@ __device__ inline float4 load16f_global(const void* p) {
                      __uint_as_float(v.z), __uint_as_float(v.w));
 }
 
-// Structure factors in reduced precision from the FP64 values.
+// Structure factors in reduced precision from the FP64 values, a thread one
+// k column of kLowRows rows, its k vector in registers; columns past 2 K and
+// rows past n are written as zeros here rather than by fills of the whole
+// array ahead (which, with a division per element for its row, took 0.29 +
+// 0.07 ms at 12000 sites and 2 K = 9834, now 0.23).
+constexpr int kLowRows = 16;
+template <int kMode>
 __global__ void __launch_bounds__(256)
-structure_factor_lowp(const double* __restrict__ pos, int n,
+structure_factor_lowp(const double* __restrict__ pos, int n, int n_pad,
                       const double* __restrict__ kv,
-                      const double* __restrict__ sw, int K, int Kp, int mode,
+                      const double* __restrict__ sw, int K, int Kp,
                       float* __restrict__ y32, __bf16* __restrict__ yhi,
                       __bf16* __restrict__ ylo) {
-  const int64_t total = int64_t(n) * K;
-  for (int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-       idx < total; idx += int64_t(gridDim.x) * blockDim.x) {
-    const int i = int(idx / K);
-    const int m = int(idx - int64_t(i) * K);
-    const double ph = kv[3 * m] * pos[3 * i] + kv[3 * m + 1] * pos[3 * i + 1] +
-                      kv[3 * m + 2] * pos[3 * i + 2];
-    double s, c;
-    sincos(ph, &s, &c);
-    const double vc = sw[m] * c, vs = sw[m] * s;
-    const int64_t oc = int64_t(i) * Kp + m, os = int64_t(i) * Kp + K + m;
-    if (mode == PYCD_PREC_F32) {
-      y32[oc] = float(vc);
-      y32[os] = float(vs);
+  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  if (m >= Kp - K) return;
+  const bool real = m < K;
+  const double kx = real ? kv[3 * m] : 0.0, ky = real ? kv[3 * m + 1] : 0.0,
+               kz = real ? kv[3 * m + 2] : 0.0, w = real ? sw[m] : 0.0;
+  // w v and, in two parts, its rounding to BF16 (of a cosine by way of
+  // FP32: a few ties in 1e8 go to the even neighbour, the low part makes up
+  // for it) and what that leaves
+  auto put = [&](int64_t o, double v, bool by_f32) {
+#pragma clang fp contract(off)
+    const double y = w * v;
+    if constexpr (kMode == PYCD_PREC_F32) {
+      y32[o] = float(y);
     } else {
-      const __bf16 hc = __bf16(float(vc)), hs = __bf16(float(vs));
-      yhi[oc] = hc;
-      yhi[os] = hs;
-      ylo[oc] = __bf16(float(vc - double(float(hc))));
-      ylo[os] = __bf16(float(vs - double(float(hs))));
+      float f = float(y);
+      asm volatile("" : "+v"(f));  // (rounded here, not folded)
+      const __bf16 h = by_f32 ? __bf16(f) : __bf16(y);
+      yhi[o] = h;
+      ylo[o] = __bf16(y - double(float(h)));
     }
+  };
+  const int i0 = blockIdx.y * kLowRows, i1 = min(i0 + kLowRows, n_pad);
+  for (int i = i0; i < i1; ++i) {
+    double s = 0.0, c = 0.0;
+    if (real && i < n) {
+      const double ph = kx * pos[3 * i] + ky * pos[3 * i + 1] +
+                        kz * pos[3 * i + 2];
+      sincos(ph, &s, &c);
+    }
+    const int64_t row = int64_t(i) * Kp;
+    if (real) put(row + m, c, true);
+    put(row + K + m, s, false);
   }
 }
 
+// The reciprocal part of a wavefront's kX x kY blocks of 16 x 16, at
+// (i0, j0), into the table; finish_table does the rest.
+template <int kX, int kY>
+__device__ __forceinline__ void store_recip(const v4f (&acc)[kX][kY],
+                                            double* __restrict__ A, int n,
+                                            int i0, int j0,
+                                            const EwaldScalars& es) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int x = 0; x < kX; ++x)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = i0 + 16 * x + (lane >> 4) * 4 + r;
+      double* row = A + int64_t(i) * n + j0 + (lane & 15);
+#pragma unroll
+      for (int y = 0; y < kY; ++y)
+        if (i < n && j0 + 16 * y + (lane & 15) < n)
+          row[16 * y] = recip_part(es, double(acc[x][y][r]));
+    }
+}
+
+// One (32 kB) x (32 kB) tile per workgroup, each wavefront a quarter of it
+// in kB x kB blocks of v_mfma_f32_16x16x4: lane l gives row (column) l mod 16
+// at k + l / 16.  Bound by the FP32 matrix rate.  K goes through LDS in
+// slices of 16 in two stages, one barrier per slice, global loads two slices
+// ahead and each k step's fragments read behind the last step's products
+// (see table_f64, which this mirrors); rows of 16 + 4 floats put a
+// wavefront's 64 reads on distinct banks, and the 40 KB of a 128 x 128
+// workgroup let four share a CU, so that the few tiles per CU of a table
+// (4.6 at 6144 sites) are worked on side by side.  With one stage, two
+// barriers a slice and the rest of the entries in the epilogue: 2.07 ms at
+// 6144 sites and 2 K = 5036 (1.3 at the matrix rate); now 1.65 and 0.15 for
+// finish_table.  64 x 64 tiles below 2048 sites, as for table_f64.  Every
+// entry is the chain over k whatever the tile.
+constexpr int kFSlice = 16;
+template <int kB>
 __global__ void __launch_bounds__(256)
-table_mfma_f32(const float* __restrict__ Y, int n, int Kp,
-               const double* __restrict__ pos, MicGeometry g, EwaldScalars es,
-               double* __restrict__ A, unsigned long long* __restrict__ pairs) {
-  __shared__ float As[kMTile][kMSlice + 1];
-  __shared__ float Bs[kMTile][kMSlice + 1];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+__attribute__((amdgpu_waves_per_eu(4)))
+table_mfma_f32(const float* __restrict__ Y, int n, int Kp, EwaldScalars es,
+               double* __restrict__ A) {
+  constexpr int kTile = 32 * kB;
+  constexpr int kRow = kFSlice + 4;
+  constexpr int kArr = kTile * kRow;
+  constexpr int kQ = kTile / 64;  // 16-byte chunks per thread and operand
+  // stage s, operand a at S + (2 s + a) kArr
+  __shared__ __attribute__((aligned(16))) float S[4 * kArr];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   int bi, bj;
-  tile_coords_upper(n, kMTile, bi, bj);
-  const int i0 = bi * kMTile, j0 = bj * kMTile;
-  const bool mirror = bi != bj;
-  const int wr = (wave >> 1) * 64, wc = (wave & 1) * 64;
-  v4f acc[4][4];
+  tile_coords_upper(n, kTile, bi, bj);
+  const int i0 = bi * kTile, j0 = bj * kTile;
+  const int wr = (wave >> 1) * (kTile / 2), wc = (wave & 1) * (kTile / 2);
+  v4f acc[kB][kB];
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int x = 0; x < kB; ++x)
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = v4f{0.f, 0.f, 0.f, 0.f};
-  const int lrow = t >> 1, lk = (t & 1) * 16;
-  const bool a_ok = i0 + lrow < n, b_ok = j0 + lrow < n;
+    for (int y = 0; y < kB; ++y) acc[x][y] = v4f{0.f, 0.f, 0.f, 0.f};
+  // loader: a thread takes 4 consecutive k of every 64th row
+  const int lrow = t >> 2, lk = (t & 3) * 4;
   const float* ya = Y + int64_t(i0 + lrow) * Kp + lk;
   const float* yb = Y + int64_t(j0 + lrow) * Kp + lk;
-  // software pipeline: slice k0 + kMSlice is loaded into registers while the
-  // matrix cores work on slice k0 from LDS
-  float4 va[4], vb[4];
+  float4 ra[kQ], rb[kQ];
   auto gload = [&](int k0) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      va[q] = a_ok ? load16f_global(ya + k0 + 4 * q)
-                   : make_float4(0.f, 0.f, 0.f, 0.f);
-      vb[q] = b_ok ? load16f_global(yb + k0 + 4 * q)
-                   : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int q = 0; q < kQ; ++q) {
+      ra[q] = load16f_global(ya + int64_t(64 * q) * Kp + k0);
+      rb[q] = load16f_global(yb + int64_t(64 * q) * Kp + k0);
     }
   };
-  auto sstore = [&]() {
+  auto sstore = [&](int stage) {
+    float* a = S + 2 * stage * kArr + lrow * kRow + lk;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      As[lrow][lk + 4 * q + 0] = va[q].x;
-      As[lrow][lk + 4 * q + 1] = va[q].y;
-      As[lrow][lk + 4 * q + 2] = va[q].z;
-      As[lrow][lk + 4 * q + 3] = va[q].w;
-      Bs[lrow][lk + 4 * q + 0] = vb[q].x;
-      Bs[lrow][lk + 4 * q + 1] = vb[q].y;
-      Bs[lrow][lk + 4 * q + 2] = vb[q].z;
-      Bs[lrow][lk + 4 * q + 3] = vb[q].w;
+    for (int q = 0; q < kQ; ++q) {
+      *reinterpret_cast<float4*>(a + 64 * q * kRow) = ra[q];
+      *reinterpret_cast<float4*>(a + kArr + 64 * q * kRow) = rb[q];
     }
+  };
+  auto lds_barrier = [] {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  float fa[2][kB], fb[2][kB];
+  auto fetch = [&](int set, int stage, int u) {
+    const float* a = S + 2 * stage * kArr + (wr + (lane & 15)) * kRow +
+                     (lane >> 4) + 4 * u;
+    const float* b = S + (2 * stage + 1) * kArr + (wc + (lane & 15)) * kRow +
+                     (lane >> 4) + 4 * u;
+#pragma unroll
+    for (int x = 0; x < kB; ++x) {
+      fa[set][x] = a[16 * x * kRow];
+      fb[set][x] = b[16 * x * kRow];
+    }
+  };
+  auto k_step = [&](int set, int next_stage, int next_u, auto&& more) {
+    fetch(set ^ 1, next_stage, next_u);
+    more();
+#pragma unroll
+    for (int x = 0; x < kB; ++x)
+#pragma unroll
+      for (int y = 0; y < kB; ++y)
+        acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+            fa[set][x], fb[set][y], acc[x][y], 0, 0, 0);
+#pragma unroll
+    for (int q = 0; q < 2 * kB; ++q) {
+      __builtin_amdgcn_sched_group_barrier(0x008, kB / 2, 0);  // MFMA
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);       // LDS read
+      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);       // LDS write
+      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);       // global load
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto step = [&](int stage, int k0) {
+    k_step(0, stage, 1, [] {});
+    k_step(1, stage, 2, [&] { sstore(stage ^ 1); });
+    k_step(0, stage, 3, [&] { gload(min(k0 + 2 * kFSlice, Kp - kFSlice)); });
+    lds_barrier();
+    k_step(1, stage ^ 1, 0, [] {});
   };
   gload(0);
-  sstore();
-  __syncthreads();
-  for (int k0 = 0; k0 < Kp; k0 += kMSlice) {
-    const bool more = k0 + kMSlice < Kp;
-    if (more) gload(k0 + kMSlice);
-#pragma unroll
-    for (int kk = 0; kk < kMSlice; kk += 4) {
-      float a[4], b[4];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        a[x] = As[wr + 16 * x + (lane & 15)][kk + (lane >> 4)];
-        b[x] = Bs[wc + 16 * x + (lane & 15)][kk + (lane >> 4)];
-      }
-#pragma unroll
-      for (int x = 0; x < 4; ++x)
-#pragma unroll
-        for (int y = 0; y < 4; ++y)
-          acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x], b[y],
-                                                           acc[x][y], 0, 0, 0);
-    }
-    __syncthreads();  // every wavefront is done with this slice
-    if (more) sstore();
-    __syncthreads();
+  sstore(0);
+  gload(min(kFSlice, Kp - kFSlice));
+  lds_barrier();
+  fetch(0, 0, 0);
+  for (int k0 = 0; k0 < Kp; k0 += 2 * kFSlice) {
+    step(0, k0);
+    step(1, k0 + kFSlice);
   }
-  unsigned cnt = 0;
-  // entry (i, j) and, off the diagonal block, its mirror (j, i): the same
-  // number, formed once (store_pair)
-#pragma unroll
-  for (int x = 0; x < 4; ++x)
-#pragma unroll
-    for (int y = 0; y < 4; ++y)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = i0 + wr + 16 * x + (lane >> 4) * 4 + r;
-        const int j = j0 + wc + 16 * y + (lane & 15);
-        if (i < n && j < n)
-          store_pair(A, n, i, j, mirror, pos, g, es, double(acc[x][y][r]),
-                     cnt);
-      }
-  count_pairs(cnt, pairs);
+  store_recip<kB, kB>(acc, A, n, i0 + wr, j0 + wc, es);
 }
 
 // K is staged in slices of kBSlice = 32 or 64: a 64-deep slice makes two
@@ -174,9 +230,7 @@ __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(2, 2)))
 table_mfma_bf16x3(const __bf16* __restrict__ Yhi,
                   const __bf16* __restrict__ Ylo, int n, int Kp,
-                  const double* __restrict__ pos, MicGeometry g,
-                  EwaldScalars es, double* __restrict__ A,
-                  unsigned long long* __restrict__ pairs) {
+                  EwaldScalars es, double* __restrict__ A) {
   constexpr int kRow = kBSlice + 8;  // padded row (bf16 elements)
   __shared__ __attribute__((aligned(16))) __bf16 Ah[kMTile * kRow];
   __shared__ __attribute__((aligned(16))) __bf16 Al[kMTile * kRow];
@@ -186,7 +240,6 @@ table_mfma_bf16x3(const __bf16* __restrict__ Yhi,
   int bi, bj;
   tile_coords_upper(n, kMTile, bi, bj);
   const int i0 = bi * kMTile, j0 = bj * kMTile;
-  const bool mirror = bi != bj;
   const int wr = (wave >> 1) * 64, wc = (wave & 1) * 64;
   v4f acc[4][4];
 #pragma unroll
@@ -257,22 +310,7 @@ table_mfma_bf16x3(const __bf16* __restrict__ Yhi,
     if (more) sstore();
     __syncthreads();
   }
-  unsigned cnt = 0;
-  // entry (i, j) and, off the diagonal block, its mirror (j, i): the same
-  // number, formed once (store_pair)
-#pragma unroll
-  for (int x = 0; x < 4; ++x)
-#pragma unroll
-    for (int y = 0; y < 4; ++y)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = i0 + wr + 16 * x + (lane >> 4) * 4 + r;
-        const int j = j0 + wc + 16 * y + (lane & 15);
-        if (i < n && j < n)
-          store_pair(A, n, i, j, mirror, pos, g, es, double(acc[x][y][r]),
-                     cnt);
-      }
-  count_pairs(cnt, pairs);
+  store_recip<4, 4>(acc, A, n, i0 + wr, j0 + wc, es);
 }
 
 // K slices of 32 in two LDS stages and three register sets: while slice t
@@ -290,9 +328,7 @@ __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(2, 2)))
 table_mfma_bf16x3_2stage(const __bf16* __restrict__ Yhi,
                          const __bf16* __restrict__ Ylo, int n, int Kp,
-                         const double* __restrict__ pos, MicGeometry g,
-                         EwaldScalars es, double* __restrict__ A,
-                         unsigned long long* __restrict__ pairs) {
+                         EwaldScalars es, double* __restrict__ A) {
   constexpr int kB = 32;
   constexpr int kRow = kB + 8;  // padded row (bf16 elements)
   constexpr int kArr = kMTile * kRow;
@@ -302,7 +338,6 @@ table_mfma_bf16x3_2stage(const __bf16* __restrict__ Yhi,
   int bi, bj;
   tile_coords_upper(n, kMTile, bi, bj);
   const int i0 = bi * kMTile, j0 = bj * kMTile;
-  const bool mirror = bi != bj;
   const int wr = (wave >> 1) * 64, wc = (wave & 1) * 64;
   v4f acc[4][4];
 #pragma unroll
@@ -393,22 +428,7 @@ table_mfma_bf16x3_2stage(const __bf16* __restrict__ Yhi,
     step(0, k0 + 4 * kB, r2, r1);
     step(1, k0 + 5 * kB, r0, r2);
   }
-  unsigned cnt = 0;
-  // entry (i, j) and, off the diagonal block, its mirror (j, i): the same
-  // number, formed once (store_pair)
-#pragma unroll
-  for (int x = 0; x < 4; ++x)
-#pragma unroll
-    for (int y = 0; y < 4; ++y)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = i0 + wr + 16 * x + (lane >> 4) * 4 + r;
-        const int j = j0 + wc + 16 * y + (lane & 15);
-        if (i < n && j < n)
-          store_pair(A, n, i, j, mirror, pos, g, es, double(acc[x][y][r]),
-                     cnt);
-      }
-  count_pairs(cnt, pairs);
+  store_recip<4, 4>(acc, A, n, i0 + wr, j0 + wc, es);
 }
 
 // 256 x 256 output tiles on 8 wavefronts (512 threads), each wavefront
@@ -423,10 +443,7 @@ table_mfma_bf16x3_2stage(const __bf16* __restrict__ Yhi,
 // block is not stored, its upper mirror writes it (as a 128 x 128 tile off
 // the diagonal does), and the two diagonal 128-blocks store both (i, j) and
 // (j, i) as formed.  Y holds whole 256-row tiles and Kp is a multiple of
-// 2 kB, so loads and LDS stores are unconditional.  The real-space part of
-// each entry it forms is in A already (table_real_part), so the epilogue
-// adds the reciprocal and self terms to it: the same operations, in the
-// same order, as store_pair.
+// 2 kB, so loads and LDS stores are unconditional.
 constexpr int kMTile2 = 256;
 
 // Two 128 x 128 tiles in one 512-thread workgroup of the 256 x 256 kernel,
@@ -450,7 +467,6 @@ __device__ __forceinline__ void bf16x3_tile_pair(
   if (dummy) idx = 2 * k;
   const int2 tl = sub[idx];
   const int i0 = tl.x * kMTile, j0 = tl.y * kMTile;
-  const bool mirror = tl.x != tl.y;
   const int wr = (wave >> 1) * 64, wc = (wave & 1) * 64;
   __bf16* Sh = S + half * (2 * 4 * kArr);
   v4f acc[4][4];
@@ -529,58 +545,7 @@ __device__ __forceinline__ void bf16x3_tile_pair(
     step(1, k0 + kB);
   }
   if (dummy) return;
-#pragma unroll
-  for (int x = 0; x < 4; ++x)
-#pragma unroll
-    for (int y = 0; y < 4; ++y)
-#pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) {
-        const int i = i0 + wr + 16 * x + (lane >> 4) * 4 + r4;
-        const int j = j0 + wc + 16 * y + (lane & 15);
-        if (i < n && j < n) {
-          const double v = finish_entry(i, j, es, A[int64_t(i) * n + j],
-                                        double(acc[x][y][r4]));
-          A[int64_t(i) * n + j] = v;
-          if (mirror) A[int64_t(j) * n + i] = v;
-        }
-      }
-}
-
-// Real-space part of every entry that a pass over 128 x 128 tiles forms as
-// (i, j) (tile row <= tile column), into A ahead of the contraction, with
-// the pairs within r_cut counted as store_pair counts them (a tile off the
-// diagonal also for its mirror).  One 256-thread workgroup per tile, full
-// occupancy: the minimum image and erfc run while no matrix work waits.
-__global__ void __launch_bounds__(256)
-table_real_part(const double* __restrict__ pos, int n, MicGeometry g,
-                EwaldScalars es, double* __restrict__ A,
-                unsigned long long* __restrict__ pairs) {
-  int bi, bj;
-  tile_coords_upper(n, kMTile, bi, bj);
-  const int i0 = bi * kMTile, j0 = bj * kMTile;
-  const bool mirror = bi != bj;
-  // a lane keeps its column j; a wavefront walks rows i the same for all
-  // of its lanes (every other row, the two halves of the workgroup
-  // interleaved), so the row positions come through scalar loads
-  const int j = j0 + (threadIdx.x & (kMTile - 1));
-  const int ih = __builtin_amdgcn_readfirstlane(threadIdx.x / kMTile);
-  const bool j_ok = j < n;
-  const double pjx = j_ok ? pos[3 * j] : 0.0;
-  const double pjy = j_ok ? pos[3 * j + 1] : 0.0;
-  const double pjz = j_ok ? pos[3 * j + 2] : 0.0;
-  const int i_end = min(kMTile, n - i0);
-  unsigned cnt = 0;
-  for (int k = ih; k < i_end; k += 2) {
-    const int i = i0 + k;
-    if (j_ok) {
-      const unsigned before = cnt;
-      A[int64_t(i) * n + j] =
-          real_part_d(i, j, pjx - pos[3 * i], pjy - pos[3 * i + 1],
-                      pjz - pos[3 * i + 2], g, es, cnt);
-      if (mirror) cnt += cnt - before;
-    }
-  }
-  count_pairs(cnt, pairs);
+  store_recip<4, 4>(acc, A, n, i0 + wr, j0 + wc, es);
 }
 
 __global__ void __launch_bounds__(512)
@@ -608,11 +573,8 @@ table_mfma_bf16x3_256(const __bf16* __restrict__ Yhi,
   tile_coords_upper(n, kMTile2, bi, bj);
   const int i0 = bi * kMTile2, j0 = bj * kMTile2;
   const int wr = (wave >> 2) * 128, wc = (wave & 3) * 64;
-  // in a diagonal tile: the upper-right 128-block is stored with its mirror,
-  // the lower-left one not at all
-  const bool diag = bi == bj;
-  const bool mirror = !diag || (wr == 0 && wc >= 128);
-  const bool skip = diag && wr == 128 && wc < 128;
+  // in a diagonal tile the lower-left 128-block is not stored
+  const bool skip = bi == bj && wr == 128 && wc < 128;
   v4f acc[8][4];
 #pragma unroll
   for (int a = 0; a < 8; ++a)
@@ -694,29 +656,14 @@ table_mfma_bf16x3_256(const __bf16* __restrict__ Yhi,
     step(1, k0 + kB);
   }
   if (skip) return;
-#pragma unroll
-  for (int x = 0; x < 8; ++x)
-#pragma unroll
-    for (int y = 0; y < 4; ++y)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = i0 + wr + 16 * x + (lane >> 4) * 4 + r;
-        const int j = j0 + wc + 16 * y + (lane & 15);
-        if (i < n && j < n) {
-          const double v = finish_entry(i, j, es, A[int64_t(i) * n + j],
-                                        double(acc[x][y][r]));
-          A[int64_t(i) * n + j] = v;
-          if (mirror) A[int64_t(j) * n + i] = v;
-        }
-      }
+  store_recip<8, 4>(acc, A, n, i0 + wr, j0 + wc, es);
 }
 
 int launch_table_mfma(pycd_ctx* ctx, int precision, const double* pos, int n,
                       const double* kv, const double* sw, int K,
                       const MicGeometry& geo, const EwaldScalars& es,
                       double* out, unsigned long long* pairs,
-                      hipEvent_t after_sf, hipEvent_t (&real)[2],
-                      bool& real_apart) {
+                      hipEvent_t after_sf, hipEvent_t (&real)[2]) {
   hipStream_t s = ctx->stream;
   // K padded to whole slices of the mode's kernel (zero columns add nothing)
   // BF16x3 default: 256 x 256 tiles from 4096 sites on, K slices of 64
@@ -725,53 +672,42 @@ int launch_table_mfma(pycd_ctx* ctx, int precision, const double* pos, int n,
   if (bvar == 0) bvar = n >= 4096 ? 4 : 2;
   const int bslice = bvar == 1 || bvar >= 3 ? 32 : 64;
   // (the two-stage kernels take K in groups of six and of two 32-slices)
-  const int slice = precision == PYCD_PREC_F32 ? kMSlice
+  const int slice = precision == PYCD_PREC_F32 ? 2 * kFSlice
                     : bvar == 3              ? 6 * bslice
                     : bvar == 4              ? 2 * bslice
                                              : bslice;
   const int Kp = std::max(slice, ((2 * K + slice - 1) / slice) * slice);
   // rows in whole tiles: the rows past n stay zero
   const int tile = precision == PYCD_PREC_BF16X3 && bvar == 4 ? kMTile2
+                   : precision == PYCD_PREC_F32 && n < 2048   ? 64
                                                               : kMTile;
   const int nb = (n + tile - 1) / tile;
-  const size_t elems = size_t(nb) * tile * Kp;
+  const int n_pad = nb * tile;
+  const size_t elems = size_t(n_pad) * Kp;
   DevBuf<float> y32;
   DevBuf<__bf16> yhi, ylo;
+  const dim3 sf_grid((Kp - K + 255) / 256, (n_pad + kLowRows - 1) / kLowRows);
   if (precision == PYCD_PREC_F32) {
     PYCD_HIP(ctx, y32.alloc(elems));
-    PYCD_HIP(ctx, hipMemsetAsync(y32.ptr, 0, elems * sizeof(float), s));
+    structure_factor_lowp<PYCD_PREC_F32><<<sf_grid, 256, 0, s>>>(
+        pos, n, n_pad, kv, sw, K, Kp, y32.ptr, nullptr, nullptr);
   } else {
     PYCD_HIP(ctx, yhi.alloc(elems));
     PYCD_HIP(ctx, ylo.alloc(elems));
-    PYCD_HIP(ctx, hipMemsetAsync(yhi.ptr, 0, elems * sizeof(__bf16), s));
-    PYCD_HIP(ctx, hipMemsetAsync(ylo.ptr, 0, elems * sizeof(__bf16), s));
+    structure_factor_lowp<PYCD_PREC_BF16X3><<<sf_grid, 256, 0, s>>>(
+        pos, n, n_pad, kv, sw, K, Kp, nullptr, yhi.ptr, ylo.ptr);
   }
-  if (K > 0) {
-    const int64_t total = int64_t(n) * K;
-    const int blocks = int(std::min<int64_t>((total + 255) / 256, 65536));
-    structure_factor_lowp<<<blocks, 256, 0, s>>>(pos, n, kv, sw, K, Kp,
-                                                 precision, y32.ptr, yhi.ptr,
-                                                 ylo.ptr);
-    PYCD_HIP(ctx, hipGetLastError());
-  }
+  PYCD_HIP(ctx, hipGetLastError());
   PYCD_HIP(ctx, hipEventRecord(after_sf, s));
-  // the real-space term has a kernel of its own (timed) only ahead of the
-  // 256 x 256-tile contraction; elsewhere it is in the epilogue
-  real_apart = precision == PYCD_PREC_BF16X3 && bvar == 4;
   const int tiles = nb * (nb + 1) / 2;
-  if (precision == PYCD_PREC_F32)
-    table_mfma_f32<<<tiles, 256, 0, s>>>(y32.ptr, n, Kp, pos, geo, es, out,
-                                         pairs);
+  if (precision == PYCD_PREC_F32 && tile == 64)
+    table_mfma_f32<2><<<tiles, 256, 0, s>>>(y32.ptr, n, Kp, es, out);
+  else if (precision == PYCD_PREC_F32)
+    table_mfma_f32<4><<<tiles, 256, 0, s>>>(y32.ptr, n, Kp, es, out);
   else if (bvar == 3)
     table_mfma_bf16x3_2stage<<<tiles, 256, 0, s>>>(yhi.ptr, ylo.ptr, n, Kp,
-                                                   pos, geo, es, out, pairs);
+                                                   es, out);
   else if (bvar == 4) {
-    const int nb1 = (n + kMTile - 1) / kMTile;
-    PYCD_HIP(ctx, hipEventRecord(real[0], s));
-    table_real_part<<<nb1 * (nb1 + 1) / 2, 256, 0, s>>>(pos, n, geo, es, out,
-                                                        pairs);
-    PYCD_HIP(ctx, hipGetLastError());
-    PYCD_HIP(ctx, hipEventRecord(real[1], s));
     // whole rounds of 256 x 256 tiles (one workgroup per CU), the rest as
     // pairs of 128 x 128 tiles; fewer tiles than one round all go whole
     int dev_cus = 0;
@@ -806,12 +742,16 @@ int launch_table_mfma(pycd_ctx* ctx, int precision, const double* pos, int n,
     PYCD_HIP(ctx, hipStreamSynchronize(s));
   }
   else if (bslice == 32)
-    table_mfma_bf16x3<32><<<tiles, 256, 0, s>>>(yhi.ptr, ylo.ptr, n, Kp, pos,
-                                                geo, es, out, pairs);
+    table_mfma_bf16x3<32><<<tiles, 256, 0, s>>>(yhi.ptr, ylo.ptr, n, Kp,
+                                                es, out);
   else
-    table_mfma_bf16x3<64><<<tiles, 256, 0, s>>>(yhi.ptr, ylo.ptr, n, Kp, pos,
-                                                geo, es, out, pairs);
+    table_mfma_bf16x3<64><<<tiles, 256, 0, s>>>(yhi.ptr, ylo.ptr, n, Kp,
+                                                es, out);
   PYCD_HIP(ctx, hipGetLastError());
+  PYCD_HIP(ctx, hipEventRecord(real[0], s));
+  launch_finish(s, std::min(tile, kMTile), pos, n, geo, es, out, pairs);
+  PYCD_HIP(ctx, hipGetLastError());
+  PYCD_HIP(ctx, hipEventRecord(real[1], s));
   PYCD_HIP(ctx, hipStreamSynchronize(s));
   return PYCD_OK;
 }
