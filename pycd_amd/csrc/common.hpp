@@ -7,10 +7,134 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
 #include "../../include/pycd_hip.h"
+
+namespace pycd {
+
+// Memory that the one-shot calls (tables, neighbour lists, displacements)
+// of a context work in.  Device blocks are kept from call to call up to
+// kMaxKept bytes, oldest given back first, and a page-locked staging buffer
+// for small transfers is made with the context; both go with it.  A block
+// is free again only when the call that took it is done with the context's
+// stream, on which every call works, so that a later call's use is ordered
+// after it; any number of threads may take at once.  An allocation that
+// fails is tried again with nothing kept.
+// (hipFree of a block of 240 MB takes 0.27 ms, hipMalloc 0.04, and copies of
+// pageable host memory 0.02-0.09 each: the 12000-site BF16x3 table 5.65 ->
+// 4.70 ms, the 6144-site FP32 one 2.20 -> 1.83, the 120-site FP64 one 262 ->
+// 177 us.)
+class Workspace {
+ public:
+  static constexpr size_t kMaxKept = size_t(512) << 20;
+  static constexpr int kMaxBlocks = 32;
+  static constexpr size_t kStaging = size_t(2) << 20;
+  // Device blocks are for work on `stream`.
+  hipError_t open(hipStream_t stream) {
+    stream_ = stream;
+    return hipHostMalloc(&staging_, kStaging, hipHostMallocDefault);
+  }
+  void close() {
+    clear();
+    if (staging_) (void)hipHostFree(staging_);
+    staging_ = nullptr;
+  }
+  // The smallest kept block of at least `bytes` and at most twice that,
+  // else a new one; *got: its size.
+  hipError_t take(size_t bytes, void** out, size_t* got) {
+    const size_t need = (bytes + 4095) & ~size_t(4095);
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      int best = -1;
+      for (int k = 0; k < n_; ++k)
+        if (kept_[k].bytes >= need && kept_[k].bytes / 2 <= need &&
+            (best < 0 || kept_[k].bytes < kept_[best].bytes))
+          best = k;
+      if (best >= 0) {
+        const Block b = remove(best);
+        *out = b.ptr;
+        *got = b.bytes;
+        return hipSuccess;
+      }
+    }
+    hipError_t e = hipMalloc(out, need);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      clear();
+      e = hipMalloc(out, need);
+    }
+    *got = e == hipSuccess ? need : 0;
+    return e;
+  }
+  void give(void* p, size_t bytes) {
+    bool kept = false;
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      if (bytes <= kMaxKept && n_ < kMaxBlocks) {
+        kept_[n_++] = {p, bytes};
+        held_ += bytes;
+        kept = true;
+      }
+    }
+    if (!kept) release(p);
+    while (release_oldest(kMaxKept)) {
+    }
+  }
+  void clear() {
+    while (release_oldest(0)) {
+    }
+  }
+  // The staging buffer, or NULL while another call has it.
+  void* take_staging() {
+    std::lock_guard<std::mutex> lock(mu_);
+    if (staging_busy_) return nullptr;
+    staging_busy_ = true;
+    return staging_;
+  }
+  void give_staging() {
+    std::lock_guard<std::mutex> lock(mu_);
+    staging_busy_ = false;
+  }
+
+ private:
+  struct Block {
+    void* ptr;
+    size_t bytes;
+  };
+  Block remove(int k) {  // the lock held
+    const Block b = kept_[k];
+    held_ -= b.bytes;
+    --n_;
+    for (; k < n_; ++k) kept_[k] = kept_[k + 1];
+    return b;
+  }
+  bool release_oldest(size_t above) {
+    void* p = nullptr;
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      if (n_ == 0 || held_ <= above) return false;
+      p = remove(0).ptr;
+    }
+    release(p);
+    return true;
+  }
+  void release(void* p) {
+    (void)hipStreamSynchronize(stream_);
+    (void)hipFree(p);
+  }
+  std::mutex mu_;
+  hipStream_t stream_ = nullptr;
+  Block kept_[kMaxBlocks];  // oldest first
+  int n_ = 0;
+  size_t held_ = 0;
+  void* staging_ = nullptr;
+  bool staging_busy_ = false;
+};
+
+}  // namespace pycd
 
 struct pycd_ctx {
   int device = 0;
@@ -23,6 +147,7 @@ struct pycd_ctx {
   double* static_scratch = nullptr;
   // table kernel variant per PYCD_PREC_* (0: the default choice)
   int table_variant[3] = {0, 0, 0};
+  pycd::Workspace work;
 };
 
 namespace pycd {
@@ -83,6 +208,97 @@ struct DevBuf {
   }
 };
 
+// Device memory of one call, from the context's workspace.  On the way out
+// of a call that failed the stream may still hold work on it; the next user
+// works on the same stream.
+template <typename T>
+struct WorkBuf {
+  T* ptr = nullptr;
+  WorkBuf() = default;
+  WorkBuf(const WorkBuf&) = delete;
+  WorkBuf& operator=(const WorkBuf&) = delete;
+  ~WorkBuf() {
+    if (ptr) work_->give(ptr, bytes_);
+  }
+  // (once per buffer)
+  hipError_t alloc(pycd_ctx* ctx, size_t n) {
+    if (n == 0) return hipSuccess;
+    work_ = &ctx->work;
+    void* p = nullptr;
+    const hipError_t e = work_->take(n * sizeof(T), &p, &bytes_);
+    if (e == hipSuccess) ptr = static_cast<T*>(p);
+    return e;
+  }
+
+ private:
+  Workspace* work_ = nullptr;
+  size_t bytes_ = 0;
+};
+
+// The context's staging buffer for one call: host data of a few small
+// copies side by side.  put()/get() return false when it does not fit (or
+// another call has the buffer); the caller then copies from its own memory.
+// Results arrive at finish(), after the stream is done.
+class Staging {
+ public:
+  explicit Staging(pycd_ctx* ctx)
+      : ctx_(ctx), base_(static_cast<char*>(ctx->work.take_staging())) {}
+  ~Staging() {
+    if (!base_) return;
+    // (no copy of a call that failed is left on the buffer)
+    if (pending_) (void)hipStreamSynchronize(ctx_->stream);
+    ctx_->work.give_staging();
+  }
+  Staging(const Staging&) = delete;
+  Staging& operator=(const Staging&) = delete;
+  bool put(void* dst, const void* src, size_t bytes, hipError_t* e) {
+    char* at = room(bytes);
+    if (!at) return false;
+    std::memcpy(at, src, bytes);
+    pending_ = true;
+    *e = hipMemcpyAsync(dst, at, bytes, hipMemcpyHostToDevice, ctx_->stream);
+    return true;
+  }
+  bool get(void* dst, const void* src, size_t bytes, hipError_t* e) {
+    char* at = n_results_ < kResults ? room(bytes) : nullptr;
+    if (!at) return false;
+    pending_ = true;
+    *e = hipMemcpyAsync(at, src, bytes, hipMemcpyDeviceToHost, ctx_->stream);
+    results_[n_results_++] = {dst, at, bytes};
+    return true;
+  }
+  hipError_t finish() {
+    const hipError_t e = hipStreamSynchronize(ctx_->stream);
+    pending_ = false;
+    if (e == hipSuccess)
+      for (int k = 0; k < n_results_; ++k)
+        std::memcpy(results_[k].dst, results_[k].src, results_[k].bytes);
+    n_results_ = 0;
+    return e;
+  }
+
+ private:
+  struct Result {
+    void* dst;
+    const char* src;
+    size_t bytes;
+  };
+  char* room(size_t bytes) {
+    const size_t need = (bytes + 255) & ~size_t(255);
+    if (!base_ || need > Workspace::kStaging - used_) return nullptr;
+    char* at = base_ + used_;
+    used_ += need;
+    return at;
+  }
+  pycd_ctx* ctx_;
+  char* base_;
+  size_t used_ = 0;
+  bool pending_ = false;
+  static constexpr int kResults = 4;
+  Result results_[kResults];
+  int n_results_ = 0;
+};
+
 // Copies `n` elements from a host-or-device pointer into device memory.
 template <typename T>
 hipError_t upload(T* dst, const T* src, size_t n, hipStream_t st) {
@@ -90,6 +306,17 @@ hipError_t upload(T* dst, const T* src, size_t n, hipStream_t st) {
   hipMemcpyKind kind =
       is_device_ptr(src) ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
   return hipMemcpyAsync(dst, src, n * sizeof(T), kind, st);
+}
+
+// Copies `n` elements to the device, through the staging buffer where the
+// source is host memory that fits it.
+template <typename T>
+hipError_t stage_up(Staging& stage, T* dst, const T* src, size_t n,
+                    hipStream_t st) {
+  if (n == 0) return hipSuccess;
+  hipError_t e = hipSuccess;
+  if (!is_device_ptr(src) && stage.put(dst, src, n * sizeof(T), &e)) return e;
+  return upload(dst, src, n, st);
 }
 
 template <typename T>

@@ -26,6 +26,11 @@ extern "C" int pycd_ctx_create(int device, pycd_ctx** out) {
     delete ctx;
     return PYCD_ERR_HIP;
   }
+  if (ctx->work.open(ctx->stream) != hipSuccess) {
+    (void)hipStreamDestroy(ctx->stream);
+    delete ctx;
+    return PYCD_ERR_HIP;
+  }
   int khz = 0;
   if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) ==
           hipSuccess &&
@@ -41,6 +46,7 @@ extern "C" void pycd_ctx_destroy(pycd_ctx* ctx) {
     pycd::DeviceGuard g(ctx->device);
     if (ctx->stream) {
       (void)hipStreamSynchronize(ctx->stream);
+      ctx->work.close();
       (void)hipStreamDestroy(ctx->stream);
     }
   }

@@ -348,8 +348,8 @@ int launch_table(pycd_ctx* ctx, int precision, const double* pos, int n,
   const int pair = 2 * kSlice;
   const int Kp = std::max(pair, (2 * K + pair - 1) / pair * pair);
   const int n_pad = nb * tile;
-  DevBuf<double> Y;
-  PYCD_HIP(ctx, Y.alloc(size_t(n_pad) * Kp));
+  WorkBuf<double> Y;
+  PYCD_HIP(ctx, Y.alloc(ctx, size_t(n_pad) * Kp));
   structure_factor_f64<<<dim3((Kp - K + 255) / 256,
                               (n_pad + kSfRows - 1) / kSfRows),
                          256, 0, s>>>(pos, n, n_pad, kv, sw, K, Kp, Y.ptr);
@@ -359,8 +359,8 @@ int launch_table(pycd_ctx* ctx, int precision, const double* pos, int n,
   const int want = k_parts(n, Kp);
   const int chunk = (Kp / pair + want - 1) / want * pair;
   const int parts = (Kp + chunk - 1) / chunk;
-  DevBuf<double> P;
-  if (parts > 1) PYCD_HIP(ctx, P.alloc(size_t(parts) * n * n));
+  WorkBuf<double> P;
+  if (parts > 1) PYCD_HIP(ctx, P.alloc(ctx, size_t(parts) * n * n));
   double* sums = parts > 1 ? P.ptr : out;
   const dim3 grid(nb * (nb + 1) / 2, parts);
   if (v == 2)
@@ -377,8 +377,6 @@ int launch_table(pycd_ctx* ctx, int precision, const double* pos, int n,
   launch_finish(s, tile, pos, n, geo, es, out, pairs);
   PYCD_HIP(ctx, hipEventRecord(real[1], s));
   PYCD_HIP(ctx, hipGetLastError());
-  // Y is released when this returns; the stream must have consumed it.
-  PYCD_HIP(ctx, hipStreamSynchronize(s));
   return PYCD_OK;
 }
 
@@ -481,25 +479,22 @@ extern "C" int pycd_pair_table(pycd_ctx* ctx, const double* pos, int64_t n,
                     (1.0 + 1e-9) + 1e-9;
   }
 
-  DevBuf<double> d_pos, d_kv, d_sw, d_A;
-  DevBuf<unsigned long long> d_pairs;
-  PYCD_HIP(ctx, d_pos.alloc(size_t(N) * 3));
-  PYCD_HIP(ctx, d_kv.alloc(size_t(K) * 3 + 3));
-  PYCD_HIP(ctx, d_sw.alloc(size_t(K) + 1));
-  PYCD_HIP(ctx, d_pairs.alloc(1));
+  WorkBuf<double> d_pos, d_kv, d_sw, d_A;
+  WorkBuf<unsigned long long> d_pairs;
+  PYCD_HIP(ctx, d_pos.alloc(ctx, size_t(N) * 3));
+  PYCD_HIP(ctx, d_kv.alloc(ctx, size_t(K) * 3 + 3));
+  PYCD_HIP(ctx, d_sw.alloc(ctx, size_t(K) + 1));
+  PYCD_HIP(ctx, d_pairs.alloc(ctx, 1));
   hipStream_t s = ctx->stream;
-  PYCD_HIP(ctx, upload(d_pos.ptr, pos, size_t(N) * 3, s));
-  if (K > 0) {
-    PYCD_HIP(ctx, hipMemcpyAsync(d_kv.ptr, st.kv.data(), sizeof(double) * 3 * K,
-                                 hipMemcpyHostToDevice, s));
-    PYCD_HIP(ctx, hipMemcpyAsync(d_sw.ptr, st.sw.data(), sizeof(double) * K,
-                                 hipMemcpyHostToDevice, s));
-  }
+  Staging stage(ctx);
+  PYCD_HIP(ctx, stage_up(stage, d_pos.ptr, pos, size_t(N) * 3, s));
+  PYCD_HIP(ctx, stage_up(stage, d_kv.ptr, st.kv.data(), 3 * size_t(K), s));
+  PYCD_HIP(ctx, stage_up(stage, d_sw.ptr, st.sw.data(), size_t(K), s));
   PYCD_HIP(ctx, hipMemsetAsync(d_pairs.ptr, 0, sizeof(unsigned long long), s));
   double* out = table_out;
   const bool out_dev = is_device_ptr(table_out);
   if (!out_dev) {
-    PYCD_HIP(ctx, d_A.alloc(size_t(N) * N));
+    PYCD_HIP(ctx, d_A.alloc(ctx, size_t(N) * N));
     out = d_A.ptr;
   }
 
@@ -516,13 +511,19 @@ extern "C" int pycd_pair_table(pycd_ctx* ctx, const double* pos, int64_t n,
     return rc;
   }
   PYCD_HIP(ctx, hipEventRecord(ev[2], s));
-  if (!out_dev)
-    PYCD_HIP(ctx, hipMemcpyAsync(table_out, out, sizeof(double) * N * size_t(N),
-                                 hipMemcpyDeviceToHost, s));
   unsigned long long pairs = 0;
-  PYCD_HIP(ctx, hipMemcpyAsync(&pairs, d_pairs.ptr, sizeof(pairs),
-                               hipMemcpyDeviceToHost, s));
-  PYCD_HIP(ctx, hipStreamSynchronize(s));
+  hipError_t e = hipSuccess;
+  if (!stage.get(&pairs, d_pairs.ptr, sizeof(pairs), &e))
+    e = hipMemcpyAsync(&pairs, d_pairs.ptr, sizeof(pairs),
+                       hipMemcpyDeviceToHost, s);
+  PYCD_HIP(ctx, e);
+  if (!out_dev) {
+    const size_t bytes = sizeof(double) * N * size_t(N);
+    if (!stage.get(table_out, out, bytes, &e))
+      e = hipMemcpyAsync(table_out, out, bytes, hipMemcpyDeviceToHost, s);
+    PYCD_HIP(ctx, e);
+  }
+  PYCD_HIP(ctx, stage.finish());
   float ms_sf = 0, ms_rest = 0, ms_real = 0;
   (void)hipEventElapsedTime(&ms_sf, ev[0], ev[1]);
   (void)hipEventElapsedTime(&ms_rest, ev[1], ev[2]);

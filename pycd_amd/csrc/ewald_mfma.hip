@@ -684,16 +684,18 @@ int launch_table_mfma(pycd_ctx* ctx, int precision, const double* pos, int n,
   const int nb = (n + tile - 1) / tile;
   const int n_pad = nb * tile;
   const size_t elems = size_t(n_pad) * Kp;
-  DevBuf<float> y32;
-  DevBuf<__bf16> yhi, ylo;
+  WorkBuf<float> y32;
+  WorkBuf<__bf16> yhi, ylo;
+  WorkBuf<int2> d_sub;
+  std::vector<int2> sub;
   const dim3 sf_grid((Kp - K + 255) / 256, (n_pad + kLowRows - 1) / kLowRows);
   if (precision == PYCD_PREC_F32) {
-    PYCD_HIP(ctx, y32.alloc(elems));
+    PYCD_HIP(ctx, y32.alloc(ctx, elems));
     structure_factor_lowp<PYCD_PREC_F32><<<sf_grid, 256, 0, s>>>(
         pos, n, n_pad, kv, sw, K, Kp, y32.ptr, nullptr, nullptr);
   } else {
-    PYCD_HIP(ctx, yhi.alloc(elems));
-    PYCD_HIP(ctx, ylo.alloc(elems));
+    PYCD_HIP(ctx, yhi.alloc(ctx, elems));
+    PYCD_HIP(ctx, ylo.alloc(ctx, elems));
     structure_factor_lowp<PYCD_PREC_BF16X3><<<sf_grid, 256, 0, s>>>(
         pos, n, n_pad, kv, sw, K, Kp, nullptr, yhi.ptr, ylo.ptr);
   }
@@ -716,7 +718,6 @@ int launch_table_mfma(pycd_ctx* ctx, int precision, const double* pos, int n,
                                         ctx->device));
     const int round = std::max(dev_cus, 1);
     const int main_tiles = tiles >= round ? (tiles / round) * round : tiles;
-    std::vector<int2> sub;
     for (int w = main_tiles; w < tiles; ++w) {
       int bi = 0, bj = 0;
       tile_coords_upper_at(n, kMTile2, w, bi, bj);
@@ -727,9 +728,8 @@ int launch_table_mfma(pycd_ctx* ctx, int precision, const double* pos, int n,
           sub.push_back(make_int2(si, sj));
         }
     }
-    DevBuf<int2> d_sub;
     if (!sub.empty()) {
-      PYCD_HIP(ctx, d_sub.alloc(sub.size()));
+      PYCD_HIP(ctx, d_sub.alloc(ctx, sub.size()));
       PYCD_HIP(ctx, hipMemcpyAsync(d_sub.ptr, sub.data(),
                                    sizeof(int2) * sub.size(),
                                    hipMemcpyHostToDevice, s));
@@ -738,8 +738,6 @@ int launch_table_mfma(pycd_ctx* ctx, int precision, const double* pos, int n,
     table_mfma_bf16x3_256<<<grid, 512, 0, s>>>(yhi.ptr, ylo.ptr, n, Kp, es,
                                                out, main_tiles, d_sub.ptr,
                                                int(sub.size()));
-    PYCD_HIP(ctx, hipGetLastError());
-    PYCD_HIP(ctx, hipStreamSynchronize(s));
   }
   else if (bslice == 32)
     table_mfma_bf16x3<32><<<tiles, 256, 0, s>>>(yhi.ptr, ylo.ptr, n, Kp,

@@ -81,18 +81,18 @@ extern "C" int pycd_msd(pycd_ctx* ctx, const double* pos, int64_t n_traj,
   hipStream_t st = ctx->stream;
   const size_t npos = size_t(n_traj) * n_path * n_carriers * 3;
   const size_t nsd = size_t(n_traj) * n_lags * n_carriers;
-  DevBuf<double> dpos, dsd;
+  WorkBuf<double> dpos, dsd;
   const double* p = pos;
   double* o = sd;
   if (!is_device_ptr(pos)) {
-    PYCD_HIP(ctx, dpos.alloc(npos));
+    PYCD_HIP(ctx, dpos.alloc(ctx, npos));
     PYCD_HIP(ctx, hipMemcpyAsync(dpos.ptr, pos, 8 * npos, hipMemcpyHostToDevice,
                                  st));
     p = dpos.ptr;
   }
   const bool out_dev = is_device_ptr(sd);
   if (!out_dev) {
-    PYCD_HIP(ctx, dsd.alloc(nsd));
+    PYCD_HIP(ctx, dsd.alloc(ctx, nsd));
     o = dsd.ptr;
   }
   // origin segments shared by `parts` workgroups, so that about 2048 (8 per
@@ -108,8 +108,8 @@ extern "C" int pycd_msd(pycd_ctx* ctx, const double* pos, int64_t n_traj,
   const int64_t units = paths * parts;
   if (units > (int64_t(1) << 31) - 1)
     return fail(ctx, PYCD_ERR_ARG, "MSD problem too large for one launch");
-  DevBuf<double> sums;
-  if (parts > 1) PYCD_HIP(ctx, sums.alloc(size_t(units) * n_lags));
+  WorkBuf<double> sums;
+  if (parts > 1) PYCD_HIP(ctx, sums.alloc(ctx, size_t(units) * n_lags));
   auto go = [&](auto* kernel) {
     kernel<<<unsigned(units), kMsdThreads, 0, st>>>(
         p, units, n_path, int(n_carriers), n_lags, int(parts), sums.ptr, o);

@@ -200,13 +200,13 @@ extern "C" int pycd_min_image_vectors(pycd_ctx* ctx, const double* pos,
   hipStream_t st = ctx->stream;
   MicGeometry g;
   fill_mic_geometry(cell, pbc, g);
-  DevBuf<double> dpos, dout;
-  PYCD_HIP(ctx, dpos.alloc(size_t(n) * 3));
+  WorkBuf<double> dpos, dout;
+  PYCD_HIP(ctx, dpos.alloc(ctx, size_t(n) * 3));
   PYCD_HIP(ctx, upload(dpos.ptr, pos, size_t(n) * 3, st));
   double* o = out;
   const bool out_dev = is_device_ptr(out);
   if (!out_dev) {
-    PYCD_HIP(ctx, dout.alloc(size_t(n) * n * 3));
+    PYCD_HIP(ctx, dout.alloc(ctx, size_t(n) * n * 3));
     o = dout.ptr;
   }
   const int64_t total = n * n;
@@ -259,16 +259,16 @@ extern "C" int pycd_hop_neighbors(pycd_ctx* ctx, const double* pos, int64_t n,
                    (1.0 + 1e-9) + 1e-6;
   }
   const size_t nout = size_t(n_centers) * n_shells * max_per_shell;
-  DevBuf<double> dpos, dvec, dfrac;
-  DevBuf<int64_t> dc, dt;
-  DevBuf<int32_t> dcount, dindex;
-  PYCD_HIP(ctx, dpos.alloc(size_t(n) * 3));
-  PYCD_HIP(ctx, dc.alloc(n_centers));
-  PYCD_HIP(ctx, dt.alloc(n_targets));
-  PYCD_HIP(ctx, dfrac.alloc(3 * size_t(n_targets)));
-  PYCD_HIP(ctx, dcount.alloc(size_t(n_centers) * n_shells));
-  PYCD_HIP(ctx, dindex.alloc(nout));
-  PYCD_HIP(ctx, dvec.alloc(nout * 3));
+  WorkBuf<double> dpos, dvec, dfrac;
+  WorkBuf<int64_t> dc, dt;
+  WorkBuf<int32_t> dcount, dindex;
+  PYCD_HIP(ctx, dpos.alloc(ctx, size_t(n) * 3));
+  PYCD_HIP(ctx, dc.alloc(ctx, n_centers));
+  PYCD_HIP(ctx, dt.alloc(ctx, n_targets));
+  PYCD_HIP(ctx, dfrac.alloc(ctx, 3 * size_t(n_targets)));
+  PYCD_HIP(ctx, dcount.alloc(ctx, size_t(n_centers) * n_shells));
+  PYCD_HIP(ctx, dindex.alloc(ctx, nout));
+  PYCD_HIP(ctx, dvec.alloc(ctx, nout * 3));
   PYCD_HIP(ctx, upload(dpos.ptr, pos, size_t(n) * 3, st));
   PYCD_HIP(ctx, hipMemcpyAsync(dc.ptr, centers, 8 * n_centers,
                                hipMemcpyHostToDevice, st));
