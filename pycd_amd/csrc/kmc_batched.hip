@@ -41,10 +41,15 @@
 // by rows of 16 lanes, a lane taking every 16th carrier, which leaves each
 // sum in the row that a lane permute hands to its process.  What bounds it:
 // alone on a SIMD, the latencies of a hop (LDS, scan, one round of gathers,
-// row sums); four to a SIMD, the issue of its ~380 vector instructions.
+// row sums); four to a SIMD, the issue of its ~350 vector instructions
+// and the ~170 cache lines that its gathers touch, about one per cycle of a
+// CU's vector cache.
 // With sites, psi and process records in LDS instead (442 vector, 244
-// scalar, 44 LDS instructions, now 377, 108, 21) a hop took 2.26 us alone
-// and 3.09 among four at up to 16 carriers; now 1.18 and 2.01.  The loop is
+// scalar, 44 LDS instructions, now 351, 106, 21) a hop took 2.26 us alone
+// and 3.09 among four at up to 16 carriers; now 1.10 and 2.0.  (The checks
+// between hops behind one counter, and the entries of several carriers in
+// flight where psi is formed anew, are 0.08 of that; FP64 rates, which form
+// it every 64 hops, 1.86 -> 1.74 at two wavefronts a SIMD.)  The loop is
 // instantiated per processes-per-lane count: with one instance for up to 4
 // the large trajectories' register spills made 4096 mixed trajectories 8%
 // slower.
@@ -265,18 +270,41 @@ __device__ inline double pair_entry(const Tab<TT>& t, const GeoPk& p,
   return double(t.at(t.row(a >> 24), rel_col(a, b, p)));
 }
 
-// sum_c q A[x, occ[c]].
-template <typename TT>
-__device__ inline double psi_from_table(const Tab<TT>& t, const GeoPk& gp,
-                                        double q, int nc, uint32_t x,
-                                        const uint32_t* occ) {
-  const RowKey key = row_key(x, gp);
-  const uint32_t row = t.row(key.sub);
-  double acc = 0.0;
-#pragma unroll 4
-  for (int c2 = 0; c2 < nc; ++c2)
-    acc = fma(q, double(t.at(row, rel_col(key, occ[c2], gp))), acc);
-  return acc;
+// sum_c q A[x, occ[c]] of a lane's kN rows x, over the carriers in order;
+// the entries of 4 carriers (2 from 4 rows on) are loaded before the first
+// is used.
+template <typename TT, int kN>
+__device__ __forceinline__ void psi_from_table(const Tab<TT>& t,
+                                               const GeoPk& gp, double q,
+                                               int nc,
+                                               const uint32_t (&x)[kN],
+                                               const uint32_t* occ,
+                                               double (&acc)[kN]) {
+  constexpr int kU = kN < 4 ? 4 : 2;
+#pragma unroll
+  for (int i = 0; i < kN; ++i) acc[i] = 0.0;
+  int c2 = 0;
+#pragma unroll 1
+  for (; c2 + kU <= nc; c2 += kU) {
+    TT v[kN][kU];
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+      const RowKey key = row_key(x[i], gp);
+      const uint32_t row = t.row(key.sub);
+#pragma unroll
+      for (int u = 0; u < kU; ++u)
+        v[i][u] = t.at(row, rel_col(key, occ[c2 + u], gp));
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+#pragma unroll
+      for (int i = 0; i < kN; ++i) acc[i] = fma(q, double(v[i][u]), acc[i]);
+  }
+#pragma unroll 1
+  for (; c2 < nc; ++c2)
+#pragma unroll
+    for (int i = 0; i < kN; ++i)
+      acc[i] = fma(q, pair_entry<TT>(t, gp, x[i], occ[c2]), acc[i]);
 }
 
 // Per (sublattice, slot) of the trajectory's family: the static part of a
@@ -748,7 +776,7 @@ __device__ __forceinline__ void kmc_batched_body(const BatchArgs& a) {
       if (a.slice_hops > 0) h = min(h, a.slice_hops - slice_done);
       return h;
     };
-    uint32_t left = 0;
+    uint32_t left = 0, todo = 0;
     // The hops of this launch, kP processes per lane (per <= kP), and the
     // state written back: outputs and resumable state, at the trajectory's
     // end, at the slice's, or at a hop boundary when it is handed over.
@@ -776,10 +804,15 @@ __device__ __forceinline__ void kmc_batched_body(const BatchArgs& a) {
       // psi at the site of carrier `lane`
       double psi_s = resume && lane < nc ? spsi[lane * zp] : 0.0;
       auto psi_anew = [&]() __attribute__((always_inline)) {
+        uint32_t x[kP + 1];
+        double v[kP + 1];
 #pragma unroll
-        for (int i = 0; i < kP; ++i)
-          psi[i] = psi_from_table<TT>(tab, gp, q, nc, px[i], occ);
-        psi_s = psi_from_table<TT>(tab, gp, q, nc, sx, occ);
+        for (int i = 0; i < kP; ++i) x[i] = px[i];
+        x[kP] = sx;
+        psi_from_table<TT>(tab, gp, q, nc, x, occ, v);
+#pragma unroll
+        for (int i = 0; i < kP; ++i) psi[i] = v[i];
+        psi_s = v[kP];
       };
       if (!resume) psi_anew();
       // lane fc + 16 r forms row r of the fresh sums with the carriers
@@ -800,32 +833,40 @@ __device__ __forceinline__ void kmc_batched_body(const BatchArgs& a) {
         const int fc_h = lane_h & 15;
 #pragma unroll
         for (int i = 0; i < kP; ++i) asm volatile("" : "+v"(pd[i]));
-        if (left == 0) {
-          asm volatile("");  // the 64-bit budget only when the count runs out
-          const int64_t b = budget();
-          if (b <= 0) {
-            finished = td.max_hops > 0 && hops >= td.max_hops;
-            break;
+        // Whatever happens between hops only now and then, at a check: the
+        // budget, pacing and hand-over every 64 hops, psi formed anew every
+        // `refresh`; `todo` hops follow without one.
+        if (todo == 0) {
+          if (left == 0) {
+            const int64_t b = budget();
+            if (b <= 0) {
+              finished = td.max_hops > 0 && hops >= td.max_hops;
+              break;
+            }
+            left = uint32_t(min<int64_t>(b, INT32_MAX));
           }
-          left = uint32_t(min<int64_t>(b, INT32_MAX));
-        }
-        --left;
-        ++slice_done;
-        if (a.progress && (uint32_t(hops) & 63u) == 0) {
-          const int busy = pace(a.progress, pslot, left + 1, lane_h);
-          if (!stolen && busy >= a.hand_busy && left >= kHandMinHops) {
-            if (lane_h == 0) box = claim_mailbox(hand_words(a.progress));
-            box = uni(__shfl(box, 0, 64));
-            if (box >= 0) break;  // hand over at this hop boundary
+          if (a.progress && (uint32_t(hops) & 63u) == 0) {
+            const int busy = pace(a.progress, pslot, left, lane_h);
+            if (!stolen && busy >= a.hand_busy && left > kHandMinHops) {
+              if (lane_h == 0) box = claim_mailbox(hand_words(a.progress));
+              box = uni(__shfl(box, 0, 64));
+              if (box >= 0) break;  // hand over at this hop boundary
+            }
           }
+          if (hops == next_refresh) {
+            next_refresh += a.refresh;
+            // bound the rounding carried by the incremental updates
+            occ[lane_h] = sx;
+            __syncthreads();
+            psi_anew();
+          }
+          todo = left;
+          if (a.progress) todo = min(todo, 64u - (uint32_t(hops) & 63u));
+          todo = uint32_t(min<int64_t>(todo, next_refresh - hops));
+          left -= todo;
+          slice_done += todo;
         }
-        if (hops == next_refresh) {
-          next_refresh += a.refresh;
-          // bound the rounding carried by the incremental updates
-          occ[lane_h] = sx;
-          __syncthreads();
-          psi_anew();
-        }
+        --todo;
         psis[lane_h] = psi_s;
         // ---- two uniforms, as random.random() draws them
         if (c_next >= c_n && mti <= kMtN - 4) {
