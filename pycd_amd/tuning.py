@@ -37,13 +37,17 @@ def lpt_order(trajs, fams):
 
 def autotune_waves(batch, trajs, occs, words, order, candidates=(2, 4, 6, 8,
                                                                   12, 16),
-                   sample=4096, hops=2000, log=None):
+                   sample=4096, hops=8000, log=None):
     """Time `hops`-hop runs of the first `sample` queued trajectories.
 
     The sample must hold several trajectories per wavefront at the largest
     candidate, or every candidate past n_traj / CUs times one trajectory
     per wave and the comparison says nothing; the default takes the whole
-    batch of the benchmark workload, each cut to `hops` hops."""
+    batch of the benchmark workload, each cut to `hops` hops.
+
+    Runs of 2000 hops rank the candidates by their start and tail: 9.0e8
+    hops/s at 8 waves per CU, 8.0e8 at 16.  From 8000 on the order is that of
+    long runs: 0.96e9 and 1.10e9 (32000 hops: 0.98e9 and 1.15e9)."""
     sub = [int(i) for i in order[:sample]]
     sub_trajs = []
     for i in sub:
