@@ -97,6 +97,11 @@ __device__ inline int msd_row(int r) { return r + (r >> 2); }
 // block's last lag below the pass's span; lim: P - pass0 - T0, the relative
 // origin bound; base: window row of relative origin 0's lag-0 row.  It reads
 // the rows below base + rb + lo + kMsdRing and the origins below rb + 2.
+// kExec: the masked steps under exec masks, which skip what no lane needs
+// (one group per wavefront: 500 lags of up to 2001 rows 16.4 -> 14.8 ms),
+// else by selects (several groups, some of whose lanes nearly always have
+// work: 100 lags 3.2 ms, 0.1 more under exec masks).
+template <bool kExec>
 __device__ inline void msd_run(const double* L, int ra, int rb, int lo,
                                int hi, int lim, int base, double* acc) {
   constexpr int kR = kMsdRing;
@@ -169,7 +174,7 @@ __device__ inline void msd_run(const double* L, int ra, int rb, int lo,
     turned();
   }
   // masked steps: pair i of step j counts while lo + i < lim - o - j, for
-  // each pair a first part of a group's lanes (an exec mask, not a select)
+  // each pair a first part of a group's lanes
   auto masked_step = [&](int j) {
     const int c = lim - (o + j);
 #pragma unroll
@@ -177,7 +182,10 @@ __device__ inline void msd_run(const double* L, int ra, int rb, int lo,
       const int q = (j + i) % kR;
       const double dx = wx[q] - ox[j & 1], dy = wy[q] - oy[j & 1],
                    dz = wz[q] - oz[j & 1];
-      if (lo + i < c) s[i] = fma(dz, dz, fma(dy, dy, fma(dx, dx, s[i])));
+      if (lo + i < c) {
+        if constexpr (kExec) asm volatile("");  // else selects
+        s[i] = fma(dz, dz, fma(dy, dy, fma(dx, dx, s[i])));
+      }
     }
     load(j);
   };
@@ -282,7 +290,7 @@ __device__ __forceinline__ void msd_unit(
       for (int b = 0; b < kMsdBlocks; ++b) {
         const int ra = max(a - boff, 0), rb = min(e - boff, n[b]);
         if (ra < rb)
-          msd_run(L, ra, rb, kBlock * b + kMsdL * lane,
+          msd_run<kQ == 64>(L, ra, rb, kBlock * b + kMsdL * lane,
                   min(span, kBlock * (b + 1)) - 1, lim, wofs, acc[b]);
         boff += (n[b] + 3) & ~3;
       }
