@@ -76,10 +76,9 @@ typedef struct {
   int32_t precision;     /* PYCD_PREC_*                                     */
   double volume;         /* |T0 . (T1 x T2)|                                */
   double ms_sf;          /* structure-factor kernel time                    */
-  double ms_real;        /* time of the real-space kernel beside the FP64   */
-                         /* and the BF16x3 256 x 256-tile contractions      */
-                         /* (included in ms_recip); 0 where the term is in  */
-                         /* the table kernel's epilogue                     */
+  double ms_real;        /* time of the kernel that adds the real-space and */
+                         /* self terms and writes the mirror (included in   */
+                         /* ms_recip)                                       */
   double ms_recip;       /* reciprocal contraction + epilogue kernel time   */
   double ms_total;       /* device time of the whole table                  */
 } pycd_ewald_report;
