@@ -75,41 +75,31 @@ struct ShellWindows {
   double far[3];
 };
 
-// Fractional coordinates of the targets, one array per axis.
-__global__ void __launch_bounds__(256)
-target_fractions(const double* __restrict__ pos,
-                 const int64_t* __restrict__ targets, int64_t n_targets,
-                 MicGeometry g, double* __restrict__ frac) {
-  const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (j >= n_targets) return;
-  const double* p = pos + 3 * targets[j];
-#pragma unroll
-  for (int k = 0; k < 3; ++k)
-    frac[k * n_targets + j] =
-        p[0] * g.inv[k] + p[1] * g.inv[3 + k] + p[2] * g.inv[6 + k];
-}
-
 // One wavefront per kC centres; lanes sweep the targets 64 at a time in
 // ascending order, and a ballot per shell gives each hit its rank.
 //
-// Bound by FP64 instructions per pair.  A pair whose wrapped fractional
-// difference exceeds `far` on an axis is beyond every window: |f_k| <= |d|
-// times the length of column k of S^-1, no image has a smaller |f_k| than
-// the wrapped one, and the margin of `far` (1e-6) is above the rounding of f
-// for sites up to 1e9 cells away.  Only
-// the others form the minimum image (9 products for f, 9 for the vector, 7
-// for each of 12 images), and 64 targets that all fail cost a subtraction,
-// a wrap and a comparison per axis.  The centres of a wavefront share the
-// targets' loads.  6144 centres x 6144 targets, shells to 3.0 A: 276 us
-// with a minimum image per pair, 76 + 4 so.
+// Few centres: bound by the chain of a sweep's steps, so the positions are
+// loaded one step ahead and their indices two.  Many: by FP64 instructions
+// per pair.  A pair whose wrapped fractional difference exceeds `far` on an
+// axis is beyond every window: |f_k| <= |d| times the length of column k of
+// S^-1, no image has a smaller |f_k| than the wrapped one, and the margin of
+// `far` (1e-6) is above the rounding of f for sites up to 1e9 cells away.
+// Only the others form the minimum image (9 products for f, 9 for the
+// vector, 7 for each of 12 images); 64 targets that all fail cost their
+// fractional coordinates (9 products, shared by the wavefront's centres)
+// and per centre and axis a subtraction, a wrap and a comparison.  Shells
+// to 3.0 A, 6144 centres x 6144 targets: 259 us with a minimum image per
+// pair, 73 so; 768 x 768: 26 and 21 us.  (With the fractional coordinates
+// read from an array that a kernel ahead filled, the second launch cost a
+// call 30-40 us up to 6144 sites.)
 template <int kC>
 __global__ void __launch_bounds__(256)
 hop_neighbor_kernel(const double* __restrict__ pos,
                     const int64_t* __restrict__ centers, int64_t n_centers,
                     const int64_t* __restrict__ targets, int64_t n_targets,
-                    const double* __restrict__ frac, MicGeometry g,
-                    ShellWindows w, int max_per, int32_t* __restrict__ count,
-                    int32_t* __restrict__ index, double* __restrict__ vec) {
+                    MicGeometry g, ShellWindows w, int max_per,
+                    int32_t* __restrict__ count, int32_t* __restrict__ index,
+                    double* __restrict__ vec) {
   const int lane = threadIdx.x & 63;
   const int64_t c0 =
       (int64_t(blockIdx.x) * 4 +
@@ -135,12 +125,25 @@ hop_neighbor_kernel(const double* __restrict__ pos,
   // axes that do not wrap subtract rint(f) times 0
   const double wrap[3] = {g.pbc[0] ? 1.0 : 0.0, g.pbc[1] ? 1.0 : 0.0,
                           g.pbc[2] ? 1.0 : 0.0};
+  // lanes past the last target repeat the first and report nothing
+  double qn[3];
+  const int64_t t0 = targets[lane < n_targets ? lane : 0];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) qn[k] = pos[3 * t0 + k];
+  int64_t tn = targets[lane + 64 < n_targets ? lane + 64 : 0];
   for (int64_t j0 = 0; j0 < n_targets; j0 += 64) {
     const int64_t j = j0 + lane;
     const bool real = j < n_targets;
-    double f[3];
+    double q[3], f[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) f[k] = frac[k * n_targets + (real ? j : 0)];
+    for (int k = 0; k < 3; ++k) {
+      q[k] = qn[k];
+      qn[k] = pos[3 * tn + k];
+    }
+    tn = targets[j + 128 < n_targets ? j + 128 : 0];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      f[k] = q[0] * g.inv[k] + q[1] * g.inv[3 + k] + q[2] * g.inv[6 + k];
 #pragma unroll
     for (int u = 0; u < kC; ++u) {
       bool near = real;
@@ -152,11 +155,8 @@ hop_neighbor_kernel(const double* __restrict__ pos,
       if (__ballot(near) == 0ull) continue;
       double v[3] = {0.0, 0.0, 0.0};
       double r = -1.0;
-      if (near) {
-        const int64_t tj = targets[j];
-        r = mic_vec(pos[3 * tj] - px[u], pos[3 * tj + 1] - py[u],
-                    pos[3 * tj + 2] - pz[u], g, v);
-      }
+      if (near)
+        r = mic_vec(q[0] - px[u], q[1] - py[u], q[2] - pz[u], g, v);
 #pragma unroll
       for (int s = 0; s < kMaxShells; ++s) {
         if (s >= w.n) break;
@@ -259,13 +259,12 @@ extern "C" int pycd_hop_neighbors(pycd_ctx* ctx, const double* pos, int64_t n,
                    (1.0 + 1e-9) + 1e-6;
   }
   const size_t nout = size_t(n_centers) * n_shells * max_per_shell;
-  WorkBuf<double> dpos, dvec, dfrac;
+  WorkBuf<double> dpos, dvec;
   WorkBuf<int64_t> dc, dt;
   WorkBuf<int32_t> dcount, dindex;
   PYCD_HIP(ctx, dpos.alloc(ctx, size_t(n) * 3));
   PYCD_HIP(ctx, dc.alloc(ctx, n_centers));
   PYCD_HIP(ctx, dt.alloc(ctx, n_targets));
-  PYCD_HIP(ctx, dfrac.alloc(ctx, 3 * size_t(n_targets)));
   PYCD_HIP(ctx, dcount.alloc(ctx, size_t(n_centers) * n_shells));
   PYCD_HIP(ctx, dindex.alloc(ctx, nout));
   PYCD_HIP(ctx, dvec.alloc(ctx, nout * 3));
@@ -274,14 +273,22 @@ extern "C" int pycd_hop_neighbors(pycd_ctx* ctx, const double* pos, int64_t n,
                                hipMemcpyHostToDevice, st));
   PYCD_HIP(ctx, hipMemcpyAsync(dt.ptr, targets, 8 * n_targets,
                                hipMemcpyHostToDevice, st));
-  target_fractions<<<unsigned((n_targets + 255) / 256), 256, 0, st>>>(
-      dpos.ptr, dt.ptr, n_targets, g, dfrac.ptr);
-  PYCD_HIP(ctx, hipGetLastError());
-  constexpr int kC = 2;
-  hop_neighbor_kernel<kC>
-      <<<unsigned((n_centers + 4 * kC - 1) / (4 * kC)), 256, 0, st>>>(
-          dpos.ptr, dc.ptr, n_centers, dt.ptr, n_targets, dfrac.ptr, g, w,
-          max_per_shell, dcount.ptr, dindex.ptr, dvec.ptr);
+  // More centres per wavefront share more of each pair's work and leave
+  // fewer wavefronts: a call with 1, 2, 4 each takes 149, 159, - us at 768
+  // centres, 657, 657, 682 at 6144, 1029, 1003, 1015 at 9600, 2008, 1841,
+  // 1824 at 17280, 14.1, 10.7, 9.0 ms at 72000.
+  const auto launch = [&](auto kernel, int per_wave) {
+    const int64_t per_block = 4 * per_wave;
+    kernel<<<unsigned((n_centers + per_block - 1) / per_block), 256, 0, st>>>(
+        dpos.ptr, dc.ptr, n_centers, dt.ptr, n_targets, g, w, max_per_shell,
+        dcount.ptr, dindex.ptr, dvec.ptr);
+  };
+  if (n_centers < 6144)
+    launch(hop_neighbor_kernel<1>, 1);
+  else if (n_centers < 16384)
+    launch(hop_neighbor_kernel<2>, 2);
+  else
+    launch(hop_neighbor_kernel<4>, 4);
   PYCD_HIP(ctx, hipGetLastError());
   PYCD_HIP(ctx, hipMemcpyAsync(count, dcount.ptr,
                                4 * size_t(n_centers) * n_shells,

@@ -53,3 +53,28 @@ def test_lists_against_numpy(n, n_centers, pbc, windows):
             if len(hits):
                 assert np.max(np.abs(vec[c, s, :len(hits)]
                                      - v[c, hits])) < 1e-11
+
+
+@pytest.mark.parametrize("n_centers", [6143, 6145, 16383, 16384, 16387])
+def test_centres_per_wavefront(n_centers):
+    """The numbers of centres around which a wavefront takes one, two or
+    four of them, with remainders; sites serve as centres many times over.
+    Bound on the vectors as above."""
+    n, lo, hi = 70, [0.5, 0.0], [3.0, 2.0]
+    g = np.random.default_rng(n_centers)
+    pos = g.uniform(-0.5, 1.5, size=(n, 3)) @ CELL
+    centers = g.integers(0, n, size=n_centers)
+    targets = g.permutation(n)
+    count, index, vec = _native.hop_neighbors(
+        pos, centers, targets, CELL, [1, 1, 1], lo, hi, max_per=n)
+    v = _images(pos[targets][None] - pos[:, None], np.ones(3, dtype=bool))
+    r = np.sqrt((v * v).sum(-1))
+    for c in range(n):
+        rows = np.flatnonzero(centers == c)
+        for s in range(2):
+            hits = np.flatnonzero((lo[s] < r[c]) & (r[c] <= hi[s]))
+            assert (count[rows, s] == len(hits)).all()
+            assert (index[rows, s, :len(hits)] == hits).all()
+            if len(hits):
+                assert np.max(np.abs(vec[rows, s, :len(hits)]
+                                     - v[c, hits])) < 1e-11
