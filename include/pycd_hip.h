@@ -52,7 +52,11 @@ extern "C" {
 typedef struct pycd_ctx pycd_ctx;
 
 /* Context: device selection, stream, scratch.  (No reference counterpart:
- * PyCD has no device state.) */
+ * PyCD has no device state.)  A context holds 2 MiB of page-locked host
+ * memory, and keeps up to 512 MiB of device memory from one pycd_pair_table,
+ * pycd_hop_neighbors, pycd_min_image_vectors or pycd_msd call to the next.
+ * The kept memory goes to whatever else this library allocates on the device
+ * once that is full; to other allocators, with pycd_ctx_destroy. */
 int pycd_ctx_create(int device, pycd_ctx** out);
 void pycd_ctx_destroy(pycd_ctx* ctx);
 const char* pycd_last_error(const pycd_ctx* ctx);

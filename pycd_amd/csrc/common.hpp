@@ -15,14 +15,20 @@
 
 namespace pycd {
 
+// hipMalloc on the current device, tried again with nothing kept there by
+// the workspaces where the device is full.  Every allocation of the library
+// goes through it.
+inline hipError_t device_malloc(void** out, size_t bytes);
+
 // Memory that the one-shot calls (tables, neighbour lists, displacements)
 // of a context work in.  Device blocks are kept from call to call up to
 // kMaxKept bytes, oldest given back first, and a page-locked staging buffer
 // for small transfers is made with the context; both go with it.  A block
 // is free again only when the call that took it is done with the context's
 // stream, on which every call works, so that a later call's use is ordered
-// after it; any number of threads may take at once.  An allocation that
-// fails is tried again with nothing kept.
+// after it; any number of threads may take at once.  Kept memory stands in
+// no other allocation's way: the library's allocations that find the device
+// full are tried again with nothing kept on it (device_malloc).
 // (hipFree of a block of 240 MB takes 0.27 ms, hipMalloc 0.04, and copies of
 // pageable host memory 0.02-0.09 each: the 12000-site BF16x3 table 5.65 ->
 // 4.70 ms, the 6144-site FP32 one 2.20 -> 1.83, the 120-site FP64 one 262 ->
@@ -32,15 +38,42 @@ class Workspace {
   static constexpr size_t kMaxKept = size_t(512) << 20;
   static constexpr int kMaxBlocks = 32;
   static constexpr size_t kStaging = size_t(2) << 20;
-  // Device blocks are for work on `stream`.
-  hipError_t open(hipStream_t stream) {
+  // Device blocks are for work on `stream` of `device`.
+  hipError_t open(int device, hipStream_t stream) {
+    device_ = device;
     stream_ = stream;
-    return hipHostMalloc(&staging_, kStaging, hipHostMallocDefault);
+    const hipError_t e =
+        hipHostMalloc(&staging_, kStaging, hipHostMallocDefault);
+    if (e != hipSuccess) return e;
+    std::lock_guard<std::mutex> lock(open_mu_);
+    next_ = open_;
+    open_ = this;
+    return hipSuccess;
   }
   void close() {
+    {
+      std::lock_guard<std::mutex> lock(open_mu_);
+      for (Workspace** w = &open_; *w; w = &(*w)->next_)
+        if (*w == this) {
+          *w = next_;
+          break;
+        }
+    }
     clear();
     if (staging_) (void)hipHostFree(staging_);
     staging_ = nullptr;
+  }
+  // Frees what the open workspaces of `device` keep.  (Not one whose stream
+  // is being captured: that stream cannot be waited for.)
+  static void give_back(int device) {
+    std::lock_guard<std::mutex> lock(open_mu_);
+    for (Workspace* w = open_; w; w = w->next_) {
+      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+      if (w->device_ == device &&
+          hipStreamIsCapturing(w->stream_, &capture) == hipSuccess &&
+          capture == hipStreamCaptureStatusNone)
+        w->clear();
+    }
   }
   // The smallest kept block of at least `bytes` and at most twice that,
   // else a new one; *got: its size.
@@ -60,12 +93,7 @@ class Workspace {
         return hipSuccess;
       }
     }
-    hipError_t e = hipMalloc(out, need);
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      clear();
-      e = hipMalloc(out, need);
-    }
+    const hipError_t e = device_malloc(out, need);
     *got = e == hipSuccess ? need : 0;
     return e;
   }
@@ -125,7 +153,12 @@ class Workspace {
     (void)hipStreamSynchronize(stream_);
     (void)hipFree(p);
   }
+  // the open workspaces of the process
+  static inline std::mutex open_mu_;
+  static inline Workspace* open_ = nullptr;
+  Workspace* next_ = nullptr;
   std::mutex mu_;
+  int device_ = 0;
   hipStream_t stream_ = nullptr;
   Block kept_[kMaxBlocks];  // oldest first
   int n_ = 0;
@@ -133,6 +166,16 @@ class Workspace {
   void* staging_ = nullptr;
   bool staging_busy_ = false;
 };
+
+inline hipError_t device_malloc(void** out, size_t bytes) {
+  const hipError_t e = hipMalloc(out, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  int device = 0;
+  (void)hipGetDevice(&device);
+  Workspace::give_back(device);
+  return hipMalloc(out, bytes);
+}
 
 }  // namespace pycd
 
@@ -202,8 +245,12 @@ struct DevBuf {
   hipError_t alloc(size_t n) {
     release();
     if (n == 0) return hipSuccess;
-    hipError_t e = hipMalloc(reinterpret_cast<void**>(&ptr), n * sizeof(T));
-    if (e == hipSuccess) count = n;
+    void* p = nullptr;
+    const hipError_t e = device_malloc(&p, n * sizeof(T));
+    if (e == hipSuccess) {
+      ptr = static_cast<T*>(p);
+      count = n;
+    }
     return e;
   }
 };

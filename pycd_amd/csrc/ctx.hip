@@ -26,7 +26,7 @@ extern "C" int pycd_ctx_create(int device, pycd_ctx** out) {
     delete ctx;
     return PYCD_ERR_HIP;
   }
-  if (ctx->work.open(ctx->stream) != hipSuccess) {
+  if (ctx->work.open(device, ctx->stream) != hipSuccess) {
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return PYCD_ERR_HIP;
@@ -65,7 +65,7 @@ extern "C" int pycd_dev_alloc(pycd_ctx* ctx, int64_t bytes, void** out) {
   if (!ctx || !out || bytes <= 0) return PYCD_ERR_ARG;
   pycd::DeviceGuard g(ctx->device);
   *out = nullptr;
-  PYCD_HIP(ctx, hipMalloc(out, size_t(bytes)));
+  PYCD_HIP(ctx, pycd::device_malloc(out, size_t(bytes)));
   return PYCD_OK;
 }
 
