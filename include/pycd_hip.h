@@ -138,8 +138,9 @@ int pycd_min_image_vectors(pycd_ctx* ctx, const double* pos, int64_t n,
  * centre c and shell s, the positions k into `targets` with
  * lo[s] < |mic(pos[targets[k]] - pos[centers[c]])| <= hi[s], ascending in k.
  * Outputs (host memory): count[c, s], index[c, s, 0..count), vec[c, s, .., 3]
- * with room for max_per_shell entries; if a shell holds more, the call fails
- * and `count` still holds the true counts.  At most 16 shells. */
+ * with room for max_per_shell entries, zeros past a shell's count; if a shell
+ * holds more, the call fails and `count` still holds the true counts.  At
+ * most 16 shells. */
 int pycd_hop_neighbors(pycd_ctx* ctx, const double* pos, int64_t n,
                        const int64_t* centers, int64_t n_centers,
                        const int64_t* targets, int64_t n_targets,

@@ -176,14 +176,22 @@ hop_neighbor_kernel(const double* __restrict__ pos,
       }
     }
   }
-  if (lane == 0) {
 #pragma unroll
-    for (int u = 0; u < kC; ++u)
+  for (int u = 0; u < kC; ++u)
 #pragma unroll
-      for (int s = 0; s < kMaxShells; ++s)
-        if (s < w.n && c0 + u < n_centers)
-          count[(c0 + u) * w.n + s] = running[u][s];
-  }
+    for (int s = 0; s < kMaxShells; ++s) {
+      if (s >= w.n || c0 + u >= n_centers) break;
+      const int64_t row = (c0 + u) * w.n + s;
+      if (lane == 0) count[row] = running[u][s];
+      // the room past the shell's entries: the block is a kept one
+      for (int r = running[u][s] + lane; r < max_per; r += 64) {
+        const int64_t o = row * max_per + r;
+        index[o] = 0;
+        vec[3 * o] = 0.0;
+        vec[3 * o + 1] = 0.0;
+        vec[3 * o + 2] = 0.0;
+      }
+    }
 }
 
 }  // namespace pycd
