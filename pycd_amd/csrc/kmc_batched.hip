@@ -1257,7 +1257,8 @@ msd_unit_kernel(const double* __restrict__ rows,
   const int64_t P = written < 1 ? 1 : (written < d.P ? written : d.P);
   double* out = scratch + d.sbase + int64_t(c) * d.M;
   msd_unit<kQ>((gptr<double>)(rows + d.row_off + 3 * c), 3 * int64_t(d.nc), P,
-               d.M, 0, 1, [&](int64_t tau, double v) { out[tau] = v; });
+               0, d.M, false, 0, 1, kMsdWin,
+               [&](int64_t tau, double v) { out[tau] = v; });
 }
 
 __global__ void __launch_bounds__(256)

@@ -88,6 +88,11 @@ inline int msd_lanes(int64_t n, F&& lags_and_work) {
   return best;
 }
 
+// Lags of a pass.
+__host__ __device__ constexpr int msd_pass(int kq) {
+  return kMsdBlocks * kMsdL * kq;
+}
+
 // LDS position of window row r
 __device__ inline int msd_row(int r) { return r + (r >> 2); }
 
@@ -221,15 +226,18 @@ struct ExactSum {
   }
 };
 
-// The sums of a path of P rows (w3 doubles apart, from src) over the
-// origins of segments part, part + parts, ...: put(tau, sum) for every
-// tau < M, each wavefront group's sums added in order.
+// The sums of a path of P rows (w3 doubles apart, from src) for the lags
+// [lag0, M), lag0 a multiple of a pass's, over the origins of segments part,
+// part + parts, ...; those of one pass where `one`: put(tau, sum) for every
+// such lag, each wavefront group's sums added in order.  A segment is as long
+// as the window allows, at most `seg` origins (a multiple of 4).
 template <int kQ, typename Put>
 __device__ __forceinline__ void msd_unit(
     const __attribute__((address_space(1))) double* src, int64_t w3,
-    int64_t P, int64_t M, int part, int parts, Put&& put) {
+    int64_t P, int64_t lag0, int64_t M, bool one, int part, int parts, int seg,
+    Put&& put) {
   constexpr int kBlock = kMsdL * kQ;            // lags per block
-  constexpr int kPass = kMsdBlocks * kBlock;    // lags per pass
+  constexpr int kPass = msd_pass(kQ);           // lags per pass
   constexpr int kRuns = kMsdWaves * (64 / kQ);  // groups
   // the window; after a pass its space takes the groups' lag sums
   __shared__ double L[3 * kMsdPlane];
@@ -238,7 +246,8 @@ __device__ __forceinline__ void msd_unit(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & (kQ - 1);
   const int run = wave * (64 / kQ) + (tid & 63) / kQ;
-  for (int64_t pass0 = 0; pass0 < M; pass0 += kPass) {
+  const int64_t lag1 = one ? min<int64_t>(lag0 + kPass, M) : M;
+  for (int64_t pass0 = lag0; pass0 < lag1; pass0 += kPass) {
     const int span = int(min<int64_t>(kPass, M - pass0));
     double acc[kMsdBlocks][kMsdL];
 #pragma unroll
@@ -247,10 +256,10 @@ __device__ __forceinline__ void msd_unit(
       for (int i = 0; i < kMsdL; ++i) acc[b][i] = 0.0;
     const bool first = pass0 == 0;
     const int nblk = (span + kBlock - 1) / kBlock;
-    const int S = msd_segment(kQ, pass0, M);
-    const int wofs = first ? 0 : S;  // window row of path row T0 + pass0
     // origins t0 < P - pass0 have a lag of this pass inside the rows
     const int64_t t_end = P - pass0;
+    const int S = min(msd_segment(kQ, pass0, M), seg);
+    const int wofs = first ? 0 : S;  // window row of path row T0 + pass0
     for (int64_t T0 = int64_t(part) * S; T0 < t_end; T0 += int64_t(parts) * S) {
       const int64_t T1 = min<int64_t>(T0 + S, t_end);
       // ---- stage the window (and, after the first pass, the origins)
