@@ -28,7 +28,7 @@
 // ahead of the window.
 //
 // Bound by FP64 issue: 3 subtractions and 3 FMAs per distance, 92% of the
-// SIMDs' cycles at 500 lags of 2001 rows (batched, 16 ms).  4096 trajectories
+// SIMDs' cycles at 500 lags of 2001 rows (batched, 17.3 ms).  4096 trajectories
 // of 1-64 carriers, 100 lags of up to 801 rows: 4.9 ms at kQ = 64, 3.1 ms at
 // kQ = 32.
 #pragma once
@@ -103,9 +103,9 @@ __device__ inline int msd_row(int r) { return r + (r >> 2); }
 // origin bound; base: window row of relative origin 0's lag-0 row.  It reads
 // the rows below base + rb + lo + kMsdRing and the origins below rb + 2.
 // kExec: the masked steps under exec masks, which skip what no lane needs
-// (one group per wavefront: 500 lags of up to 2001 rows 16.4 -> 14.8 ms),
-// else by selects (several groups, some of whose lanes nearly always have
-// work: 100 lags 3.2 ms, 0.1 more under exec masks).
+// (one group per wavefront: 1024 x 32 paths of 2001 rows, 500 lags 6.9 -> 6.5
+// ms), else by selects (several groups, some of whose lanes nearly always
+// have work: 100 lags 3.2 ms, 0.1 more under exec masks).
 template <bool kExec>
 __device__ inline void msd_run(const double* L, int ra, int rb, int lo,
                                int hi, int lim, int base, double* acc) {
@@ -128,18 +128,13 @@ __device__ inline void msd_run(const double* L, int ra, int rb, int lo,
     oy[p] = L[ob + off(p) + 1];
     oz[p] = L[ob + off(p) + 2];
   }
-  // Sums in three levels, so that no chain of roundings is long: up to 4
-  // turns in s, those of the run in r, the runs in acc.
+  // Sums in three levels, so that no chain of roundings is long: a turn's in
+  // s, those of the run in r, the runs in acc.  (One level: 2-norm error of
+  // the batch's means 1e-15; 4 turns to a chain 1.4e-16; this 0.9e-16, as
+  // NumPy's pairwise sums, for 2.5% of the time of one level at 500 lags.)
   double r[kMsdL], s[kMsdL];
 #pragma unroll
-  for (int i = 0; i < kMsdL; ++i) r[i] = s[i] = 0.0;
-  auto flush = [&] {
-#pragma unroll
-    for (int i = 0; i < kMsdL; ++i) {
-      r[i] += s[i];
-      s[i] = 0.0;
-    }
-  };
+  for (int i = 0; i < kMsdL; ++i) r[i] = 0.0;
   // below fast_end every lane's lags up to hi have rows inside the written
   // rows
   const int fast_end = min(rb, lim - hi);
@@ -162,7 +157,10 @@ __device__ inline void msd_run(const double* L, int ra, int rb, int lo,
     o += kR;
     vb += 3 * (kR / 4 * 5);
     ob += 3 * (kR / 4 * 5);
-    if (((o - ra) & (4 * kR - 1)) == 0) flush();
+  };
+  auto add_turn = [&] {
+#pragma unroll
+    for (int i = 0; i < kMsdL; ++i) r[i] += s[i];
   };
   while (o + kR <= fast_end) {
 #pragma unroll
@@ -172,11 +170,14 @@ __device__ inline void msd_run(const double* L, int ra, int rb, int lo,
         const int q = (j + i) % kR;
         const double dx = wx[q] - ox[j & 1], dy = wy[q] - oy[j & 1],
                      dz = wz[q] - oz[j & 1];
-        s[i] = fma(dz, dz, fma(dy, dy, fma(dx, dx, s[i])));
+        // (a turn's first square needs no zero to be added to)
+        const double x2 = j == 0 ? dx * dx : fma(dx, dx, s[i]);
+        s[i] = fma(dz, dz, fma(dy, dy, x2));
       }
       load(j);
     }
     turned();
+    add_turn();
   }
   // masked steps: pair i of step j counts while lo + i < lim - o - j, for
   // each pair a first part of a group's lanes
@@ -195,17 +196,24 @@ __device__ inline void msd_run(const double* L, int ra, int rb, int lo,
     load(j);
   };
   // whole turns, then the last part of a turn
+  auto zero = [&] {
+#pragma unroll
+    for (int i = 0; i < kMsdL; ++i) s[i] = 0.0;
+  };
   while (o + kR <= rb) {
+    zero();
 #pragma unroll
     for (int j = 0; j < kR; ++j) masked_step(j);
     turned();
+    add_turn();
   }
+  zero();
 #pragma unroll
   for (int j = 0; j < kR; ++j) {
     if (o + j >= rb) break;
     masked_step(j);
   }
-  flush();
+  add_turn();
 #pragma unroll
   for (int i = 0; i < kMsdL; ++i) acc[i] += r[i];
 }
