@@ -473,15 +473,22 @@ __device__ inline uint32_t pop_ticket(const BatchArgs& a, int& bin) {
 // fewer the launch hands over from any busy SIMD to idle ones (4096 mixed
 // trajectories of 4000 hops, 1-64 carriers, whole run with its MSD: 22.3 ms
 // with idle SIMDs only and 2048 hops to spare, 20.8 so).  Words of `hand`:
-//   [0] trajectories not yet finished   [1] mailboxes taken by donors
-//   [2] mailboxes opened                [3] mailboxes (0: hand-over off)
+//   [kHandLeft] trajectories not yet finished
+//   [kHandTaken] mailboxes taken by donors
+//   [kHandOpened] mailboxes opened
+//   [kHandCap] mailboxes (0: hand-over off)
 //   [kHandHdr + k] mailbox k: 0 empty, kMailClosed, or trajectory index + 1.
+// The counts sit on cache lines of their own: atomics on one line, of whatever
+// XCD, are carried out one after another (side by side in one line, 4096
+// trajectories that fill their paths after 2 hops took 0.50 ms, now 0.25; of
+// 600 hops and 2 carriers 1.36, now 1.27).
 // Every wait ends: a mailbox is filled only while its donor's trajectory is
 // unfinished, an empty mailbox is closed (by CAS) once none is, and a wait
 // also gives up after kHandWaitTicks.  A trajectory is handed over at most
 // once (a wavefront never passes on what it received), so at most
 // grid + n_traj mailboxes are opened.
-constexpr int kHandHdr = 4;
+constexpr int kHandLeft = 0, kHandTaken = 32, kHandOpened = 64,
+              kHandCap = 96, kHandHdr = 128;
 constexpr uint32_t kMailClosed = 0xffffffffu;
 constexpr uint32_t kHandMinHops = 256;           // hops left to be worth it
 constexpr uint64_t kHandWaitTicks = 2000000000;  // 20 s at 100 MHz
@@ -493,18 +500,19 @@ __device__ inline uint32_t* hand_words(uint32_t* progress) {
 // Mailbox index of a waiting wavefront taken for a hand-over, or -1
 // (lane 0 only).
 __device__ inline int claim_mailbox(uint32_t* hand) {
-  const uint32_t cap = hand[3];
+  const uint32_t cap = hand[kHandCap];
   for (int attempt = 0; attempt < 4; ++attempt) {
-    const uint32_t head = __hip_atomic_load(hand + 1, __ATOMIC_RELAXED,
-                                            __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t open = min(__hip_atomic_load(hand + 2, __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_AGENT),
-                              cap);
+    const uint32_t head = __hip_atomic_load(
+        hand + kHandTaken, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t open =
+        min(__hip_atomic_load(hand + kHandOpened, __ATOMIC_RELAXED,
+                              __HIP_MEMORY_SCOPE_AGENT),
+            cap);
     if (head >= open) return -1;
     uint32_t expect = head;
     if (__hip_atomic_compare_exchange_strong(
-            hand + 1, &expect, head + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-            __HIP_MEMORY_SCOPE_AGENT))
+            hand + kHandTaken, &expect, head + 1, __ATOMIC_RELAXED,
+            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
       return int(head);
   }
   return -1;
@@ -513,9 +521,9 @@ __device__ inline int claim_mailbox(uint32_t* hand) {
 // Opens a mailbox and waits for a trajectory: its index, or -1 when none
 // is left to hand over or hand-over is off (lane 0 only).
 __device__ inline int wait_for_trajectory(uint32_t* hand) {
-  const uint32_t cap = hand[3];
+  const uint32_t cap = hand[kHandCap];
   if (cap == 0u) return -1;
-  const uint32_t k = atomicAdd(hand + 2, 1u);
+  const uint32_t k = atomicAdd(hand + kHandOpened, 1u);
   if (k >= cap) return -1;
   uint32_t* box = hand + kHandHdr + k;
   const uint64_t t0 = wall_clock64();
@@ -528,8 +536,8 @@ __device__ inline int wait_for_trajectory(uint32_t* hand) {
     if (v != 0u) return int(v - 1u);
     // the shared count only every 8th look, to keep the waiters off it
     if ((it & 7u) == 7u &&
-        (__hip_atomic_load(hand, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-             0u ||
+        (__hip_atomic_load(hand + kHandLeft, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT) == 0u ||
          wall_clock64() - t0 > kHandWaitTicks)) {
       uint32_t expect = 0u;
       if (__hip_atomic_compare_exchange_strong(
@@ -646,7 +654,8 @@ __device__ __forceinline__ void kmc_batched_body(const BatchArgs& a) {
     }
     const TrajOut o0 = a.out[tr];
     if (uni(o0.done)) {
-      if (a.progress && lane == 0) atomicSub(hand_words(a.progress), 1u);
+      if (a.progress && lane == 0)
+        atomicSub(hand_words(a.progress) + kHandLeft, 1u);
       continue;
     }
     const bool resume = uni(o0.started) != 0;
@@ -1199,7 +1208,8 @@ __device__ __forceinline__ void kmc_batched_body(const BatchArgs& a) {
       again = tr;  // that wavefront stopped waiting: resume it here
       continue;
     }
-    if (a.progress && lane == 0) atomicSub(hand_words(a.progress), 1u);
+    if (a.progress && lane == 0)
+      atomicSub(hand_words(a.progress) + kHandLeft, 1u);
   }
 }
 
@@ -1295,7 +1305,7 @@ __global__ void hand_reset(uint32_t* h, int64_t n, uint32_t active,
                            uint32_t cap) {
   for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
        i += int64_t(gridDim.x) * blockDim.x)
-    h[i] = i == 0 ? active : (i == 3 ? cap : 0u);
+    h[i] = i == kHandLeft ? active : (i == kHandCap ? cap : 0u);
 }
 
 __global__ void reset_outputs(TrajOut* o, int64_t n) {
