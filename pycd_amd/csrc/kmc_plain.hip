@@ -595,6 +595,13 @@ kmc_hop_kernel(HopArgs a, const KmcDev* __restrict__ dv, HopRoles roles,
       if (a.hop_proc) a.hop_proc[block + lane] = plog;
     }
   };
+  // A hop that spans several path rows: with up to 32 carriers lane l writes
+  // carrier l mod n_c's entries of every (64 / n_c)-th of them.  (With each
+  // lane writing its own carrier's alone, 1 carrier with 16 slots and 301 rows
+  // in 3 hops took 10.5 us a hop, the 256 threads of the kernel before 6.6,
+  // now 6.7; 4 slots and 67000 rows a hop 6500 us, now 297.)
+  const int copies = nc <= 32 ? 64 / nc : 1;
+  const int copy = lane / (nc <= 32 ? nc : 64), cc = lane - copy * nc;
   // clock, energy, log and path rows of hop h
   auto tick = [&](double g_sel) {
     const int hl = int(h & 63);
@@ -626,12 +633,26 @@ kmc_hop_kernel(HopArgs a, const KmcDev* __restrict__ dv, HopRoles roles,
       for (int64_t r = start + lane; r < dp_hi; r += 64) a.dpath[r] = g_sel;
       for (int64_t r = start + lane; r < end; r += 64) a.epath[r] = energy;
     }
-    if (own) {
-      const int w = 3 * nc;
+    const int w = 3 * nc;
+    if (copies > 1 && end - start >= 4) {
+      double v[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const double x = bse[k] + dsp[k];
+        v[k] = from32(__builtin_amdgcn_ds_bpermute(4 * cc, lo32(x)),
+                      __builtin_amdgcn_ds_bpermute(4 * cc, hi32(x)));
+      }
+      if (copy < copies)
+        for (int64_t r = start + copy; r < end; r += copies)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) a.rows[r * w + 3 * cc + k] = v[k];
+    } else if (own) {
       for (int64_t r = start; r < end; ++r)
 #pragma unroll
         for (int k = 0; k < 3; ++k)
           a.rows[r * w + 3 * c + k] = bse[k] + dsp[k];
+    }
+    if (own) {
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         bse[k] += dsp[k];

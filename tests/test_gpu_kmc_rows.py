@@ -64,3 +64,15 @@ def _same(gpu, ora):
 def test_helpers_of_many_slots(nc, z):
     gpu, ora = _runs(nc, z, 2001, 1.0, 200, 97)
     _same(gpu, ora)
+
+
+@pytest.mark.parametrize("rows_per_hop", [2.0, 300.0])
+@pytest.mark.parametrize("nc,z", [(1, 1), (1, 16), (2, 4), (3, 8), (7, 5),
+                                  (22, 3), (31, 2), (32, 2), (33, 2),
+                                  (70, 1)])
+def test_hops_over_many_rows(nc, z, rows_per_hop):
+    """1 to 32 carriers share a wavefront's lanes between path rows, more do
+    not; hops of none to a few rows, and of hundreds."""
+    gpu, ora = _runs(nc, z, 9001, rows_per_hop, 60, 13)
+    assert gpu["start"] > 60
+    _same(gpu, ora)
