@@ -188,7 +188,8 @@ typedef struct pycd_kmc pycd_kmc;
 
 /* Uploads the tables, forms phi_lattice = A q_lattice and the self terms
  * A[s,s] - A[s,n] of every slot.  The table pointer may be released by the
- * caller afterwards. */
+ * caller afterwards.  A session takes n_c (104 z + 88) up to 61424 (z = 4:
+ * 121 carriers), z up to 64. */
 int pycd_kmc_create(pycd_ctx* ctx, const pycd_kmc_problem* pb,
                     pycd_kmc** out);
 void pycd_kmc_destroy(pycd_kmc* s);

@@ -231,14 +231,14 @@ __device__ __forceinline__ void with_count_up(int n, F&& f) {
 // carriers the helper's z n_c gathers are the longest of the three.
 struct HopLds {
   int nc, z, look;
-  __host__ __device__ int np() const { return nc * z; }
+  __host__ __device__ constexpr int np() const { return nc * z; }
   // rates of p at (p mod per) kStride + p / per, so that lane l's processes
   // l per .. l per + per - 1 are read on distinct banks
   static constexpr int kStride = 65;
-  __host__ __device__ int per() const { return (np() + 63) / 64; }
+  __host__ __device__ constexpr int per() const { return (np() + 63) / 64; }
   // psi of the site rows, charges, rates, dG0, hop vectors, the mover's
   // rows; sites, targets and look-ahead with their codes; the end flag
-  __host__ __device__ size_t bytes() const {
+  __host__ __device__ constexpr size_t bytes() const {
     return 8 * (2 * size_t(nc) + size_t(per()) * kStride + 4 * size_t(np()) +
                 2 * size_t(z) + 2) +
            8 * (size_t(nc) + size_t(np()) + (look ? size_t(np()) * z : 0)) + 8;
@@ -253,12 +253,33 @@ constexpr int kHopWaves = 16;  // at most
 struct HopRoles {
   int process, site, helper;
   HopRoles() = default;
-  HopRoles(int nc, int z)
+  constexpr HopRoles(int nc, int z)
       : process((nc * z + 63) / 64), site((nc + 63) / 64),
         helper(std::max(1, std::min((z + 3) / 4,
                                     kHopWaves - process - site))) {}
-  int threads() const { return 64 * (process + site + helper); }
+  constexpr int threads() const { return 64 * (process + site + helper); }
+  // Every process and carrier is owned by a lane, a lane sums at most 10
+  // processes, and the block holds the wavefronts.
+  constexpr bool fit(int nc, int z) const {
+    return process <= 10 && threads() <= 64 * kHopWaves &&
+           64 * process >= nc * z && 64 * site >= nc;
+  }
 };
+
+// The sessions that pycd_kmc_create takes: n_c (104 z + 88) <= kSessionMost
+// (z = 4: 121 carriers), all of which the hop kernel can run.
+constexpr int64_t kSessionMost = 61424;
+constexpr bool session_fits(int64_t nc, int64_t z) {
+  return nc * (104 * z + 88) <= kSessionMost;
+}
+constexpr bool every_session_runs() {
+  for (int z = 1; z <= 64; ++z)
+    for (int nc = 1; session_fits(nc, z); ++nc)
+      if (!HopRoles(nc, z).fit(nc, z) || HopLds{nc, z, 0}.bytes() > 65536)
+        return false;
+  return true;
+}
+static_assert(every_session_runs(), "the hop kernel holds every session");
 
 template <bool kCompact, bool kLook>
 __global__ void __launch_bounds__(64 * kHopWaves)
@@ -896,7 +917,7 @@ struct pycd_kmc {
   size_t hop_smem = 0;
   // PYCD_KMC_WAVE may be named, and what was named
   bool wave_ok = false;
-  size_t wave_smem = 0;
+  size_t wave_bytes = 0;
   int32_t variant = PYCD_KMC_AUTO;
   bool begun = false;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -1063,12 +1084,12 @@ hipError_t pack_hop_inputs(pycd_kmc* s) {
   return hipGetLastError();
 }
 
-// The sessions for which PYCD_KMC_WAVE can be named: those of few enough
-// carriers for one wavefront to keep every table entry that a hop reads in
-// LDS (entries of carrier pairs in groups of 4 for n_c z + n_c rows, psi and
-// charges, sites with codes, z z targets per carrier).  0 for the others.
-// Both names run the same kernel.
-size_t wave_lds_bytes(int nc, int z) {
+// The sessions for which PYCD_KMC_WAVE can be named, a line of the interface:
+// few carriers, and the bytes of every table entry that their rates read
+// (those of carrier pairs in groups of 4 for n_c z + n_c rows, psi and
+// charges, sites with codes, z z targets per carrier) within a workgroup's
+// LDS.  0 for the others.  Both names run the same kernel.
+size_t rate_entry_bytes(int nc, int z) {
   const int nproc = nc * z;
   if (nc > 64 || nproc > 256 || z > 8) return 0;
   const size_t ncp = (((size_t(nc) + 1) / 2) + 3) & ~size_t(3);
@@ -1087,13 +1108,10 @@ extern "C" int pycd_kmc_create(pycd_ctx* ctx, const pycd_kmc_problem* pb,
   DeviceGuard guard(ctx->device);
   const int64_t N = pb->n_sites;
   const int nc = pb->n_carriers, z = pb->z, mz = pb->max_z;
-  const size_t smem = sizeof(double) * (size_t(nc) * (1 + z) + 11 * size_t(nc) * z +
-                                        9 * size_t(nc)) +
-                      sizeof(int32_t) * (size_t(nc) * z + nc) +
-                      sizeof(uint32_t) * (size_t(nc) * z + nc) + 16;
-  if (smem > 60 * 1024)
+  if (!session_fits(nc, z))
     return fail(ctx, PYCD_ERR_ARG,
-                "n_c=%d, z=%d need %zu B of LDS (limit 60 KiB)", nc, z, smem);
+                "n_c=%d, z=%d: a session takes n_c (104 z + 88) up to %lld",
+                nc, z, (long long)kSessionMost);
   // Host-side validation of the slot table (every index the kernel reads).
   std::vector<int32_t> nb(size_t(N) * mz);
   {
@@ -1186,16 +1204,15 @@ extern "C" int pycd_kmc_create(pycd_ctx* ctx, const pycd_kmc_problem* pb,
     S_HIP(hipDeviceGetAttribute(&lds_max,
                                 hipDeviceAttributeMaxSharedMemoryPerBlock,
                                 ctx->device));
-    s->wave_smem = wave_lds_bytes(nc, z);
+    s->wave_bytes = rate_entry_bytes(nc, z);
     s->hop_roles = HopRoles(nc, z);
     HopLds hl{nc, z, z * z <= 64 * s->hop_roles.helper ? 1 : 0};
     if (hl.bytes() + 512 > size_t(lds_max)) hl.look = 0;
     s->hop_look = hl.look;
     s->hop_smem = hl.bytes();
-    // (512 bytes of 2^(j/64) beside the dynamic part; one wavefront's 32-bit
-    // table offsets)
+    // (512 bytes of 2^(j/64) are beside the dynamic part)
     const double tab_bytes = 8.0 * double(s->compact ? s->geo.nu : N) * N;
-    s->wave_ok = s->wave_smem > 0 && s->wave_smem + 512 <= size_t(lds_max) &&
+    s->wave_ok = s->wave_bytes > 0 && s->wave_bytes + 512 <= size_t(lds_max) &&
                  tab_bytes < 4294967296.0;
   }
 #undef S_HIP
@@ -1210,9 +1227,10 @@ extern "C" int pycd_kmc_set_variant(pycd_kmc* s, int32_t variant) {
     return fail(s->ctx, PYCD_ERR_ARG, "unknown kernel variant %d", variant);
   if (variant == PYCD_KMC_WAVE && !s->wave_ok)
     return fail(s->ctx, PYCD_ERR_ARG,
-                "the one-wavefront kernel needs n_c <= 64, n_c z <= 256, "
-                "z <= 8 and %zu B of LDS (n_c=%d, z=%d)",
-                s->wave_smem, s->pb.n_carriers, s->pb.z);
+                "PYCD_KMC_WAVE is for n_c <= 64, n_c z <= 256, z <= 8, the "
+                "entries its rates read (%zu B) within a workgroup's LDS and "
+                "a table below 4 GiB (n_c=%d, z=%d)",
+                s->wave_bytes, s->pb.n_carriers, s->pb.z);
   s->variant = variant;
   return PYCD_OK;
 }
@@ -1336,13 +1354,7 @@ hipError_t launch_hop_t(const pycd_kmc* s, hipStream_t st, const HopArgs& args,
 
 hipError_t launch_hop(const pycd_kmc* s, hipStream_t st, const HopArgs& args,
                       int32_t* status) {
-  // every process and carrier is owned by a lane; the kernel sums at most
-  // 10 processes per lane
-  const HopRoles& r = s->hop_roles;
-  if (r.threads() > 64 * kHopWaves || r.process > 10 ||
-      64 * r.process < s->pb.n_carriers * s->pb.z ||
-      64 * r.site < s->pb.n_carriers)
-    return hipErrorInvalidValue;
+  if (!s->hop_roles.fit(s->pb.n_carriers, s->pb.z)) return hipErrorInvalidValue;
   if (s->compact)
     return s->hop_look ? launch_hop_t<true, true>(s, st, args, status)
                        : launch_hop_t<true, false>(s, st, args, status);
