@@ -60,9 +60,11 @@ structure_factor_lowp(const double* __restrict__ pos, int n, int n_pad,
   const bool real = m < K;
   const double kx = real ? kv[3 * m] : 0.0, ky = real ? kv[3 * m + 1] : 0.0,
                kz = real ? kv[3 * m + 2] : 0.0, w = real ? sw[m] : 0.0;
-  // w v and, in two parts, its rounding to BF16 (of a cosine by way of
-  // FP32: a few ties in 1e8 go to the even neighbour, the low part makes up
-  // for it) and what that leaves
+  // w v and, in two parts, its rounding to BF16 and what that leaves.  A
+  // cosine is rounded by way of FP32, a sine at once: 8.5e-6 of the cosines
+  // go to the other neighbour for that (an FP32 value lies halfway between
+  // two BF16 ones once in 65536), and the low part holds the difference.
+  // Tables of this mode have had these bits from the start.
   auto put = [&](int64_t o, double v, bool by_f32) {
 #pragma clang fp contract(off)
     const double y = w * v;
