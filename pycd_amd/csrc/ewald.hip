@@ -263,8 +263,12 @@ reduce_parts(const double* __restrict__ P, int n, int parts, int tile,
 // +/- pairs) of (j, i) are the negatives of those of (i, j).  A tile on the
 // diagonal has both as formed, so its blocks write no mirror.
 //
-// kRows: rows of a block.  16 instead of 64 where those blocks are fewer
-// than two per CU (120 sites: 18 -> 7 us).
+// kRows: rows of a block.  16 instead of 64 below 128 blocks of 64, where a
+// block's rows one after another take longer than there is to do beside them;
+// above, 64 write whole lines of the mirror.  Device time of this kernel with
+// 16 and 64 rows: 3 tiles 9.6 and 20.5 us, 45 17 and 22, 78 25 and 23, 120 33
+// and 26 (without order among the sites 16 rows are the faster ones there),
+// 190 46 and 30, 435 91 and 41.
 template <int kTile, int kRows>
 __global__ void __launch_bounds__(256)
 finish_table(const double* __restrict__ pos, int n, MicGeometry g,
@@ -317,7 +321,7 @@ void launch_finish(hipStream_t s, int tile, const double* pos, int n,
   const int nb = (n + tile - 1) / tile, tiles = nb * (nb + 1) / 2;
   if (tile != 64)
     finish_table<128, 64><<<4 * tiles, 256, 0, s>>>(pos, n, geo, es, A, pairs);
-  else if (tiles >= 512)
+  else if (tiles >= 128)
     finish_table<64, 64><<<tiles, 256, 0, s>>>(pos, n, geo, es, A, pairs);
   else
     finish_table<64, 16><<<4 * tiles, 256, 0, s>>>(pos, n, geo, es, A, pairs);
