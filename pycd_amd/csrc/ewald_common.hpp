@@ -246,6 +246,16 @@ __device__ inline void tile_coords_upper(int n, int tile, int& bi, int& bj) {
   tile_coords_upper_at(n, tile, int(blockIdx.x), bi, bj);
 }
 
+// Sites from which the FP64 and FP32 contractions take 128 x 128 tiles: they
+// read half the rows of Y and of LDS per product, but come in few rounds over
+// the CUs (4.6 workgroups each at 6144 sites), the last one partly empty.  A
+// call with 64 and with 128, FP64: 2160 sites and 887 k vectors 308 and 347
+// us, 3024 and 1248 533 and 726, 4704 and 1932 1509 and 1537, 5376 and 2200
+// 2158 and 2247, 6144 and 2508 3150 and 3097, 12000 and 4917 23500 and 21500;
+// FP32: 242 and 284, 373 and 490, 907 and 953, 1242 and 1339, 1820 and 1820,
+// 12300 and 11360.
+constexpr int kTile128From = 6144;
+
 // Adds the real-space and self terms to the entries that a contraction over
 // the upper triangle of `tile` x `tile` tiles (64 or 128) left in A, and
 // writes the mirrors of the tiles off the diagonal (finish_table, ewald.hip).
