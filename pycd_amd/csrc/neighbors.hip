@@ -282,9 +282,10 @@ extern "C" int pycd_hop_neighbors(pycd_ctx* ctx, const double* pos, int64_t n,
   PYCD_HIP(ctx, hipMemcpyAsync(dt.ptr, targets, 8 * n_targets,
                                hipMemcpyHostToDevice, st));
   // More centres per wavefront share more of each pair's work and leave
-  // fewer wavefronts: a call with 1, 2, 4 each takes 149, 159, - us at 768
-  // centres, 657, 657, 682 at 6144, 1029, 1003, 1015 at 9600, 2008, 1841,
-  // 1824 at 17280, 14.1, 10.7, 9.0 ms at 72000.
+  // fewer wavefronts: a call (as many targets, two shells of 4) with 1, 2, 4
+  // each takes 170, 177, 203 us at 4116 centres, 195, 198, 228 at 5376, 230,
+  // 228, 257 at 6144, 323, 294, 322 at 8748, 469, 392, 405 at 12000, 661, 533,
+  // 502 at 15972, 1104, 790, 740 at 22464.
   const auto launch = [&](auto kernel, int per_wave) {
     const int64_t per_block = 4 * per_wave;
     kernel<<<unsigned((n_centers + per_block - 1) / per_block), 256, 0, st>>>(
@@ -293,7 +294,7 @@ extern "C" int pycd_hop_neighbors(pycd_ctx* ctx, const double* pos, int64_t n,
   };
   if (n_centers < 6144)
     launch(hop_neighbor_kernel<1>, 1);
-  else if (n_centers < 16384)
+  else if (n_centers < 13824)
     launch(hop_neighbor_kernel<2>, 2);
   else
     launch(hop_neighbor_kernel<4>, 4);

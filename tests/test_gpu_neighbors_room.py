@@ -10,7 +10,8 @@ CELL = np.array([[9.0, 0.4, -0.7], [-4.1, 8.2, 0.3], [0.9, -0.5, 12.0]])
 
 
 @pytest.mark.parametrize("n,n_centers", [(1, 1), (65, 65), (130, 7),
-                                         (70, 6145), (70, 16387)])
+                                         (70, 6145), (70, 13823),
+                                         (70, 13824), (70, 16387)])
 def test_nothing_of_an_earlier_call_is_left(n, n_centers):
     """A call with every target in its shells, then one of the same sizes
     (so in the same memory) with few or none: zeros past the counts, for
