@@ -174,7 +174,7 @@ MsdSplit msd_split(int64_t paths, int64_t P, int64_t M) {
       blocks * P <= 450000)
     return s;
   s.kq = paths < 64 ? 16 : msd_lanes(1, [&](int64_t) {
-    return std::make_pair(M, 1.0);
+    return MsdCase{P, M, 1.0};
   });
   const int64_t pass = msd_pass(s.kq);
   if (paths < kFill) s.passes = (M + pass - 1) / pass;

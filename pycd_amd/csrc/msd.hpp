@@ -10,8 +10,7 @@
 // owns the kMsdL consecutive lags pass0 + 4 kQ b + kMsdL q + i.  A wavefront
 // holds 64 / kQ groups, which walk different origins: kQ = 64 leaves most
 // lanes without a lag when M is small (100 lags: 39 lanes of 64), so kQ is
-// the one whose whole blocks cover M with the fewest lags (msd_lanes).  For
-// a block, a group walks consecutive origins t0 and keeps r(t0 + lag) of its
+// the one that takes the fewest steps (msd_lanes).  For a block, a group walks consecutive origins t0 and keeps r(t0 + lag) of its
 // lane's lags in a ring of kMsdRing registers, so a step reads the origin
 // (one address for the group) and one new position, and forms kMsdL squared
 // distances.  Origin t0 has work in block b only while
@@ -36,7 +35,6 @@
 #include "common.hpp"
 
 #include <cstdint>
-#include <utility>
 
 namespace pycd {
 
@@ -61,26 +59,46 @@ __host__ __device__ inline int msd_segment(int kq, int64_t pass0, int64_t M) {
   return (pass0 == 0 ? room : room / 2) & ~3;
 }
 
-// Lags formed for M of them by groups of kq lanes: whole blocks.
-inline int64_t msd_lags_formed(int kq, int64_t M) {
-  const int64_t block = kMsdL * kq;
-  return (M + block - 1) / block * block;
+// Wavefront steps of a path of P rows and M lags with groups of kq lanes: its
+// (block, origin) steps over the groups, and what a block of a segment costs
+// besides (its runs' first reads, the masked steps), 10, 28 and 16 steps at kq
+// = 64, 32 and 16 (in proportion below 150 origins).
+inline double msd_cost(int kq, int64_t P, int64_t M) {
+  const int64_t block = kMsdL * kq, pass = kMsdBlocks * block;
+  const double extra = kq == 64 ? 10 : kq == 32 ? 28 : 16;
+  double steps = 0.0;
+  for (int64_t p0 = 0; p0 < M && p0 < P; p0 += pass) {
+    const int64_t S = msd_segment(kq, p0, M), n = P - p0;
+    const double segments = n < 150 ? n / 150.0 : double((n + S - 1) / S);
+    for (int64_t lag = p0; lag < p0 + pass && lag < M; lag += block)
+      steps += extra * segments +
+               (P > lag ? double(P - lag) * kq / (64 * kMsdWaves) : 0.0);
+  }
+  return steps;
 }
 
-// Lanes per group, 64, 32 or 16, for `n` units of M[k] lags and w[k] origins:
-// the fewest distances formed, the wider group on a tie (it needs fewer
-// passes over the rows).
+// Lanes per group, 64, 32 or 16, for `n` kinds of paths: case_of(k) gives
+// their rows, lags and number.  Fewest steps; the wider group on a tie (it
+// needs fewer passes over the rows).  Over 211 pairs of 20 to 5001 rows and 5
+// to 1500 lags, each timed with all three, the choice takes 0.4% longer than
+// the best on average and 12% at most; by the lags in whole blocks alone it
+// was up to 33% (401 rows, 130 lags: 64 lanes 0.21 ms, 32 0.25, 16 0.23; 64
+// lags 0.19, 0.13, 0.08).
+struct MsdCase {
+  int64_t P, M;
+  double paths;
+};
 template <typename F>
-inline int msd_lanes(int64_t n, F&& lags_and_work) {
+inline int msd_lanes(int64_t n, F&& case_of) {
   int best = 64;
   double least = 0.0;
   for (int kq = 64; kq >= 16; kq /= 2) {
     double cost = 0.0;
     for (int64_t k = 0; k < n; ++k) {
-      const auto lw = lags_and_work(k);
-      cost += double(msd_lags_formed(kq, lw.first)) * lw.second;
+      const MsdCase c = case_of(k);
+      cost += msd_cost(kq, c.P, c.M) * c.paths;
     }
-    if (kq == 64 || cost < 0.95 * least) {
+    if (kq == 64 || cost < least) {
       best = kq;
       least = cost;
     }
