@@ -98,16 +98,14 @@ class Workspace {
     return e;
   }
   void give(void* p, size_t bytes) {
-    bool kept = false;
-    {
+    void* out = p;  // what is not kept: a block too large, or the oldest one
+    if (bytes <= kMaxKept) {
       std::lock_guard<std::mutex> lock(mu_);
-      if (bytes <= kMaxKept && n_ < kMaxBlocks) {
-        kept_[n_++] = {p, bytes};
-        held_ += bytes;
-        kept = true;
-      }
+      out = n_ == kMaxBlocks ? remove(0).ptr : nullptr;
+      kept_[n_++] = {p, bytes};
+      held_ += bytes;
     }
-    if (!kept) release(p);
+    if (out) release(out);
     while (release_oldest(kMaxKept)) {
     }
   }

@@ -41,12 +41,14 @@ namespace sim {
 inline size_t used[2] = {0, 0};
 inline int current = 0;
 inline bool broken = false;  // a capturing stream was waited for
+inline size_t mallocs = 0;
 inline std::map<void*, std::pair<int, size_t>> blocks;
 constexpr size_t kHolds = size_t(1000) << 20;
 }
 inline hipError_t hipMalloc(void** p, size_t n) {
   if (sim::used[sim::current] + n > sim::kHolds) return hipErrorOutOfMemory;
   *p = std::malloc(1);
+  ++sim::mallocs;
   sim::used[sim::current] += n;
   sim::blocks[*p] = {sim::current, n};
   return hipSuccess;
@@ -153,6 +155,25 @@ int main() {
   check(!sim::broken, "no capturing stream is waited for");
   check(pycd_dev_alloc(b, int64_t(900 * kMiB), &p) == 0, "afterwards");
   check(pycd_dev_free(b, p) == 0, "pycd_dev_free");
+  // calls of many sizes: the oldest blocks make room for the newest
+  pycd_ctx_destroy(a);
+  check(pycd_ctx_create(0, &a) == 0, "context");
+  const size_t others = sim::blocks.size();
+  for (int k = 0; k < 100; ++k) {
+    pycd::DeviceGuard g(0);
+    pycd::WorkBuf<char> one;
+    check(one.alloc(a, (size_t(k) * 5 + 1) << 12) == hipSuccess, "block");
+  }
+  const size_t before = sim::mallocs;
+  for (int k = 90; k < 100; ++k) {
+    pycd::DeviceGuard g(0);
+    pycd::WorkBuf<char> one;
+    check(one.alloc(a, (size_t(k) * 5 + 1) << 12) == hipSuccess, "block");
+  }
+  check(sim::mallocs == before, "the newest sizes are kept");
+  check(sim::blocks.size() == others + 32, "no more than 32 blocks are");
+  pycd_ctx_destroy(a);
+  check(pycd_ctx_create(0, &a) == 0, "context");
   // contexts that are gone
   one_shot(b, 400);
   pycd_ctx_destroy(b);
