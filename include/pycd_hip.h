@@ -212,7 +212,7 @@ int pycd_kmc_table_rows(const pycd_kmc* s, int64_t* rows);
 /* Instance of the hop loop.  PYCD_KMC_WAVE: few carriers (n_c <= 64,
  * n_c z <= 256, z <= 8, the table entries of every carrier at every site
  * the rates need within a workgroup's LDS and a table below 4 GiB);
- * PYCD_KMC_WORKGROUP: any size; PYCD_KMC_AUTO (the default):
+ * PYCD_KMC_WORKGROUP: any session; PYCD_KMC_AUTO (the default):
  * PYCD_KMC_WAVE where it applies.  One kernel serves all of them, so they
  * give the same results bit for bit and take the same time.  Asking for
  * PYCD_KMC_WAVE where it does not apply is an argument error.

@@ -11,8 +11,9 @@
 // structure factors Y[i, m] = sqrt(w_m) cos(k_m . r_i),
 // Y[i, K + m] = sqrt(w_m) sin(k_m . r_i): A_recip = 2/eps * Y Y^T, because
 // cos(k.(r_j - r_i)) = cos(k.r_i) cos(k.r_j) + sin(k.r_i) sin(k.r_j).  The
-// contraction kernel fuses the real-space term (minimum image + erfc), the
-// self term and the final store, so the N x N table is written once.
+// contraction writes the upper triangle of tiles; finish_table adds the
+// real-space term (minimum image + erfc) and the self term and writes the
+// mirror.
 #include "common.hpp"
 #include "ewald_common.hpp"
 
