@@ -60,6 +60,8 @@ def _same(gpu, ora):
     (5, 17),           # five, none
     (3, 33), (1, 61),  # helpers beyond the slots' groups of four, and all 14
     (9, 64),           # as many as the process wavefronts leave room for
+    (42, 13), (35, 16),  # look-aheads that take the block past 64 KiB of LDS
+    (30, 17), (121, 4),  # the most carriers, none and one
 ])
 def test_helpers_of_many_slots(nc, z):
     gpu, ora = _runs(nc, z, 2001, 1.0, 200, 97)
