@@ -119,7 +119,8 @@ int pycd_pair_table(pycd_ctx* ctx, const double* pos, int64_t n,
  *                     3 = slices of 32 in two LDS stages, 4 = 256 x 256
  *                     tiles (8 wavefronts) in two LDS stages
  *   PYCD_PREC_F32     1 (the only one)
- *   0 = the default (FP64: 128 x 128 from 6144 sites on; BF16x3: 4 from
+ *   0 = the default (FP64: by the rounds of tiles over the CUs, on 256 of
+ *   them 64 x 64 up to 2432 sites and 128 x 128 from 9537; BF16x3: 4 from
  *   4096 sites on, 2 below). */
 int pycd_set_table_variant(pycd_ctx* ctx, int32_t precision, int32_t variant);
 /* The variant set for `precision` (0 = default), or -1 for a bad call. */

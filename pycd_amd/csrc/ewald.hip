@@ -344,9 +344,9 @@ int launch_table(pycd_ctx* ctx, int precision, const double* pos, int n,
     return launch_table_mfma(ctx, precision, pos, n, kv, sw, K, geo, es, out,
                              pairs, after_sf, real);
   hipStream_t s = ctx->stream;
-  // tile variant: 1 = 64 x 64, 2 = 128 x 128; 0 picks by kTile128From
+  // tile variant: 1 = 64 x 64, 2 = 128 x 128; 0 picks (wide_tiles)
   int v = ctx->table_variant[PYCD_PREC_F64];
-  if (v == 0) v = n >= kTile128From ? 2 : 1;
+  if (v == 0) v = wide_tiles(n, ctx->cu_count) ? 2 : 1;
   const int tile = v == 2 ? 128 : 64;
   const int nb = (n + tile - 1) / tile;
   // K in whole pairs of slices, rows in whole tiles

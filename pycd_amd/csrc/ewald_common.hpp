@@ -246,15 +246,22 @@ __device__ inline void tile_coords_upper(int n, int tile, int& bi, int& bj) {
   tile_coords_upper_at(n, tile, int(blockIdx.x), bi, bj);
 }
 
-// Sites from which the FP64 and FP32 contractions take 128 x 128 tiles: they
-// read half the rows of Y and of LDS per product, but come in few rounds over
-// the CUs (4.6 workgroups each at 6144 sites), the last one partly empty.  A
-// call with 64 and with 128, FP64: 2160 sites and 887 k vectors 308 and 347
-// us, 3024 and 1248 533 and 726, 4704 and 1932 1509 and 1537, 5376 and 2200
-// 2158 and 2247, 6144 and 2508 3150 and 3097, 12000 and 4917 23500 and 21500;
-// FP32: 242 and 284, 373 and 490, 907 and 953, 1242 and 1339, 1820 and 1820,
-// 12300 and 11360.
-constexpr int kTile128From = 6144;
+// True where the FP64 and FP32 contractions of n sites take 128 x 128 tiles,
+// else 64 x 64.  Larger ones read half the rows of Y and of LDS per product (a
+// 64 tile costs about 1.09 of a quarter), but their last round over the CUs
+// can be nearly empty.  A call with 64 and with 128, FP64: 2160 sites and 887
+// k vectors 308 and 347 us, 2592 and 1051 410 and 407, 3024 and 1248 533 and
+// 726, 4704 and 1932 1509 and 1537, 5376 and 2200 2158 and 2247, 6144 and 2508
+// 3150 and 3097, 7776 and 3198 6420 and 6190, 12000 and 4917 23500 and 21500;
+// FP32: 242 and 284, 305 and 323, 373 and 490, 907 and 953, 1242 and 1339,
+// 1820 and 1820, 3580 and 3440, 12300 and 11360.
+inline bool wide_tiles(int n, int cus) {
+  const auto rounds = [&](int64_t tile) {
+    const int64_t nb = (n + tile - 1) / tile, tiles = nb * (nb + 1) / 2;
+    return (tiles + cus - 1) / cus;
+  };
+  return 4.0 * double(rounds(128)) <= 1.09 * double(rounds(64));
+}
 
 // Adds the real-space and self terms to the entries that a contraction over
 // the upper triangle of `tile` x `tile` tiles (64 or 128) left in A, and

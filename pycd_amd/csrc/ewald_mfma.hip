@@ -124,7 +124,7 @@ __device__ __forceinline__ void store_recip(const v4f (&acc)[kX][kY],
 // (4.6 at 6144 sites) are worked on side by side.  With one stage, two
 // barriers a slice and the rest of the entries in the epilogue: 2.07 ms at
 // 6144 sites and 2 K = 5036 (1.3 at the matrix rate); now 1.65 and 0.15 for
-// finish_table.  64 x 64 tiles below kTile128From, as for table_f64.  Every
+// finish_table.  64 x 64 or 128 x 128 tiles as for table_f64 (wide_tiles).  Every
 // entry is the chain over k whatever the tile.
 constexpr int kFSlice = 16;
 template <int kB>
@@ -681,8 +681,9 @@ int launch_table_mfma(pycd_ctx* ctx, int precision, const double* pos, int n,
   const int Kp = std::max(slice, ((2 * K + slice - 1) / slice) * slice);
   // rows in whole tiles: the rows past n stay zero
   const int tile =
-      precision == PYCD_PREC_F32 ? (n < kTile128From ? 64 : kMTile)
-                                 : (bvar == 4 ? kMTile2 : kMTile);
+      precision == PYCD_PREC_F32
+          ? (wide_tiles(n, ctx->cu_count) ? kMTile : 64)
+          : (bvar == 4 ? kMTile2 : kMTile);
   const int nb = (n + tile - 1) / tile;
   const int n_pad = nb * tile;
   const size_t elems = size_t(n_pad) * Kp;

@@ -59,8 +59,9 @@ def test_edge_sizes(n, pbc, mode, variants):
         assert np.array_equal(got, first), v
 
 
-@pytest.mark.parametrize("mode,n", [("f32", 2047), ("f32", 6143),
-                                    ("f64", 6143), ("bf16x3", 4095)])
+@pytest.mark.parametrize("mode,n", [("f32", 2047), ("f32", 2432),
+                                    ("f64", 2432), ("f32", 6080),
+                                    ("f64", 6400), ("bf16x3", 4095)])
 def test_sizes_about_the_choice_of_kernel(mode, n):
     """One site fewer than, as many as and one more than where the default
     kernel changes: the entries of the sites in common are the same bits."""
