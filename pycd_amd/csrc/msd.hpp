@@ -121,9 +121,11 @@ __device__ inline int msd_row(int r) { return r + (r >> 2); }
 // origin bound; base: window row of relative origin 0's lag-0 row.  It reads
 // the rows below base + rb + lo + kMsdRing and the origins below rb + 2.
 // kExec: the masked steps under exec masks, which skip what no lane needs
-// (one group per wavefront: 1024 x 32 paths of 2001 rows, 500 lags 6.9 -> 6.5
-// ms), else by selects (several groups, some of whose lanes nearly always
-// have work: 100 lags 3.2 ms, 0.1 more under exec masks).
+// (one group per wavefront: 1024 x 32 paths of 2001 rows, 500 lags 6.94 -> 6.63
+// ms), else by selects (four groups, some of whose lanes nearly always have
+// work: 2048 x 32 of 401 rows, 60 lags 0.69 ms, 0.73 under exec masks).  Two
+// groups lie between: 120 lags of the same paths 1.17 and 1.12 ms, 100 lags of
+// 4096 x 16 of 801 rows 1.99 and 1.97.
 template <bool kExec>
 __device__ inline void msd_run(const double* L, int ra, int rb, int lo,
                                int hi, int lim, int base, double* acc) {
